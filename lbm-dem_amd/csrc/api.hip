@@ -896,14 +896,17 @@ extern "C" int lbdem_init(lbdem_ctx* c) {
     return 0;
 }
 
-static int check_errors(lbdem_ctx* c) {
-    DevScalars hs;
-    HIPCHK(hipMemcpyAsync(&hs, c->sc, sizeof(hs), hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(hipStreamSynchronize(c->stream));
+static int scalar_errors(lbdem_ctx* c, const DevScalars& hs) {
     if (hs.typeError) return c->fail(LBDEM_E_TYPE, "TYPE ERROR: streaming met an unsupported neighbour type");
     if (hs.listOverflow) return c->fail(LBDEM_E_CAPACITY, "an interface/object list overflowed its capacity");
     if (hs.nbrOverflow) return c->fail(LBDEM_E_CAPACITY, "neighbour list capacity (64) exceeded");
     return 0;
+}
+static int check_errors(lbdem_ctx* c) {
+    DevScalars hs;
+    HIPCHK(hipMemcpyAsync(&hs, c->sc, sizeof(hs), hipMemcpyDeviceToHost, c->stream));
+    HIPCHK(hipStreamSynchronize(c->stream));
+    return scalar_errors(c, hs);
 }
 
 // --------------------------- steps ---------------------------
@@ -1275,7 +1278,7 @@ extern "C" int lbdem_get_info(lbdem_ctx* c, lbdem_info* in) {
     in->lastExtraMass = hs.lastExtraMass;
     in->lastSurplus = hs.lastSurplus;
     in->precision = c->box.prec;
-    return check_errors(c);
+    return scalar_errors(c, hs);
 }
 
 extern "C" int lbdem_get_types(lbdem_ctx* c, uint8_t* type, uint8_t* pflag, int32_t* solid) {
@@ -1410,37 +1413,34 @@ static int fetch(lbdem_ctx* c, double* dst, const double* src, size_t n) {
     return 0;
 }
 
+// n records packed on the device and copied at once
+static int fetch_records(lbdem_ctx* c, const RecordMap& m, int n, double* rec) {
+    const size_t bytes = size_t(n) * size_t(m.cols) * sizeof(double);
+    double* d = c->tmp(bytes);
+    if (!d) return c->fail(LBDEM_E_NOMEM, "device allocation failed");
+    dem_pack_records(m, n, d, c->stream);
+    HIPCHK(hipGetLastError());
+    HIPCHK(hipMemcpyAsync(rec, d, bytes, hipMemcpyDeviceToHost, c->stream));
+    HIPCHK(hipStreamSynchronize(c->stream));
+    return 0;
+}
+
 extern "C" int lbdem_get_particles(lbdem_ctx* c, double* rec) {
     NEED_INIT;
     const int np = c->dp.nPart;
     if (np == 0) return 0;
     const DemState& d = c->ds;
-    const double* srcs[] = {d.x0, d.x1, d.w1, d.FHydro, d.MHydro, d.FContact, d.MContact, d.FLub, d.MLub, d.FRep,
-                            d.FTotal, d.MTotal, d.FGrav};
-    const int offs[] = {LBDEM_P_X0, LBDEM_P_X1, LBDEM_P_W1, LBDEM_P_FHYDRO, LBDEM_P_MHYDRO, LBDEM_P_FCONTACT,
-                        LBDEM_P_MCONTACT, LBDEM_P_FLUB, LBDEM_P_MLUB, LBDEM_P_FREP, LBDEM_P_FTOTAL, LBDEM_P_MTOTAL,
-                        LBDEM_P_FGRAV};
-    std::vector<double> buf(3 * size_t(np));
-    for (int k = 0; k < 13; ++k) {
-        if (fetch(c, buf.data(), srcs[k], 3 * np)) return LBDEM_E_DEVICE;
-        HIPCHK(hipStreamSynchronize(c->stream));
-        for (int i = 0; i < np; ++i) for (int a = 0; a < 3; ++a) rec[size_t(i) * LBDEM_P_REC + offs[k] + a] = buf[3 * i + a];
-    }
-    const double* s2[] = {d.xiw, d.xio};
-    const int o2[] = {LBDEM_P_XIW, LBDEM_P_XIO};
-    for (int k = 0; k < 2; ++k) {
-        if (fetch(c, buf.data(), s2[k], 3 * np)) return LBDEM_E_DEVICE;
-        HIPCHK(hipStreamSynchronize(c->stream));
-        for (int i = 0; i < np; ++i) for (int a = 0; a < 3; ++a) rec[size_t(i) * LBDEM_P_REC + o2[k] + a] = buf[3 * i + a];
-    }
-    const double* s1[] = {d.fluidVol, d.r, d.m};
-    const int o1[] = {LBDEM_P_FLUIDVOL, LBDEM_P_R, LBDEM_P_M};
-    for (int k = 0; k < 3; ++k) {
-        if (fetch(c, buf.data(), s1[k], np)) return LBDEM_E_DEVICE;
-        HIPCHK(hipStreamSynchronize(c->stream));
-        for (int i = 0; i < np; ++i) rec[size_t(i) * LBDEM_P_REC + o1[k]] = buf[i];
-    }
-    return 0;
+    RecordMap m{};
+    m.cols = LBDEM_P_REC;
+    m.add(LBDEM_P_X0, d.x0, 3); m.add(LBDEM_P_X1, d.x1, 3); m.add(LBDEM_P_W1, d.w1, 3);
+    m.add(LBDEM_P_FHYDRO, d.FHydro, 3); m.add(LBDEM_P_MHYDRO, d.MHydro, 3);
+    m.add(LBDEM_P_FCONTACT, d.FContact, 3); m.add(LBDEM_P_MCONTACT, d.MContact, 3);
+    m.add(LBDEM_P_FLUB, d.FLub, 3); m.add(LBDEM_P_MLUB, d.MLub, 3); m.add(LBDEM_P_FREP, d.FRep, 3);
+    m.add(LBDEM_P_FTOTAL, d.FTotal, 3); m.add(LBDEM_P_MTOTAL, d.MTotal, 3); m.add(LBDEM_P_FGRAV, d.FGrav, 3);
+    m.add(LBDEM_P_FLUIDVOL, d.fluidVol, 1);
+    m.add(LBDEM_P_XIW, d.xiw, 3); m.add(LBDEM_P_XIO, d.xio, 3);
+    m.add(LBDEM_P_R, d.r, 1); m.add(LBDEM_P_M, d.m, 1);
+    return fetch_records(c, m, np, rec);
 }
 
 extern "C" int lbdem_get_objects(lbdem_ctx* c, double* rec) {
@@ -1448,24 +1448,15 @@ extern "C" int lbdem_get_objects(lbdem_ctx* c, double* rec) {
     const int no = c->dp.nObj;
     if (no == 0) return 0;
     const DemState& d = c->ds;
-    const double* srcs[] = {d.ox0, d.ox1, d.ow1, d.oFHydro, d.oMHydro, d.oFContact, d.oMContact, d.oFLub, d.oMLub,
-                            d.oFTotal, d.oMTotal, d.oFGrav};
-    const int offs[] = {LBDEM_O_X0, LBDEM_O_X1, LBDEM_O_W1, LBDEM_O_FHYDRO, LBDEM_O_MHYDRO, LBDEM_O_FCONTACT,
-                        LBDEM_O_MCONTACT, LBDEM_O_FLUB, LBDEM_O_MLUB, LBDEM_O_FTOTAL, LBDEM_O_MTOTAL, LBDEM_O_FGRAV};
-    std::vector<double> buf(3 * size_t(no));
-    for (int k = 0; k < 12; ++k) {
-        if (fetch(c, buf.data(), srcs[k], 3 * no)) return LBDEM_E_DEVICE;
-        HIPCHK(hipStreamSynchronize(c->stream));
-        for (int i = 0; i < no; ++i) for (int a = 0; a < 3; ++a) rec[size_t(i) * LBDEM_O_REC + offs[k] + a] = buf[3 * i + a];
-    }
-    const double* s1[] = {d.or_, d.om};
-    const int o1[] = {LBDEM_O_R, LBDEM_O_M};
-    for (int k = 0; k < 2; ++k) {
-        if (fetch(c, buf.data(), s1[k], no)) return LBDEM_E_DEVICE;
-        HIPCHK(hipStreamSynchronize(c->stream));
-        for (int i = 0; i < no; ++i) rec[size_t(i) * LBDEM_O_REC + o1[k]] = buf[i];
-    }
-    return 0;
+    RecordMap m{};
+    m.cols = LBDEM_O_REC;
+    m.add(LBDEM_O_X0, d.ox0, 3); m.add(LBDEM_O_X1, d.ox1, 3); m.add(LBDEM_O_W1, d.ow1, 3);
+    m.add(LBDEM_O_FHYDRO, d.oFHydro, 3); m.add(LBDEM_O_MHYDRO, d.oMHydro, 3);
+    m.add(LBDEM_O_FCONTACT, d.oFContact, 3); m.add(LBDEM_O_MCONTACT, d.oMContact, 3);
+    m.add(LBDEM_O_FLUB, d.oFLub, 3); m.add(LBDEM_O_MLUB, d.oMLub, 3);
+    m.add(LBDEM_O_FTOTAL, d.oFTotal, 3); m.add(LBDEM_O_MTOTAL, d.oMTotal, 3); m.add(LBDEM_O_FGRAV, d.oFGrav, 3);
+    m.add(LBDEM_O_R, d.or_, 1); m.add(LBDEM_O_M, d.om, 1);
+    return fetch_records(c, m, no, rec);
 }
 
 extern "C" int lbdem_get_bodies(lbdem_ctx* c, double* rec) {
@@ -1560,15 +1551,11 @@ extern "C" int lbdem_get_walls(lbdem_ctx* c, double* rec) {
     const int nw = c->dp.nWall;
     if (nw == 0) return 0;
     const DemState& d = c->ds;
-    const double* srcs[] = {d.wFHydro, d.wFContact, d.wFLub, d.wFTotal};
-    const int offs[] = {LBDEM_W_FHYDRO, LBDEM_W_FCONTACT, LBDEM_W_FLUB, LBDEM_W_FTOTAL};
-    std::vector<double> buf(3 * size_t(nw));
-    for (int k = 0; k < 4; ++k) {
-        if (fetch(c, buf.data(), srcs[k], 3 * nw)) return LBDEM_E_DEVICE;
-        HIPCHK(hipStreamSynchronize(c->stream));
-        for (int i = 0; i < nw; ++i) for (int a = 0; a < 3; ++a) rec[size_t(i) * LBDEM_W_REC + offs[k] + a] = buf[3 * i + a];
-    }
-    return 0;
+    RecordMap m{};
+    m.cols = LBDEM_W_REC;
+    m.add(LBDEM_W_FHYDRO, d.wFHydro, 3); m.add(LBDEM_W_FCONTACT, d.wFContact, 3);
+    m.add(LBDEM_W_FLUB, d.wFLub, 3); m.add(LBDEM_W_FTOTAL, d.wFTotal, 3);
+    return fetch_records(c, m, nw, rec);
 }
 
 extern "C" int lbdem_get_neighbors(lbdem_ctx* c, int cap, int* count, int* list) {

@@ -2265,18 +2265,40 @@ void lb_total_mass(const Box& b, double* out, hipStream_t s) {
     else launch<&k_total_mass<float>, 1024, 1>(1024, 256, s, b.g.N, b.type, (const float*)b.mass, out);
 }
 
+// node counts by kind, read as words of four type bytes (N type bytes are padded to 256 by the
+// allocator, the tail is taken byte by byte). Each thread keeps its counts in registers and a block
+// adds them once per kind: with one atomic per thread the five counters took 177 us on the
+// 256x320x256 box and 78 us on a 64^3 box (a quarter of a million atomics on one cache line).
+constexpr int CNT_BLOCKS = 512, CNT_KINDS = 5;
 __device__ inline void k_count_types(int64_t N, const uint8_t* type, int* counts) {
-    int c[5] = {0, 0, 0, 0, 0};
-    for (int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; i < N; i += int64_t(gridDim.x) * blockDim.x) {
-        const uint8_t t = type[i];
-        const uint8_t b = t & T_BASE;
+    __shared__ int red[CNT_KINDS];
+    if (threadIdx.x < CNT_KINDS) red[threadIdx.x] = 0;
+    __syncthreads();
+    int c[CNT_KINDS] = {0, 0, 0, 0, 0};
+    auto one = [&](uint32_t t) {
+        const uint32_t b = t & T_BASE;
         c[0] += b == T_FLUID; c[1] += b == T_IF; c[2] += b == T_OBJ; c[3] += (t & T_PMASK) != 0;
         c[4] += b == T_GAS;
+    };
+    const uint32_t* t32 = reinterpret_cast<const uint32_t*>(type);
+    const int64_t nw = N / 4, step = int64_t(gridDim.x) * blockDim.x, t0 = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+    for (int64_t i = t0; i < nw; i += step) {
+        const uint32_t w = t32[i];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) one((w >> (8 * k)) & 0xFFu);
     }
-    for (int j = 0; j < 5; ++j) if (c[j]) atomicAdd(&counts[j], c[j]);
+    for (int64_t i = 4 * nw + t0; i < N; i += step) one(type[i]);
+#pragma unroll
+    for (int j = 0; j < CNT_KINDS; ++j) {
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) c[j] += __shfl_xor(c[j], off, 64);
+        if (__lane_id() == 0 && c[j]) atomicAdd(&red[j], c[j]);
+    }
+    __syncthreads();
+    if (threadIdx.x < CNT_KINDS && red[threadIdx.x]) atomicAdd(&counts[threadIdx.x], red[threadIdx.x]);
 }
 void lb_count_types(const Box& b, int* counts, hipStream_t s) {
-    launch<&k_count_types, 1024, 1>(1024, 256, s, b.g.N, b.type, counts);
+    launch<&k_count_types, 256, 1>(CNT_BLOCKS, 256, s, b.g.N, b.type, counts);
 }
 
 }  // namespace lbdem

@@ -314,6 +314,19 @@ bool dem_step(const DemParams& p, DemState& d, DevScalars* sc, int demTimeStep, 
               hipEvent_t hydroReady = nullptr);
 void dem_refresh_views(const DemParams& p, DemState& d, hipStream_t s);
 
+// records of a download (particles, impactors, walls): column q of a record is component comp[q]
+// of an array with width[q] values per item
+constexpr int REC_COLS = 48;
+struct RecordMap {
+    const double* src[REC_COLS];
+    uint8_t width[REC_COLS], comp[REC_COLS];
+    int cols;
+    void add(int col, const double* p, int w) {
+        for (int a = 0; a < w; ++a) { src[col + a] = p; width[col + a] = uint8_t(w); comp[col + a] = uint8_t(a); }
+    }
+};
+void dem_pack_records(const RecordMap& m, int n, double* out, hipStream_t s);
+
 // run pool hooks: a context carves its buffers from [base, base+bytes) instead of allocating
 // them (set before lbdem_init); the stream a context enqueues on
 int ctx_use_region(lbdem_ctx* c, void* base, size_t bytes);

@@ -238,6 +238,11 @@ class Simulation:
         rc = lib.lib.lbdem_create(C.byref(params), C.byref(self.ctx))
         self._check(rc, "lbdem_create")
         n = len(particles.r)
+        # record counts of the downloads (fixed for the context's life)
+        self._n = n
+        self._no = len(objects.r)
+        self._nb = len(objects.bodies.r) if objects.bodies is not None else 0
+        self._nw = sum(1 for b in params.boundary if 5 <= b <= 8)
         size = np.ascontiguousarray(particles.size, dtype=np.int32)
         r = np.ascontiguousarray(particles.r, dtype=np.float64)
         x0 = np.ascontiguousarray(particles.x0, dtype=np.float64).reshape(-1)
@@ -289,7 +294,8 @@ class Simulation:
     def stress(self):
         """(global 5 x 3 x 3: totalStress, hydroStress, lubStress, contactStress, electroStress; STotal
         of every particle, n x 3 x 3; disp, n x 3) of the last DEM step."""
-        n = self.info()["nParticles"]
+        self.synchronize()
+        n = self._n
         g = np.zeros(45, np.float64)
         st = np.zeros(max(n, 1) * 9, np.float64)
         d = np.zeros(max(n, 1) * 3, np.float64)
@@ -300,7 +306,8 @@ class Simulation:
     def particle_stress(self) -> np.ndarray:
         """n x 44 records of lbdem_get_particle_stress (STotal, SElas, SVisc, SVisc_h, overlap, disp,
         coord, lub_coord) of the last DEM step."""
-        n = self.info()["nParticles"]
+        self.synchronize()
+        n = self._n
         rec = np.zeros((max(n, 1), 44), np.float64)
         self._check(self.lib.lib.lbdem_get_particle_stress(self.ctx, _ptr(rec, C.c_double)),
                     "lbdem_get_particle_stress")
@@ -362,32 +369,28 @@ class Simulation:
                     "lbdem_get_fields_noalloc" if noalloc else "lbdem_get_fields")
         return (f.reshape(Q, N) if want_f else None), m, n
 
+    def _records(self, fn: str, n: int, rec: int) -> np.ndarray:
+        """n records of a download, after the steps enqueued so far (raises what they reported)."""
+        self.synchronize()
+        out = np.zeros((max(n, 1), rec), np.float64)
+        self._check(getattr(self.lib.lib, fn)(self.ctx, _ptr(out, C.c_double)), fn)
+        return out[:n]
+
     def particles(self) -> np.ndarray:
-        n = self.info()["nParticles"]
-        rec = np.zeros((max(n, 1), P["REC"]), np.float64)
-        self._check(self.lib.lib.lbdem_get_particles(self.ctx, _ptr(rec, C.c_double)), "lbdem_get_particles")
-        return rec[:n]
+        return self._records("lbdem_get_particles", self._n, P["REC"])
 
     def objects(self) -> np.ndarray:
-        n = self.info()["nObjects"]
-        rec = np.zeros((max(n, 1), O["REC"]), np.float64)
-        self._check(self.lib.lib.lbdem_get_objects(self.ctx, _ptr(rec, C.c_double)), "lbdem_get_objects")
-        return rec[:n]
+        return self._records("lbdem_get_objects", self._no, O["REC"])
 
     def bodies(self) -> np.ndarray:
-        n = self.info()["nBodies"]
-        rec = np.zeros((max(n, 1), B["REC"]), np.float64)
-        self._check(self.lib.lib.lbdem_get_bodies(self.ctx, _ptr(rec, C.c_double)), "lbdem_get_bodies")
-        return rec[:n]
+        return self._records("lbdem_get_bodies", self._nb, B["REC"])
 
     def walls(self) -> np.ndarray:
-        n = self.info()["nWalls"]
-        rec = np.zeros((max(n, 1), W["REC"]), np.float64)
-        self._check(self.lib.lib.lbdem_get_walls(self.ctx, _ptr(rec, C.c_double)), "lbdem_get_walls")
-        return rec[:n]
+        return self._records("lbdem_get_walls", self._nw, W["REC"])
 
     def neighbors(self, cap: int = 64):
-        n = self.info()["nParticles"]
+        self.synchronize()
+        n = self._n
         cnt = np.zeros(max(n, 1), np.int32)
         lst = np.full((max(n, 1), cap), -1, np.int32)
         self._check(self.lib.lib.lbdem_get_neighbors(self.ctx, cap, _ptr(cnt, C.c_int), _ptr(lst, C.c_int)),

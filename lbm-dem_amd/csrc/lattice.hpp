@@ -1,0 +1,130 @@
+// Device helpers shared by the lattice kernels (lb.hip and the fused kernel's translation units).
+#pragma once
+#include "lbdem_internal.hpp"
+#include "launch.hpp"
+
+#include <climits>
+
+namespace lbdem {
+
+template <typename S> struct Types;
+template <> struct Types<double> { using C = double; using M = double; };
+template <> struct Types<float> { using C = float; using M = float; };
+template <> struct Types<__half> { using C = float; using M = float; };
+
+__device__ inline bool is_active(uint8_t t) { t &= T_BASE; return t == T_FLUID || t == T_IF; }
+
+// insideSphere with the reference's rounding (myvector.cpp:171-176): no contraction
+__device__ inline bool inside_sphere(double px, double py, double pz, double cx, double cy, double cz, double r) {
+#pragma clang fp contract(off)
+    const double dx = px - cx, dy = py - cy, dz = pz - cz;
+    const double s = dx * dx + dy * dy + dz * dz;
+    return s < r * r;
+}
+
+__device__ inline void cell_xyz(const Geom& g, int64_t i, int& x, int& y, int& z) {
+    if ((uint64_t(i) | uint64_t(g.X) * uint64_t(g.Y)) <= 0xffffffffull) {  // 32-bit quotients
+        const uint32_t u = uint32_t(i), sxy = uint32_t(g.X) * uint32_t(g.Y);
+        const uint32_t zz = u / sxy, rem = u - zz * sxy, yy = rem / uint32_t(g.X);
+        z = int(zz);
+        y = int(yy);
+        x = int(rem - yy * uint32_t(g.X));
+        return;
+    }
+    z = int(i / (int64_t(g.X) * g.Y));
+    const int64_t rem = i - int64_t(z) * g.X * g.Y;
+    y = int(rem / g.X);
+    x = int(rem - int64_t(y) * g.X);
+}
+
+// lattice vectors for a direction index known only at run time: 2-bit fields of packed words
+constexpr uint64_t pack_dir(int axis) {
+    uint64_t k = 0;
+    for (int q = 0; q < Q; ++q) k |= uint64_t((axis == 0 ? cxq(q) : axis == 1 ? cyq(q) : czq(q)) + 1) << (2 * q);
+    return k;
+}
+constexpr uint64_t PACK_CX = pack_dir(0), PACK_CY = pack_dir(1), PACK_CZ = pack_dir(2);
+constexpr bool opp_rule_ok() {
+    for (int q = 1; q < Q; ++q)
+        if (oppq(q) != ((q - 1) ^ 1) + 1) return false;
+    return true;
+}
+static_assert(opp_rule_ok(), "opposite-direction rule");
+__device__ inline int cx_rt(int q) { return int((PACK_CX >> (2 * q)) & 3u) - 1; }
+__device__ inline int cy_rt(int q) { return int((PACK_CY >> (2 * q)) & 3u) - 1; }
+__device__ inline int cz_rt(int q) { return int((PACK_CZ >> (2 * q)) & 3u) - 1; }
+__device__ inline int opp_rt(int q) { return q == 0 ? 0 : ((q - 1) ^ 1) + 1; }
+__device__ inline double w_rt(int q) { return q == 0 ? 12.0 / 36.0 : (q < 7 ? 2.0 / 36.0 : 1.0 / 36.0); }
+// Per-axis index offsets of the wrapped neighbour rule: nb(q) = i + ox[cx+1] + oy[cy+1] + oz[cz+1]
+// (offsets fit 32 bits: initialisation rejects boxes with 19*N >= 2^31)
+struct Offs {
+    int32_t ox[3], oy[3], oz[3];
+    __device__ Offs(const Geom& g, int x, int y, int z) {
+        const int32_t sy = g.X, sz = g.X * g.Y;
+        ox[1] = 0; oy[1] = 0; oz[1] = 0;
+        ox[0] = (x - 1 == 0 && g.per[0]) ? g.X - 3 : -1;
+        ox[2] = (x + 1 == g.X - 1 && g.per[1]) ? -(g.X - 3) : 1;
+        oy[0] = (y - 1 == 0 && g.per[2]) ? (g.Y - 3) * sy : -sy;
+        oy[2] = (y + 1 == g.Y - 1 && g.per[3]) ? -(g.Y - 3) * sy : sy;
+        oz[0] = (z - 1 == 0 && g.per[4]) ? (g.Z - 3) * sz : -sz;
+        oz[2] = (z + 1 == g.Z - 1 && g.per[5]) ? -(g.Z - 3) * sz : sz;
+    }
+    // selects and packed direction words, not indexed arrays: a direction known only at run
+    // time must not put tables or offsets in scratch memory
+    __device__ int32_t d(int q) const {
+        const int cx = cx_rt(q), cy = cy_rt(q), cz = cz_rt(q);
+        return (cx < 0 ? ox[0] : (cx > 0 ? ox[2] : 0)) + (cy < 0 ? oy[0] : (cy > 0 ? oy[2] : 0)) +
+               (cz < 0 ? oz[0] : (cz > 0 ? oz[2] : 0));
+    }
+};
+
+__device__ inline int32_t offs_rt(const Offs& o, int q) { return o.d(q); }
+
+// slot holding the post-streaming population q of cell i in layout L (0 natural, 1 swapped)
+__device__ inline int64_t load_slot(const Geom& g, int64_t i, const Offs& o, int q, int L) {
+    return L == 0 ? int64_t(q) * g.N + i : int64_t(opp_rt(q)) * g.N + i + o.d(opp_rt(q));
+}
+
+template <typename C>
+__device__ inline void equilibrium_offsets(C n, C ux, C uy, C uz, C* geq) {
+    const C usq = ux * ux + uy * uy + uz * uz;
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+        const C cu = C(cxq(q)) * ux + C(cyq(q)) * uy + C(czq(q)) * uz;
+        geq[q] = C(wq(q)) * ((n - C(1)) + n * (C(3) * cu + C(4.5) * cu * cu - C(1.5) * usq));
+    }
+}
+
+constexpr int FX = FUSED_TILE_X, FY = FUSED_TILE_Y;  // 64x4 threads: 4 row segments, each lane walks FZ cells
+                                                     // along z (FZ 1, 2, 4 or 8, chosen per box)
+constexpr int HS = 64;                  // per-block particle hash slots
+constexpr int PART_STRIDE = PART_STRIDE_;  // per-block partials: obj (7*MAX_OBJ_PART) + walls 18
+constexpr int MAX_OBJ_PART = 2;
+// block partials of the fused kernel (sPart, doubles): object o's force and torque at 7 o, the
+// bounce-back mass term of all object links at 6, wall w's force at 7 MAX_OBJ_PART + 3 w
+constexpr int PART_BB = 6, PART_WALL = 7 * MAX_OBJ_PART;
+
+// check nodes and source directions of the slip reflection (LB.cpp:1454-1482; see k_slip)
+__host__ __device__ constexpr int slip1Check(int j) {
+    constexpr int c[Q] = {0, 0, 0, 0, 0, 0, 0, 1, 2, 3, 4, 3, 4, 5, 6, 1, 2, 6, 5};
+    return c[j];
+}
+__host__ __device__ constexpr int slip1Dir(int j) {
+    constexpr int c[Q] = {0, 0, 0, 0, 0, 0, 0, 9, 10, 8, 7, 13, 14, 12, 11, 18, 17, 15, 16};
+    return c[j];
+}
+__host__ __device__ constexpr int slip2Check(int j) {
+    constexpr int c[Q] = {0, 0, 0, 0, 0, 0, 0, 3, 4, 2, 1, 5, 6, 4, 3, 5, 6, 1, 2};
+    return c[j];
+}
+__host__ __device__ constexpr int slip2Dir(int j) {
+    constexpr int c[Q] = {0, 0, 0, 0, 0, 0, 0, 10, 9, 7, 8, 14, 13, 11, 12, 17, 18, 16, 15};
+    return c[j];
+}
+
+// the fused step in storage type S (fused.hpp, instantiated once per storage type)
+template <typename S>
+void launch_fused(Box& b, const Consts& k, const PartLB* plb, const ObjLB* olb, DevScalars* sc, bool diag,
+                  bool storeVel, hipStream_t s, hipEvent_t ev0, hipEvent_t ev1);
+
+}  // namespace lbdem

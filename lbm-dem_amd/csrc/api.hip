@@ -72,13 +72,9 @@ struct lbdem_ctx {
     std::vector<double> brad, bx0, bx1, bk, bL0;  // bodies (lbdem_set_bodies)
     // device
     hipStream_t stream = nullptr;
-    // lbdem_cycle defers a step's free-surface pass to the start of the next step and runs it on
-    // fsStream beside that step's DEM step (the two touch disjoint state); the coupling step
-    // waits for both
-    hipStream_t fsStream = nullptr;
-    hipEvent_t evFork = nullptr, evJoin = nullptr, evHydro = nullptr;
+    // lbdem_cycle leaves a step's free surface to the launches of the next step's DEM step (lb_front;
+    // the two touch disjoint state)
     bool fsDeferred = false;
-    bool streamError = false;  // an event record or wait of the overlap failed
     Box box{};
     Consts k{};
     DemParams dp{};
@@ -92,11 +88,14 @@ struct lbdem_ctx {
     char* region = nullptr;
     size_t regionSize = 0, regionUsed = 0;
     size_t devBytes = 0;
-    // steady-state step pairs replayed from a captured HIP graph (see lbdem_cycle)
-    // one captured pair per phase: AA parity x which history buffer is current
+    // steady-state steps replayed from captured HIP graphs (see lbdem_cycle): one per chunk length and
+    // phase (AA parity x which history buffer is current)
+    static constexpr int NCHUNK = 3, PHASES = 4;
+    static constexpr int CHUNK[NCHUNK] = {16, 4, 1};
     bool useGraphs = true, graphFailed = false;
-    hipGraph_t graph[4] = {nullptr, nullptr, nullptr, nullptr};
-    hipGraphExec_t graphExec[4] = {nullptr, nullptr, nullptr, nullptr};
+    hipGraph_t graph[NCHUNK][PHASES] = {};
+    hipGraphExec_t graphExec[NCHUNK][PHASES] = {};
+    int asked[PHASES] = {0, 0, 0, 0};  // single steps run at this phase without a graph
     double* xiFirst = nullptr;  // the buffer that is current at initialisation
     lbdem_batch* batch = nullptr;  // set while the context is advanced through a batch
     // tile tuner: the first LB steps run the fused kernel once per AA parity with each candidate
@@ -144,22 +143,18 @@ struct lbdem_ctx {
         return p;
     }
     ~lbdem_ctx() {
-        for (int q = 0; q < 4; ++q) {
-            if (graphExec[q]) (void)hipGraphExecDestroy(graphExec[q]);
-            if (graph[q]) (void)hipGraphDestroy(graph[q]);
-        }
+        for (int n = 0; n < NCHUNK; ++n)
+            for (int q = 0; q < PHASES; ++q) {
+                if (graphExec[n][q]) (void)hipGraphExecDestroy(graphExec[n][q]);
+                if (graph[n][q]) (void)hipGraphDestroy(graph[n][q]);
+            }
         for (hipEvent_t e : evPool) (void)hipEventDestroy(e);
         for (auto& pr : tuneEv)
             for (hipEvent_t e : pr)
                 if (e) (void)hipEventDestroy(e);
-        if (fsStream) (void)hipStreamSynchronize(fsStream);
         if (stream) (void)hipStreamSynchronize(stream);
         for (void* p : allocs) (void)hipFree(p);
         if (dTmp && !tmpPlanned) (void)hipFree(dTmp);
-        if (evFork) (void)hipEventDestroy(evFork);
-        if (evJoin) (void)hipEventDestroy(evJoin);
-        if (evHydro) (void)hipEventDestroy(evHydro);
-        if (fsStream) (void)hipStreamDestroy(fsStream);
         if (stream) (void)hipStreamDestroy(stream);
     }
     // download scratch: the planned buffer, replaced by a hipMalloc of its own when a download
@@ -495,7 +490,6 @@ static bool plan_buffers(const Plan& p, Box& b, DemState& d, DevScalars*& sc, do
     A(b.coverCount, COVER_BLOCKS + UNCOVER_BLOCKS_MAX);
     A(b.changed, size_t(b.changedCap));
     A(b.blockPart, size_t(b.blockPartCap));
-    A(b.blockFlag, size_t(std::max(fused_grid_blocks(p.g, 1, LBDEM_PREC_FP32), fused_grid_blocks(p.g, 1, LBDEM_PREC_FP16))));
     A(b.bcm, N);
     if (p.visc) A(b.visc, N * p.celt);
     else b.visc = nullptr;
@@ -517,11 +511,8 @@ static bool plan_buffers(const Plan& p, Box& b, DemState& d, DevScalars*& sc, do
     A(d.xiCur, 3 * slots); A(d.xiNext, 3 * slots);
     A(d.cellCount, size_t(p.ncell)); A(d.cellStart, size_t(p.ncell)); A(d.cellFill, size_t(p.ncell));
     A(d.cellItems, np1); A(d.cellKey, np1);
-    A(d.objContrib, np1 * 12 * no1);
-    A(d.wallContrib, np1 * 6 * size_t(std::max(p.nw, 1)));
-    A(d.objSum, 12 * MAX_OBJECTS);
-    A(d.redPart, 2 * 64 * 12 * MAX_OBJECTS);
-    A(d.wallSum, 6 * MAX_WALLS);
+    A(d.redPart, size_t(dem_force_blocks(int(np1))) * DEM_RED_COLS);
+    A(d.redFlag, size_t(dem_force_blocks(int(np1))));
     A(d.blockMax, VEL_SLOTS);
     double** ovecs[] = {&d.ox0, &d.ox1, &d.ow1, &d.oFHydro, &d.oMHydro, &d.oFContact, &d.oMContact, &d.oFLub,
                         &d.oMLub, &d.oFTotal, &d.oMTotal, &d.oFGrav};
@@ -614,10 +605,6 @@ extern "C" int lbdem_init(lbdem_ctx* c) {
         return c->fail(LBDEM_E_DEVICE, std::string("hipGetSymbolAddress of the download scratch failed: ") +
                                            hipGetErrorString(hipError_t(e)));
     HIPCHK(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
-    HIPCHK(hipStreamCreateWithFlags(&c->fsStream, hipStreamNonBlocking));
-    HIPCHK(hipEventCreateWithFlags(&c->evFork, hipEventDisableTiming));
-    HIPCHK(hipEventCreateWithFlags(&c->evJoin, hipEventDisableTiming));
-    HIPCHK(hipEventCreateWithFlags(&c->evHydro, hipEventDisableTiming));
     if (const char* g = std::getenv("LBDEM_GRAPHS")) c->useGraphs = std::atoi(g) != 0;
     if (!c->tuned)
         for (auto& pr : c->tuneEv)
@@ -851,7 +838,7 @@ extern "C" int lbdem_init(lbdem_ctx* c) {
 
     c->xiFirst = d.xiCur;
     dem_refresh_views(P, d, st);
-    dem_neighbor_list(P, d, c->sc, true, st);   // DEM.cpp:294
+    lb_front(b, k, c->sc, false, false, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, &P, &d, 0, true, st);  // the list, DEM.cpp:294
     if (c->restart) {
         const size_t nr = rNode.size();
         double* dRec = nullptr;
@@ -910,23 +897,27 @@ static int check_errors(lbdem_ctx* c) {
 }
 
 // --------------------------- steps ---------------------------
-// hydroReady: the previous LB step's hydrodynamic sums are finalised on another stream; the
-// integration (the first DEM launch that reads them) waits for it
-static void enqueue_dem(lbdem_ctx* c, hipEvent_t hydroReady = nullptr) {  // DEM::discreteElementStep (DEM.cpp:359-401)
+// the launches before the coupling (lb_front): the finalisation of the fused kernel's sums and the free
+// surface of the last LB step, the neighbour list and the forces of the next DEM step
+static void enqueue_front(lbdem_ctx* c, bool hydro, bool fs, bool dem) {
+    lb_front(c->box, c->k, c->sc, hydro, fs, c->ds.FHydro, c->ds.MHydro, c->ds.fluidVol, c->ds.oFHydro, c->ds.oMHydro,
+             c->ds.wFHydro, dem ? &c->dp : nullptr, dem ? &c->ds : nullptr, int(c->demTimeStep), false, c->stream);
+}
+// DEM::discreteElementStep (DEM.cpp:359-401), with the free surface (and the sums before it) that the
+// previous LB step left
+static void enqueue_dem(lbdem_ctx* c, bool fs = false) {
     c->demTimeStep++;
     c->demTime += c->deltat;
-    dem_neighbor_list(c->dp, c->ds, c->sc, false, c->stream);
-    if (!dem_step(c->dp, c->ds, c->sc, int(c->demTimeStep), c->stream, hydroReady)) c->streamError = true;
+    enqueue_front(c, fs, fs, true);
+    dem_integrate(c->dp, c->ds, int(c->demTimeStep), c->stream);
 }
-static void enqueue_coupling(lbdem_ctx* c) {  // LB::latticeBoltzmannCouplingStep (LB.cpp:432-467)
+// LB::latticeBoltzmannCouplingStep (LB.cpp:432-467); lbFollows: the LB step is enqueued next
+static void enqueue_coupling(lbdem_ctx* c, bool lbFollows = false) {
     // the lists of the rebuild resolve overlaps unless the reference builds none (no z-cell)
     const bool lists = c->dp.nlx == 0 || c->dp.nlz > 0;
     const bool cells = c->dp.nlx > 0 && c->dp.nlz > 0;  // the rebuild sorted the particles by link cell
-    lb_flags_rebuild_compute(c->box, c->k, c->ds.plb, c->sc, c->ds.nbrCount, c->ds.nbrList, lists,
-                             cells ? c->ds.cellItems : nullptr, c->stream);
-    lb_object_update(c->box, c->k, c->ds.olb, c->sc, c->stream);
-    lb_flags_rebuild_apply(c->box, c->sc, c->stream);
-    lb_find_new_active(c->box, c->k, c->ds.plb, c->sc, c->stream);
+    lb_coupling(c->box, c->k, c->ds.plb, c->ds.olb, c->sc, c->ds.nbrCount, c->ds.nbrList, lists,
+                cells ? c->ds.cellItems : nullptr, lbFollows, c->stream);
 }
 // picks the fastest candidate from the timed launches (waits for the last of them)
 static void finish_tuning(lbdem_ctx* c) {
@@ -948,14 +939,12 @@ static void finish_tuning(lbdem_ctx* c) {
     c->tuned = true;
 }
 
-// the particle, impactor and wall sums of the fused kernel (and the counters of the free-surface
-// pass that follows)
-static void enqueue_hydro(lbdem_ctx* c, hipStream_t s) {
+// the particle, impactor and wall sums of the fused kernel
+static void enqueue_hydro(lbdem_ctx* c) {
     lb_hydro_finalize(c->box, c->k, c->ds.FHydro, c->ds.MHydro, c->ds.fluidVol, c->sc, c->ds.oFHydro, c->ds.oMHydro,
-                      c->ds.wFHydro, true, s);
+                      c->ds.wFHydro, true, c->stream);
 }
-// finalize = false: the hydrodynamic finalisation is left to the next step's fork (it goes with
-// the deferred free surface)
+// finalize = false: the sums are finalised with the free surface that follows
 static void enqueue_lb(lbdem_ctx* c, bool finalize = true) {  // LB::latticeBolzmannStep (LB.cpp:400-418)
     if (!c->forceField && !c->lbFReset) {  // LB.cpp:1303-1305
         c->k.lbF[0] = c->k.lbF[1] = c->k.lbF[2] = 0.0;
@@ -987,9 +976,8 @@ static void enqueue_lb(lbdem_ctx* c, bool finalize = true) {  // LB::latticeBolz
     lb_fused_step(c->box, c->k, c->ds.plb, c->ds.olb, c->sc, true, storeVel || c->stress, c->stream, e0, e1);
     if (c->stress)
         lb_hydro_stress(c->box, c->ds.plb, c->dp.nPart, c->unit.Length, c->unit.Force, c->ds.shydro, c->stream);
-    if (finalize) enqueue_hydro(c, c->stream);
+    if (finalize) enqueue_hydro(c);
 }
-static void enqueue_fs(lbdem_ctx* c, hipStream_t s) { lb_free_surface(c->box, c->k, c->sc, s); }
 
 #define NEED_INIT                                                           \
     if (!c) return LBDEM_E_ARG;                                             \
@@ -1001,72 +989,55 @@ extern "C" int lbdem_lb_step(lbdem_ctx* c) { NEED_INIT; if (c->batch) return c->
 extern "C" int lbdem_fs_step(lbdem_ctx* c) {
     NEED_INIT;
     if (c->batch) return c->fail(LBDEM_E_STATE, "in a batch");
-    if (c->freeSurface) enqueue_fs(c, c->stream);
+    if (c->freeSurface) enqueue_front(c, false, true, false);
     HIPCHK(hipGetLastError());
     return 0;
 }
 
-// one goCycle (main.cpp:38-67) minus the output. With deferFs the step's free-surface pass is
-// left for the next step (or flush_fs), which runs it on fsStream beside its DEM step: the free
-// surface reads and writes the lattice (populations, types, mass, interface lists) and the DEM
-// step the particles and the hydrodynamic sums the LB step left, so the order between them does
-// not matter; the coupling step waits for both, as it follows both in goCycle.
-static void enqueue_step(lbdem_ctx* c, bool deferFs = false) {
+// the free surface left by the last step, with the finalisation of the sums before it
+static void flush_fs(lbdem_ctx* c) {
+    if (!c->fsDeferred) return;
+    c->fsDeferred = false;
+    enqueue_front(c, true, true, false);
+}
+// one goCycle (main.cpp:38-67) minus the output. With deferFs the step's free surface is left for the
+// next step (or flush_fs), whose DEM step it shares launches with: the free surface reads and writes
+// the lattice and the DEM forces the particles, so the order between them does not matter, and the
+// integration, the first to read the fused kernel's sums, follows both.
+static void enqueue_step(lbdem_ctx* c, bool deferFs) {
     c->realTime += c->unit.Time;
     ++c->currentTimeStep;
     ++c->lbTime;
-    bool join = false;
-    hipEvent_t hydroReady = nullptr;
-    if (c->fsDeferred) {  // the previous step's hydrodynamic sums and free surface (LB.cpp:422-430)
+    if (c->prm.demSolve) {
+        const bool fs = c->fsDeferred;
         c->fsDeferred = false;
-        if (c->prm.demSolve) {
-            if (hipEventRecord(c->evFork, c->stream) != hipSuccess ||
-                hipStreamWaitEvent(c->fsStream, c->evFork, 0) != hipSuccess)
-                c->streamError = true;
-            enqueue_hydro(c, c->fsStream);
-            if (hipEventRecord(c->evHydro, c->fsStream) != hipSuccess) c->streamError = true;
-            hydroReady = c->evHydro;
-            enqueue_fs(c, c->fsStream);
-            if (hipEventRecord(c->evJoin, c->fsStream) != hipSuccess) c->streamError = true;
-            join = true;
-        } else {
-            enqueue_hydro(c, c->stream);
-            enqueue_fs(c, c->stream);
-        }
+        enqueue_dem(c, fs);
+    } else {
+        flush_fs(c);
     }
-    if (c->prm.demSolve) enqueue_dem(c, hydroReady);
-    if (join && hipStreamWaitEvent(c->stream, c->evJoin, 0) != hipSuccess) c->streamError = true;
     if (c->demTime >= c->prm.demInitialRepeat) {
-        if (c->prm.demSolve) enqueue_coupling(c);
-        const bool defer = deferFs && c->freeSurface;
-        enqueue_lb(c, !defer);
-        if (c->freeSurface) {
-            if (defer) c->fsDeferred = true;
-            else enqueue_fs(c, c->stream);
-        }
+        if (c->prm.demSolve) enqueue_coupling(c, true);
+        enqueue_lb(c, !c->freeSurface);
+        c->fsDeferred = c->freeSurface;
+        if (!deferFs) flush_fs(c);
     } else if (c->demTime <= c->prm.demInitialRepeat) {
         if (c->prm.demSolve) enqueue_coupling(c);
     }
 }
-// the deferred hydrodynamic finalisation and free-surface pass, on the context's stream (every
-// lbdem_cycle ends with them)
-static void flush_fs(lbdem_ctx* c) {
-    if (!c->fsDeferred) return;
-    c->fsDeferred = false;
-    enqueue_hydro(c, c->stream);
-    enqueue_fs(c, c->stream);
+// n steps that leave whole steps behind
+static void enqueue_steps(lbdem_ctx* c, int n) {
+    for (int k = 0; k < n; ++k) enqueue_step(c, true);
+    flush_fs(c);
 }
-// lbdem_cycle overlaps a step's free surface with the next DEM step
-static bool overlap_fs(const lbdem_ctx* c) { return c->freeSurface && c->prm.demSolve; }
 
-// A pair of steps has the same launches with the same arguments as every later pair once
+// A step has the same launches with the same arguments as every later step of its phase once
 //  * every step compares its DEM step number past objWaitTime (the only use of the number in
 //    the kernels: DEM.cpp:716-730, 777-783, 2727),
 //  * the LB path runs (demTime >= demInitialRepeat, which stays true),
 //  * the one-off reset of the lattice force (LB.cpp:1303-1305) is done;
 // the AA parity and the tangential-history buffers alternate with period two. Every
-// data-dependent branch is a device flag, so the pair can be captured once and replayed.
-static bool steady_pairs(const lbdem_ctx* c) {
+// data-dependent branch is a device flag, so steps can be captured once and replayed.
+static bool steady_steps(const lbdem_ctx* c) {
     if (!c->useGraphs || c->graphFailed || c->profiling || !c->tuned) return false;
     if (c->velState == 1) return false;  // the next LB step stores every node's velocity
     if (c->prm.demSolve && c->demTimeStep < unsigned(std::max(c->prm.objWaitTime, 0)) + 1u) return false;
@@ -1074,12 +1045,6 @@ static bool steady_pairs(const lbdem_ctx* c) {
     if (!c->forceField && !c->lbFReset) return false;
     return true;
 }
-static bool graph_ready(const lbdem_ctx* c) {
-    if (!steady_pairs(c)) return false;
-    if (c->fsDeferred != overlap_fs(c)) return false;  // a pair starts with the previous free surface
-    return true;
-}
-
 struct HostStepState {
     unsigned lbTime, demTimeStep, currentTimeStep;
     double demTime, realTime;
@@ -1102,10 +1067,11 @@ static void restore_host(lbdem_ctx* c, const HostStepState& h) {
 // the launches of a step pair depend on the phase: AA parity and current history buffer
 static int graph_phase(const lbdem_ctx* c) { return c->box.parity * 2 + (c->ds.xiCur == c->xiFirst ? 0 : 1); }
 
-// captures two steps into c->graphExec[phase] and launches them: 1 on success; 0 when capture
+// captures CHUNK[n] steps into c->graphExec[n][phase] and launches them: 1 on success; 0 when capture
 // or instantiation failed (host state restored, graphs switched off for this context, nothing
-// executed); -1 when the launch of the captured steps failed
-static int capture_pair(lbdem_ctx* c) {
+// executed); -1 when the launch of the captured steps failed. The steps are one chain of launches on
+// one stream: a graph without branches.
+static int capture_steps(lbdem_ctx* c, int n) {
     const int ph = graph_phase(c);
     const HostStepState h = save_host(c);
     if (hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal) != hipSuccess) {
@@ -1113,79 +1079,84 @@ static int capture_pair(lbdem_ctx* c) {
         c->graphFailed = true;
         return 0;
     }
-    const bool defer = overlap_fs(c);
-    enqueue_step(c, defer);
-    enqueue_step(c, defer);
+    enqueue_steps(c, lbdem_ctx::CHUNK[n]);
     hipGraph_t g = nullptr;
     const hipError_t e = hipStreamEndCapture(c->stream, &g);
     hipGraphExec_t ge = nullptr;
-    if (e != hipSuccess || !g || c->streamError || hipGraphInstantiate(&ge, g, nullptr, nullptr, 0) != hipSuccess) {
+    if (e != hipSuccess || !g || hipGraphInstantiate(&ge, g, nullptr, nullptr, 0) != hipSuccess) {
         if (g) (void)hipGraphDestroy(g);
         (void)hipGetLastError();
         restore_host(c, h);
-        c->streamError = false;
         c->graphFailed = true;
         return 0;
     }
-    c->graph[ph] = g;
-    c->graphExec[ph] = ge;
-    // the host counters now describe the two captured steps; run them
+    c->graph[n][ph] = g;
+    c->graphExec[n][ph] = ge;
+    // the host counters now describe the captured steps; run them
     return hipGraphLaunch(ge, c->stream) == hipSuccess ? 1 : -1;
 }
 
-// what two enqueue_step calls do to the host counters (AA parity and history buffers return to
-// their values after a pair)
-static void advance_pair(lbdem_ctx* c) {
-    c->velState = 0;  // two LB steps without the velocity store
-    for (int k = 0; k < 2; ++k) {
+// what n enqueue_step calls do to the host counters; an odd n also flips the AA parity and, with
+// particles, the history buffers
+static void advance_steps(lbdem_ctx* c, int n) {
+    c->velState = 0;  // LB steps without the velocity store
+    for (int k = 0; k < n; ++k) {
         c->realTime += c->unit.Time;
         ++c->currentTimeStep;
         ++c->lbTime;
         if (c->prm.demSolve) { ++c->demTimeStep; c->demTime += c->deltat; }
     }
+    if (n % 2) {
+        c->box.parity ^= 1;
+        if (c->prm.demSolve && c->dp.nPart > 0) std::swap(c->ds.xiCur, c->ds.xiNext);
+    }
 }
 
+// Steps in chunks of 16, 4 and 1 that are captured once per phase and replayed: within a chunk every
+// free surface but the last shares the next step's launches, and a replay costs the host one call.
+// Chunks of 16 and 4 are captured when first asked for, single steps when a phase asks a second time.
 extern "C" int lbdem_cycle(lbdem_ctx* c, int nsteps) {
     NEED_INIT;
     if (c->batch) return c->fail(LBDEM_E_STATE, "the context is advanced through its batch");
     int s = 0;
     while (s < nsteps) {
-        if (nsteps - s >= 2 && graph_ready(c)) {
-            if (hipGraphExec_t ge = c->graphExec[graph_phase(c)]) {
+        if (steady_steps(c)) {
+            flush_fs(c);  // a chunk starts with whole steps behind it
+            const int ph = graph_phase(c);
+            int n = 0;
+            while (lbdem_ctx::CHUNK[n] > nsteps - s) ++n;
+            if (hipGraphExec_t ge = c->graphExec[n][ph]) {
                 HIPCHK(hipGraphLaunch(ge, c->stream));
-                advance_pair(c);
-                s += 2;
+                advance_steps(c, lbdem_ctx::CHUNK[n]);
+                s += lbdem_ctx::CHUNK[n];
                 continue;
             }
-            const int r = capture_pair(c);
-            if (r < 0) {
-                flush_fs(c);
-                return c->fail(LBDEM_E_DEVICE, "launch of the captured step pair failed");
-            }
-            if (r == 1) {
-                s += 2;
-                continue;
+            if (lbdem_ctx::CHUNK[n] > 1 || c->asked[ph]++ > 0) {
+                const int r = capture_steps(c, n);
+                if (r < 0) return c->fail(LBDEM_E_DEVICE, "launch of the captured steps failed");
+                if (r == 1) {
+                    s += lbdem_ctx::CHUNK[n];
+                    continue;
+                }
             }
         }
-        enqueue_step(c, overlap_fs(c));
+        enqueue_step(c, true);
         ++s;
     }
     flush_fs(c);  // every call leaves whole steps behind
-    if (c->streamError) {
-        c->streamError = false;
-        return c->fail(LBDEM_E_DEVICE, "ordering of the free-surface stream failed");
-    }
     HIPCHK(hipGetLastError());
     return 0;
 }
 
 static void drop_graphs(lbdem_ctx* c) {
-    for (int q = 0; q < 4; ++q) {
-        if (c->graphExec[q]) (void)hipGraphExecDestroy(c->graphExec[q]);
-        if (c->graph[q]) (void)hipGraphDestroy(c->graph[q]);
-        c->graphExec[q] = nullptr;
-        c->graph[q] = nullptr;
-    }
+    for (int n = 0; n < lbdem_ctx::NCHUNK; ++n)
+        for (int q = 0; q < lbdem_ctx::PHASES; ++q) {
+            if (c->graphExec[n][q]) (void)hipGraphExecDestroy(c->graphExec[n][q]);
+            if (c->graph[n][q]) (void)hipGraphDestroy(c->graph[n][q]);
+            c->graphExec[n][q] = nullptr;
+            c->graph[n][q] = nullptr;
+        }
+    std::fill(std::begin(c->asked), std::end(c->asked), 0);
 }
 
 extern "C" int lbdem_set_tile(lbdem_ctx* c, int tileZ) {
@@ -1220,12 +1191,10 @@ extern "C" int lbdem_get_tuning(lbdem_ctx* c, lbdem_tuning* t) {
         t->candidateZ[q] = lbdem_ctx::CAND[q];
         t->candidateMs[q] = c->tuneMs[q];
     }
-    // Between calls the deferred free-surface pass has been flushed, so an lbdem_cycle call takes
-    // its first step alone and replays pairs from the phase one step later (AA parity and, with
-    // particles, the history buffer flip every step).
-    int next = graph_phase(c);
-    if (!c->fsDeferred && overlap_fs(c)) next ^= 2 | ((c->prm.demSolve && !c->pr.empty()) ? 1 : 0);
-    t->pairCaptured = steady_pairs(c) && c->graphExec[next] ? 1 : 0;
+    // a chunk that the next lbdem_cycle call of its length replays
+    t->pairCaptured = 0;
+    for (int n = 0; n < lbdem_ctx::NCHUNK; ++n)
+        if (steady_steps(c) && c->graphExec[n][graph_phase(c)]) t->pairCaptured = 1;
     return 0;
 }
 
@@ -1704,7 +1673,7 @@ struct lbdem_batch {
     }
 };
 
-// the contexts' start-up is over: the launches of a step pair repeat (see graph_ready)
+// the contexts' start-up is over: the launches of a step pair repeat (see steady_steps)
 static bool steady(const lbdem_ctx* c) {
     if (!c->initialised || c->profiling || !c->tuned) return false;
     if (c->prm.demSolve && c->demTimeStep < unsigned(std::max(c->prm.objWaitTime, 0)) + 1u) return false;
@@ -1729,8 +1698,7 @@ static int batch_record(lbdem_batch* B, BatchPhase& P) {
         lbdem_ctx* c = B->m[i];
         saved[i] = save_host(c);
         current_recorder() = &rec[i];
-        enqueue_step(c);
-        enqueue_step(c);
+        enqueue_steps(c, 2);
         current_recorder() = nullptr;
     }
     auto undo = [&](const std::string& why) {
@@ -1961,7 +1929,7 @@ extern "C" int lbdem_batch_cycle(lbdem_batch* B, int nsteps) {
         if (!P.recorded) {
             if (int e = batch_record(B, P)) return e;  // advances the members' counters
         } else {
-            for (lbdem_ctx* c : B->m) advance_pair(c);
+            for (lbdem_ctx* c : B->m) advance_steps(c, 2);
         }
         batch_prepare_pair(B, P);  // host work done before the timed launch
         if (slot >= 0) BATCHCHK(hipEventRecord(B->tuneEv[slot][0], B->stream));

@@ -1,0 +1,19 @@
+// Redistribution and forces (front.hpp) with float node masses.
+#include "front.hpp"
+
+namespace lbdem {
+
+template <>
+void launch_front6<float>(const RedistArgs& r, float* mass, const ForceArgs& f, hipStream_t s) {
+    const int g = r.blocks + f.blocks, bs = FS_THREADS;
+    const bool few = f.p.nPart <= DEM_FEW;
+    if (f.p.stress) {
+        if (few) launch<&k_front6<float, true, DEM_LANES_FEW>, FS_THREADS, 1>(g, bs, s, r, mass, f);
+        else launch<&k_front6<float, true, DEM_LANES_MANY>, FS_THREADS, 1>(g, bs, s, r, mass, f);
+    } else {
+        if (few) launch<&k_front6<float, false, DEM_LANES_FEW>, FS_THREADS, 1>(g, bs, s, r, mass, f);
+        else launch<&k_front6<float, false, DEM_LANES_MANY>, FS_THREADS, 1>(g, bs, s, r, mass, f);
+    }
+}
+
+}  // namespace lbdem

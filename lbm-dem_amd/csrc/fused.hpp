@@ -23,11 +23,11 @@ struct FusedArgs {
     const ObjLB* olb;
     double* hacc;
     double* blockPart;
-    int32_t* blockFlag;
     const uint64_t* bcm;
     DevScalars* sc;
     int nseg, nby, nbz;  // 64-node segments per row (tiles per row with 2-byte storage), row groups, z-slabs
     int gridBlocks;  // the box's grid (a batch launch covers the largest box; the rest return)
+    int partStride;  // of the columns of blockPart (the largest grid of the box, whatever the walk)
     int storeVel;    // every active node's density and velocity into aux (else interface nodes only)
     Consts k;
 };
@@ -549,10 +549,23 @@ __device__ inline void k_fused(FusedArgs<S> a) {
             }
         }
     }
-    // object / wall partials: written only by blocks that have any, flagged for the reduction
-    const int any = __syncthreads_or(tid < PART_STRIDE && sPart[tid] != 0.0);
-    if (any && tid < PART_STRIDE) a.blockPart[int64_t(tid) * a.gridBlocks + b0] = sPart[tid];
-    if (tid == 0) a.blockFlag[b0] = any;
+    // object / wall partials: a block that has any appends them, column by column, to the records
+    // the finalisation sums (the sums above are complete since the block's synchronisation before
+    // flush_particles; one wavefront holds them all). The impactor's records, a few hundred, have a
+    // list of their own: the free surface needs their extra mass first.
+    static_assert(PART_STRIDE <= FX, "one wavefront appends the block's partials");
+    if (threadIdx.y == 0) {
+        const bool used = tid < PART_STRIDE && sPart[tid] != 0.0;
+        const uint32_t m = uint32_t(__ballot(used));
+        constexpr uint32_t objBits = (1u << PART_WALL) - 1u;
+        int pos = 0;
+        if (tid == 0 && (m & objBits)) pos = atomicAdd(&a.sc->nPartObj, 1);
+        if (tid == PART_WALL && (m & ~objBits)) pos = atomicAdd(&a.sc->nPartWall, 1);
+        const int po = __shfl(pos, 0, 64), pw = __shfl(pos, PART_WALL, 64);
+        if ((m & objBits) && tid < PART_WALL) a.blockPart[int64_t(tid) * a.partStride + po] = sPart[tid];
+        if ((m & ~objBits) && tid >= PART_WALL && tid < PART_STRIDE)
+            a.blockPart[int64_t(tid) * a.partStride + pw] = sPart[tid];
+    }
 }
 
 // Slip walls (LB.cpp:1454-1482, slip static walls): a diagonal link j (j > 6) of an active node A
@@ -618,12 +631,13 @@ void launch_fused(Box& b, const Consts& k, const PartLB* plb, const ObjLB* olb, 
     a.mass = (typename Types<S>::M*)b.mass; a.aux = (typename Types<S>::C*)b.aux;
     a.visc = (typename Types<S>::C*)b.visc;
     a.ifList = b.ifList; a.ifCap = b.ifCap;
-    a.plb = plb; a.olb = olb; a.hacc = b.hacc; a.blockPart = b.blockPart; a.blockFlag = b.blockFlag; a.bcm = b.bcm; a.sc = sc;
+    a.plb = plb; a.olb = olb; a.hacc = b.hacc; a.blockPart = b.blockPart; a.bcm = b.bcm; a.sc = sc;
     a.k = k;
     const int fz = b.fz;
     a.nseg = (b.g.X + FX - 1) / FX; a.nby = (b.g.Y + FY - 1) / FY; a.nbz = (b.g.Z + fz - 1) / fz;
     const int grid = fused_grid_blocks(b.g, fz, b.prec);
     a.gridBlocks = grid;
+    a.partStride = b.blockPartCap / PART_STRIDE;
     a.storeVel = storeVel ? 1 : 0;
     const bool fs = k.freeSurface != 0;
     if (ev0) (void)hipEventRecord(ev0, s);

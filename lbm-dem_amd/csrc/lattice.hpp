@@ -104,6 +104,84 @@ constexpr int MAX_OBJ_PART = 2;
 // bounce-back mass term of all object links at 6, wall w's force at 7 MAX_OBJ_PART + 3 w
 constexpr int PART_BB = 6, PART_WALL = 7 * MAX_OBJ_PART;
 
+// Position in a list for each lane of the wavefront that calls this now (any subset of its
+// lanes, in divergent code too): one atomic reservation per wavefront, lanes in lane order.
+__device__ inline int wave_reserve(int* count) {
+    const unsigned long long m = __ballot(1);
+    const int lane = __lane_id();
+    const int leader = __ffsll(m) - 1;
+    int base = 0;
+    if (lane == leader) base = atomicAdd(count, __popcll(m));
+    base = __shfl(base, leader, 64);
+    return base + __popcll(m & ((1ull << lane) - 1ull));
+}
+
+// a node changed between active and non-active (or among non-active types): its neighbourhood is
+// re-marked before the next LB step; an overflowing list asks for a full re-mark instead
+__device__ inline void push_changed(int32_t* changed, int cap, DevScalars* sc, int32_t i) {
+    const int pos = wave_reserve(&sc->nChanged);
+    if (pos < cap) changed[pos] = i;
+    else atomicOr(&sc->fullMark, 1);
+}
+
+__device__ inline void list_push(int32_t* list, int* count, int cap, int32_t v, int* overflow) {
+    const int pos = wave_reserve(count);
+    if (pos < cap) list[pos] = v;
+    else atomicOr(overflow, 1);
+}
+
+// Block-wide forms of the two above for the passes over the whole interface list, where one
+// atomic per wavefront on one counter serialises (every thread of the block must call them, the
+// same number of times; sTmp: blockDim.x / 64 + 1 ints or doubles of LDS, reused by the next call):
+// positions in a list for the threads with `want`, one reservation per block, block-major then
+// wave then lane order; and a sum into one global total, one atomic per block.
+__device__ inline int block_reserve(int* count, bool want, int* sTmp) {
+    const unsigned long long m = __ballot(want);
+    const int lane = __lane_id(), wave = threadIdx.x / 64, nw = blockDim.x / 64;
+    if (lane == 0) sTmp[wave] = __popcll(m);
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        int acc = 0;
+        for (int w = 0; w < nw; ++w) {
+            const int c = sTmp[w];
+            sTmp[w] = acc;
+            acc += c;
+        }
+        sTmp[nw] = acc ? atomicAdd(count, acc) : 0;
+    }
+    __syncthreads();
+    const int r = sTmp[nw] + sTmp[wave] + __popcll(m & ((1ull << lane) - 1ull));
+    __syncthreads();
+    return r;
+}
+template <typename T>
+__device__ inline void block_add(T* dst, T v, T* sTmp) {
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+    const int wave = threadIdx.x / 64, nw = blockDim.x / 64;
+    if (__lane_id() == 0) sTmp[wave] = v;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        T t = 0;
+        for (int w = 0; w < nw; ++w) t += sTmp[w];
+        if (t != T(0)) atomicAdd(dst, t);
+    }
+    __syncthreads();
+}
+
+// per-thread partial sums into one global total: summed over the wavefront first (every lane of
+// the wavefront must call this), one atomic per wavefront that has a nonzero sum
+__device__ inline void wave_add(double* dst, double v) {
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+    if (__lane_id() == 0 && v != 0.0) atomicAdd(dst, v);
+}
+__device__ inline void wave_add(int* dst, int v) {
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+    if (__lane_id() == 0 && v != 0) atomicAdd(dst, v);
+}
+
 // check nodes and source directions of the slip reflection (LB.cpp:1454-1482; see k_slip)
 __host__ __device__ constexpr int slip1Check(int j) {
     constexpr int c[Q] = {0, 0, 0, 0, 0, 0, 0, 1, 2, 3, 4, 3, 4, 5, 6, 1, 2, 6, 5};

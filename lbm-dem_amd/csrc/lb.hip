@@ -4,7 +4,9 @@
 //   * free-surface mass exchange and interface conversion (LB.cpp:1548-1852)
 //   * particle flags and the moving-object (impactor) node update (LB.cpp:683-711, 797-943,
 //     1875-1899, 1980-2029; findNewSolid, LB.cpp:2032-2100, changes no flag)
-#include "lattice.hpp"
+#include "front.hpp"
+
+#include <utility>
 
 namespace lbdem {
 
@@ -192,10 +194,19 @@ __device__ inline uint64_t link_classes(const Geom& g, const uint8_t* type, cons
     const Offs o(g, x, y, z);
     uint64_t m = 0;
     int wprim = -1;
+    // every neighbour's type and solid index loaded up front, so that the loads overlap: an index
+    // loaded only for impactor neighbours is one dependent load after the other (k_mark 8.2 us on a
+    // 64^3 box, 15 us on 256x320x256, most of it that)
+    uint8_t tfs[Q];
+    int32_t sis[Q];
 #pragma unroll
     for (int j = 1; j < Q; ++j) {
-        const int32_t nb = i + o.d(j);
-        const uint8_t tf = type[nb];
+        tfs[j] = type[i + o.d(j)];
+        sis[j] = solid[i + o.d(j)];
+    }
+#pragma unroll
+    for (int j = 1; j < Q; ++j) {
+        const uint8_t tf = tfs[j];
         const uint8_t ty = tf & T_BASE;
         uint64_t cls = BC_OTHER;
         if (ty == T_FLUID || ty == T_IF) {
@@ -207,7 +218,7 @@ __device__ inline uint64_t link_classes(const Geom& g, const uint8_t* type, cons
             if (wprim < 0) wprim = w;
             cls = w == wprim ? BC_WALL : BC_OTHER;
         } else if (ty == T_OBJ) {
-            const int32_t si = solid[nb];
+            const int32_t si = sis[j];
             cls = si == 0 ? BC_OBJ0 : (si == 1 ? BC_OBJ1 : BC_OTHER);
         }
         m |= cls << (BC_BITS * (j - 1));
@@ -237,7 +248,7 @@ __device__ inline uint32_t inactive_bytes(uint32_t w) {
     m |= m >> 14;
     return m & 0xFu;
 }
-constexpr int MARK_GRID = 1024;  // blocks of k_mark (grid-stride; the full pass is rare)
+constexpr int MARK_GRID = 512;  // blocks of k_mark (grid-stride; the full pass is rare)
 __device__ __attribute__((always_inline)) inline void mark_full_w(Geom g, uint8_t* type, const int32_t* solid, uint64_t* bcm) {
     const int W = g.X / 4;
     const uint32_t* t32 = reinterpret_cast<const uint32_t*>(type);
@@ -307,12 +318,28 @@ __device__ inline void mark_full_b(Geom g, uint8_t* type, const int32_t* solid, 
     for (int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; i < g.N; i += int64_t(gridDim.x) * blockDim.x)
         mark_node(g, type, solid, bcm, int32_t(i));
 }
+// end of the coupling step's flag pass (flags_compute set kminP to INT_MAX): taken by the marking, or
+// by a launch of its own after a coupling step without an LB step
+__device__ inline void couple_end(DevScalars* sc) {
+    if (!sc->newNeighborList) return;
+    if (sc->kminP == INT_MAX) sc->kminP = -1;
+    sc->newNeighborList = 0;
+}
+__device__ inline void k_couple_end(DevScalars* sc) { couple_end(sc); }
+
 // One launch: the full pass when the full-pass flag is set (initialisation, a flag rebuild that
 // clears wall indices, change-list overflow), else the incremental pass: the stencil
 // neighbourhood (wrapped) of every node on the change list. A node reached from several changed
 // nodes is marked several times with the same result.
 __device__ inline void k_mark(Geom g, uint8_t* type, const int32_t* solid, uint64_t* bcm, const int32_t* changed, int cap,
-                              const DevScalars* sc) {
+                              DevScalars* sc) {
+    // the coupling before this launch is complete and the fused kernel comes next: its counters start
+    // at zero, and the flag pass of a list rebuild has been taken
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        couple_end(sc);
+        sc->nIf = 0;
+        sc->nPartObj = sc->nPartWall = 0;
+    }
     if (sc->fullMark) {
         if (g.X % 4 == 0) mark_full_w(g, type, solid, bcm);
         else mark_full_b(g, type, solid, bcm);
@@ -333,7 +360,7 @@ __device__ inline void k_mark(Geom g, uint8_t* type, const int32_t* solid, uint6
 
 void lb_mark_edges(const Box& b, DevScalars* sc, hipStream_t s) {
     launch_gs<&k_mark, 256, 1>(MARK_GRID, 256, s, b.g, b.type, b.solid, b.bcm, b.changed, b.changedCap, sc);
-    // the list and the full-pass flag are reset by the next kernel (k_begin_lb)
+    // the list and the full-pass flag are reset by the finalisation of the fused kernel's sums
 }
 
 int fused_grid_blocks(const Geom& g, int fz, int prec) {
@@ -342,510 +369,68 @@ int fused_grid_blocks(const Geom& g, int fz, int prec) {
     return ((nseg * nby * nbz + 7) / 8) * 8;                              // XCD-spread tiles
 }
 
-// end of findNewActive's scan (LB.cpp:1980-2029): the lowest node still inside its particle
-// becomes the next step's starting point (-1: none)
-__device__ inline void fna_finish(DevScalars* sc) {
-    if (!sc->needScan) return;
-    sc->kminP = sc->kstar == INT_MAX ? -1 : sc->kstar;
-    sc->needScan = 0;
-}
-
-// after the edge marking, before the fused kernel: the findNewActive scan's result is taken, the
-// change list is consumed, the interface list starts empty (the particle sums were zeroed by the previous step's k_hydro_finalize, or
-// at initialisation)
-__device__ inline void k_begin_lb(DevScalars* sc) {
-    fna_finish(sc);
-    sc->fullMark = 0;
-    sc->nChanged = 0;
-    sc->nIf = 0;
-}
-
 void lb_fused_step(Box& b, const Consts& k, const PartLB* plb, const ObjLB* olb, DevScalars* sc, bool diag,
                    bool storeVel, hipStream_t s, hipEvent_t ev0, hipEvent_t ev1) {
-    launch<&k_begin_lb, 1024, 1>(1, 1, s, sc);
     if (b.prec == LBDEM_PREC_FP64) launch_fused<double>(b, k, plb, olb, sc, diag, storeVel, s, ev0, ev1);
     else if (b.prec == LBDEM_PREC_FP32) launch_fused<float>(b, k, plb, olb, sc, diag, storeVel, s, ev0, ev1);
     else launch_fused<__half>(b, k, plb, olb, sc, diag, storeVel, s, ev0, ev1);
 }
 
-// deterministic sum of the flagged per-block partials, unit conversion of all hydrodynamic results
-// (LB.cpp:1966-1977, 1536-1543)
-constexpr int HF_THREADS = 1024;
-__device__ inline void k_hydro_finalize(int nblk, const double* part, const int32_t* flag, Consts k, double* hacc, double* FHydro,
-                                 double* MHydro, double* fluidVol, DevScalars* sc, double* objFH, double* objMH,
-                                 double* wallFH, int diag, int* count2) {
+__device__ inline void k_hydro_finalize(HydroArgs a, Consts k, DevScalars* sc) {
     __shared__ double red[HF_THREADS / 64];
-    const int tid = threadIdx.x;
-    if (blockIdx.x == 0 && tid == 0) {  // counters of the free-surface pass that follows (LB.cpp:422-430)
-        sc->surplus = 0.0;
-        sc->nFilled = sc->nEmptied = sc->nNewIf = 0;
-        sc->nIfFinal = 0;
-        *count2 = 0;
-    }
-    if (blockIdx.x < PART_STRIDE) {
-        // column c of the partial table (one block per column), summed in a fixed order: strided
-        // per-thread sums, a wavefront butterfly, then the waves in order
-        const int c = blockIdx.x;
-        if (c >= 7 * MAX_OBJ_PART && !diag) return;
-        if (c < 7 * MAX_OBJ_PART && c / 7 >= k.nObj && c != 6) return;            // no such object
-        if (c >= 7 * MAX_OBJ_PART && (c - 7 * MAX_OBJ_PART) / 3 >= k.nWall) return;  // no such wall
-        // four flag loads (and then four value loads) in flight per thread; the additions keep the
-        // order of one strided pass (a skipped block adds +0.0, which leaves the sum unchanged)
-        double acc = 0.0;
-        const int bs = int(blockDim.x);
-        const double* col = part + int64_t(c) * nblk;
-        int b = tid;
-        for (; b + 3 * bs < nblk; b += 4 * bs) {
-            const int32_t f0 = flag[b], f1 = flag[b + bs], f2 = flag[b + 2 * bs], f3 = flag[b + 3 * bs];
-            const double v0 = f0 ? col[b] : 0.0, v1 = f1 ? col[b + bs] : 0.0;
-            const double v2 = f2 ? col[b + 2 * bs] : 0.0, v3 = f3 ? col[b + 3 * bs] : 0.0;
-            acc += v0; acc += v1; acc += v2; acc += v3;
-        }
-        for (; b < nblk; b += bs)
-            if (flag[b]) acc += col[b];
-#pragma unroll
-        for (int off = 32; off > 0; off >>= 1) acc += __shfl_xor(acc, off, 64);
-        if ((tid & 63) == 0) red[tid / 64] = acc;
-        __syncthreads();
-        if (tid == 0) {
-            double v = 0.0;
-            for (int w = 0; w < HF_THREADS / 64; ++w) v += red[w];
-            if (c < 7 * MAX_OBJ_PART) {
-                const int o = c / 7, comp = c % 7;
-                if (o < k.nObj) {
-                    if (comp < 3) objFH[3 * o + comp] = v * k.unitForce;
-                    else if (comp < 6) objMH[3 * o + comp - 3] = v * k.unitTorque;
-                }
-                if (c == 6) { sc->extraMass = v; sc->lastExtraMass = v; }
-            } else {
-                const int w = (c - 7 * MAX_OBJ_PART) / 3, comp = (c - 7 * MAX_OBJ_PART) % 3;
-                if (w < k.nWall) wallFH[3 * w + comp] = v * k.unitForce;
-            }
-        }
-    } else {
-        const int p = (blockIdx.x - PART_STRIDE) * blockDim.x + tid;
-        if (p < k.nPart) {
-            double* h = hacc + int64_t(p) * 8;
-            for (int c = 0; c < 3; ++c) {
-                FHydro[3 * p + c] = h[c] * k.unitForce;
-                MHydro[3 * p + c] = h[3 + c] * k.unitTorque;
-            }
-            fluidVol[p] = h[6] * k.unitVolume;
-            for (int c = 0; c < 8; ++c) h[c] = 0.0;  // zero for the next LB step's sums
-        }
-    }
+    if (int(blockIdx.x) < a.blocks) hydro_finalize(a, k, sc, int(blockIdx.x), red);
+}
+static HydroArgs hydro_args(const Box& b, const Consts& k, double* FHydro, double* MHydro, double* fluidVol, double* objFH,
+                            double* objMH, double* wallFH, bool diag) {
+    HydroArgs a;
+    a.part = b.blockPart; a.stride = b.blockPartCap / PART_STRIDE; a.hacc = b.hacc;
+    a.FHydro = FHydro; a.MHydro = MHydro; a.fluidVol = fluidVol; a.objFH = objFH; a.objMH = objMH; a.wallFH = wallFH;
+    a.diag = diag ? 1 : 0;
+    a.blocks = PART_STRIDE + (k.nPart + HF_THREADS - 1) / HF_THREADS;
+    return a;
 }
 
 void lb_hydro_finalize(const Box& b, const Consts& k, double* FHydro, double* MHydro, double* fluidVol,
                        DevScalars* sc, double* objFH, double* objMH, double* wallFH, bool diag, hipStream_t s) {
-    const int nblk = fused_grid_blocks(b.g, b.fz, b.prec);
-    const int grid = PART_STRIDE + (k.nPart + HF_THREADS - 1) / HF_THREADS;
-    int* count2 = (int*)(b.ifList2 + b.ifCap);  // free-surface counter stored after the list
-    launch<&k_hydro_finalize, HF_THREADS, 1>(grid, HF_THREADS, s, nblk, b.blockPart, b.blockFlag, k, b.hacc, FHydro, MHydro, fluidVol, sc, objFH, objMH, wallFH, diag ? 1 : 0, count2);
+    const HydroArgs a = hydro_args(b, k, FHydro, MHydro, fluidVol, objFH, objMH, wallFH, diag);
+    launch<&k_hydro_finalize, HF_THREADS, 1>(a.blocks, HF_THREADS, s, a, k, sc);
 }
 
-// ------------------------------------------------------------------------------------------
-// free surface (LB.cpp:1548-1852)
-// ------------------------------------------------------------------------------------------
-constexpr int LIST_GRID = 256;  // blocks of the free-surface list passes (few items: launch ramp dominates)
-
-template <typename S, int L>
-__device__ inline void k_fs_mass(Geom g, const S* f, const uint8_t* type, const typename Types<S>::M* mass,
-                          const typename Types<S>::C* aux, const int32_t* ifList, typename Types<S>::M* newMass,
-                          DevScalars* sc, int32_t* filledFlag, int slipDyn, double s1) {
-    using C = typename Types<S>::C;
-    using M = typename Types<S>::M;
-    const int nIf = sc->nIf;
-    const double addE = sc->extraMass / double(nIf);
-    for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < nIf; k += gridDim.x * blockDim.x) {
-        const int64_t i = ifList[k];
-        int x, y, z;
-        cell_xyz(g, i, x, y, z);
-        const Offs o(g, x, y, z);
-        const C mi = C(double(mass[i]) + addE);
-        // every neighbour's type, populations and mass are loaded up front (all addresses are
-        // nodes of the box), so the loads overlap; the sum then runs in direction order
-        uint8_t ty[Q];
-        C a1[Q], a2[Q], mj[Q];
-#pragma unroll
-        for (int j = 1; j < Q; ++j) {
-            const int64_t yj = i + o.d(j);
-            ty[j] = type[yj] & T_BASE;
-            a1[j] = StoreT<S>::ld(f + int64_t(j) * g.N + yj);
-            a2[j] = StoreT<S>::ld(f + int64_t(oppq(j)) * g.N + i);
-            mj[j] = C(mass[yj]);
-        }
-        C dm = 0;
-#pragma unroll
-        for (int j = 1; j < Q; ++j) {
-            const bool slipLink = slipDyn && ty[j] == T_WALL;
-            if (ty[j] != T_IF && ty[j] != T_FLUID && ty[j] != T_OBJ && !slipLink) continue;
-            const C ms = L == 1 ? (a1[j] - a2[j]) : (a2[j] - a1[j]);  // incoming(opp j) - outgoing(j), offsets
-            if (ty[j] == T_IF) dm += C(0.5) * (C(double(mj[j]) + addE) + mi) * ms;
-            else if (ty[j] == T_FLUID) dm += ms;
-            else if (slipLink) {  // moving slip wall (LB.cpp:1595-1625): (1 - S) of the mass on a slip link
-                bool slipped = false;
-                if (j > 6) {
-                    const uint8_t t1 = ty[slip1Check(j)], t2 = ty[slip2Check(j)];
-                    slipped = (t1 == T_FLUID || t1 == T_IF) != (t2 == T_FLUID || t2 == T_IF);
-                }
-                dm += (slipped ? C(1.0 - s1) * mi : mi) * ms;
-            } else {
-                dm += mi * ms;
-            }
-        }
-        newMass[k] = M(mi + dm);
-    }
+// blocks of the free surface's passes over the interface list, which holds about one node per column
+// of the box (the passes stride over longer lists)
+static int fs_blocks(const Geom& g) {
+    const int64_t n = (int64_t(g.X) * g.Z * 5 / 4 + FS_THREADS - 1) / FS_THREADS;
+    return int(n < 8 ? 8 : (n > 256 ? 256 : n));
 }
-
-// Position in a list for each lane of the wavefront that calls this now (any subset of its
-// lanes, in divergent code too): one atomic reservation per wavefront, lanes in lane order.
-__device__ inline int wave_reserve(int* count) {
-    const unsigned long long m = __ballot(1);
-    const int lane = __lane_id();
-    const int leader = __ffsll(m) - 1;
-    int base = 0;
-    if (lane == leader) base = atomicAdd(count, __popcll(m));
-    base = __shfl(base, leader, 64);
-    return base + __popcll(m & ((1ull << lane) - 1ull));
-}
-
-// a node changed between active and non-active (or among non-active types): its neighbourhood is
-// re-marked before the next LB step; an overflowing list asks for a full re-mark instead
-__device__ inline void push_changed(int32_t* changed, int cap, DevScalars* sc, int32_t i) {
-    const int pos = wave_reserve(&sc->nChanged);
-    if (pos < cap) changed[pos] = i;
-    else atomicOr(&sc->fullMark, 1);
-}
-
-__device__ inline void list_push(int32_t* list, int* count, int cap, int32_t v, int* overflow) {
-    const int pos = wave_reserve(count);
-    if (pos < cap) list[pos] = v;
-    else atomicOr(overflow, 1);
-}
-
-// Block-wide forms of the two above for the passes over the whole interface list, where one
-// atomic per wavefront on one counter serialises (every thread of the block must call them, the
-// same number of times; sTmp: blockDim.x / 64 + 1 ints or doubles of LDS, reused by the next call):
-// positions in a list for the threads with `want`, one reservation per block, block-major then
-// wave then lane order; and a sum into one global total, one atomic per block.
-__device__ inline int block_reserve(int* count, bool want, int* sTmp) {
-    const unsigned long long m = __ballot(want);
-    const int lane = __lane_id(), wave = threadIdx.x / 64, nw = blockDim.x / 64;
-    if (lane == 0) sTmp[wave] = __popcll(m);
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        int acc = 0;
-        for (int w = 0; w < nw; ++w) {
-            const int c = sTmp[w];
-            sTmp[w] = acc;
-            acc += c;
-        }
-        sTmp[nw] = acc ? atomicAdd(count, acc) : 0;
-    }
-    __syncthreads();
-    const int r = sTmp[nw] + sTmp[wave] + __popcll(m & ((1ull << lane) - 1ull));
-    __syncthreads();
-    return r;
-}
-template <typename T>
-__device__ inline void block_add(T* dst, T v, T* sTmp) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-    const int wave = threadIdx.x / 64, nw = blockDim.x / 64;
-    if (__lane_id() == 0) sTmp[wave] = v;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        T t = 0;
-        for (int w = 0; w < nw; ++w) t += sTmp[w];
-        if (t != T(0)) atomicAdd(dst, t);
-    }
-    __syncthreads();
-}
-
-// per-thread partial sums into one global total: summed over the wavefront first (every lane of
-// the wavefront must call this), one atomic per wavefront that has a nonzero sum
-__device__ inline void wave_add(double* dst, double v) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-    if (__lane_id() == 0 && v != 0.0) atomicAdd(dst, v);
-}
-__device__ inline void wave_add(int* dst, int v) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-    if (__lane_id() == 0 && v != 0) atomicAdd(dst, v);
-}
-
-// assign new mass, classify filled / emptied (findInterfaceMutants, LB.cpp:1669-1698)
 template <typename S>
-__device__ inline void k_fs_mutants(uint8_t* type, typename Types<S>::M* mass, const typename Types<S>::C* aux, int64_t N,
-                             const int32_t* ifList, const typename Types<S>::M* newMass, int32_t* filled,
-                             int32_t* emptied, int cap, DevScalars* sc, int32_t* marker, int32_t* changed,
-                             int changedCap) {
-    const int nIf = sc->nIf;
-    for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < nIf; k += gridDim.x * blockDim.x) {
-        const int64_t i = ifList[k];
-        const auto m = newMass[k];
-        mass[i] = m;
-        const auto n = aux[i];
-        if (m > n) {
-            type[i] = (type[i] & (T_PMASK | T_EDGE)) | T_FLUID;  // active to active: edge bit stays
-            marker[i] = -3;
-            list_push(filled, &sc->nFilled, cap, int32_t(i), &sc->listOverflow);
-        } else if (m < 0) {
-            type[i] = (type[i] & T_PMASK) | T_GAS;
-            list_push(emptied, &sc->nEmptied, cap, int32_t(i), &sc->listOverflow);
-            push_changed(changed, changedCap, sc, int32_t(i));
-        }
+static void front(Box& b, const Consts& k, DevScalars* sc, const HydroArgs& h, bool fs, const NbrArgs& n,
+                  const ForceArgs& f, hipStream_t s) {
+    FsArgs<S> a;
+    a.g = b.g; a.f = (S*)b.f; a.type = b.type;
+    a.mass = (typename Types<S>::M*)b.mass; a.aux = (typename Types<S>::C*)b.aux; a.visc = (typename Types<S>::C*)b.visc;
+    a.ifList = b.ifList; a.newMass = (typename Types<S>::M*)b.ifNewMass; a.list2 = b.ifList2;
+    a.filled = b.filled; a.emptied = b.emptied; a.newIf = b.newIf; a.marker = b.donor; a.changed = b.changed;
+    a.count2 = (int*)(b.ifList2 + b.ifCap);  // counter stored after the list
+    a.sc = sc; a.cap = b.ifCap; a.changedCap = b.changedCap;
+    a.slipDyn = k.slip == 2 ? 1 : 0; a.s1 = k.slipCoef;
+    a.blocks = fs ? fs_blocks(b.g) : 0;
+    launch_front<S>(a, h, k, n, f, b.parity, s);
+}
+void lb_front(Box& b, const Consts& k, DevScalars* sc, bool hydro, bool fs, double* FHydro, double* MHydro,
+              double* fluidVol, double* objFH, double* objMH, double* wallFH, const DemParams* dp, DemState* ds,
+              int demTimeStep, bool forceList, hipStream_t s) {
+    HydroArgs h = hydro_args(b, k, FHydro, MHydro, fluidVol, objFH, objMH, wallFH, true);
+    if (!hydro) h.blocks = 0;
+    NbrArgs n{};
+    ForceArgs f{};
+    if (ds && (dp->nPart > 0 || forceList)) {
+        n = nbr_args(*dp, *ds, sc, forceList);
+        if (!forceList) f = force_args(*dp, *ds, demTimeStep);
     }
-}
-
-// gas neighbours of filled nodes: donor = highest-index filled neighbour (LB.cpp:1704-1728)
-__device__ inline void k_fs_donors(Geom g, const uint8_t* type, const int32_t* filled, int32_t* donor, int32_t* newIf,
-                            int cap, DevScalars* sc) {
-    const int nF = sc->nFilled;
-    for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < nF; k += gridDim.x * blockDim.x) {
-        const int64_t i = filled[k];
-        int x, y, z;
-        cell_xyz(g, i, x, y, z);
-        const Offs o(g, x, y, z);
-        uint32_t gasMask = 0;  // neighbour types loaded up front so the loads overlap
-#pragma unroll
-        for (int j = 1; j < Q; ++j) gasMask |= uint32_t((type[i + o.d(j)] & T_BASE) == T_GAS) << j;
-        for (uint32_t m = gasMask; m; m &= m - 1u) {  // gas neighbours in direction order
-            const int j = __ffs(m) - 1;
-            const int64_t yj = i + o.d(j);
-            const int old = atomicMax(&donor[yj], int32_t(i));
-            if (old < 0) list_push(newIf, &sc->nNewIf, cap, int32_t(yj), &sc->listOverflow);
-        }
-    }
-}
-
-// initialise the new interface nodes from their donor (node::initialize with the donor's
-// u, visc and hydroForce+lbF, mass 0.01*rho0)
-template <typename S, int L>
-__device__ inline void k_fs_new_from_donor(Geom g, S* f, uint8_t* type, typename Types<S>::M* mass,
-                                    typename Types<S>::C* aux, typename Types<S>::C* visc, const int32_t* newIf,
-                                    const int32_t* donor, DevScalars* sc, Consts k, int32_t* changed, int changedCap) {
-    using C = typename Types<S>::C;
-    const int nN = sc->nNewIf;
-    for (int kk = blockIdx.x * blockDim.x + threadIdx.x; kk < nN; kk += gridDim.x * blockDim.x) {
-        const int64_t gi = newIf[kk];
-        const int64_t d = donor[gi];
-        const int64_t N = g.N;
-        type[gi] = (type[gi] & T_PMASK) | T_IF;
-        push_changed(changed, changedCap, sc, int32_t(gi));
-        const double n = k.rho0;
-        const double ux = (double(aux[4 * N + d]) + k.lbF[0]) / 2.0 / n + double(aux[N + d]);
-        const double uy = (double(aux[5 * N + d]) + k.lbF[1]) / 2.0 / n + double(aux[2 * N + d]);
-        const double uz = (double(aux[6 * N + d]) + k.lbF[2]) / 2.0 / n + double(aux[3 * N + d]);
-        int x, y, z;
-        cell_xyz(g, gi, x, y, z);
-        const Offs o(g, x, y, z);
-        const double usq = ux * ux + uy * uy + uz * uz;
-        for (int q = 0; q < Q; ++q) {
-            const double vu = ux * cxq(q) + uy * cyq(q) + uz * czq(q);
-            const double feq = wq(q) * n * (1.0 + 3.0 * vu + 4.5 * vu * vu - 1.5 * usq);
-            StoreT<S>::st(f + load_slot(g, gi, o, q, L), C(feq - wq(q)));
-        }
-        mass[gi] = typename Types<S>::M(0.01 * k.rho0);
-        aux[gi] = C(n);
-        aux[N + gi] = C(ux); aux[2 * N + gi] = C(uy); aux[3 * N + gi] = C(uz);
-        aux[4 * N + gi] = C(0); aux[5 * N + gi] = C(0); aux[6 * N + gi] = C(0);
-        if (visc) visc[gi] = visc[d];  // the donor's viscosity (LB.cpp:1719)
-    }
-    if (blockIdx.x == 0 && threadIdx.x == 0) atomicAdd(&sc->surplus, -0.01 * k.rho0 * double(nN));
-}
-
-// fluid neighbours of emptied nodes become interface with 99% of their density (LB.cpp:1730-1748)
-template <typename S>
-__device__ inline void k_fs_from_emptied(Geom g, uint8_t* type, typename Types<S>::M* mass, typename Types<S>::C* aux,
-                                  const int32_t* emptied, int32_t* marker, int32_t* newIf, int cap, DevScalars* sc) {
-    using C = typename Types<S>::C;
-    using M = typename Types<S>::M;
-    const int nE = sc->nEmptied;
-    double gained = 0.0;
-    for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < nE; k += gridDim.x * blockDim.x) {
-        const int64_t i = emptied[k];
-        int x, y, z;
-        cell_xyz(g, i, x, y, z);
-        const Offs o(g, x, y, z);
-        // neighbour types loaded up front so the loads overlap; the marker CAS below decides which
-        // thread converts a node, so a type read early changes nothing
-        uint32_t fluidMask = 0;
-#pragma unroll
-        for (int j = 0; j < Q; ++j) fluidMask |= uint32_t((type[i + o.d(j)] & T_BASE) == T_FLUID) << j;
-        for (uint32_t m = fluidMask; m; m &= m - 1u) {  // fluid neighbours in direction order
-            const int j = __ffs(m) - 1;
-            const int64_t l = i + o.d(j);
-            double nl;
-            int old = atomicCAS(&marker[l], -1, -2);
-            if (old == -1) {
-                nl = double(mass[l]);               // ordinary fluid node: mass holds its density
-            } else if (old == -3 && atomicCAS(&marker[l], -3, -4) == -3) {
-                nl = double(aux[l]);                // filled this step: density kept in aux
-            } else {
-                continue;
-            }
-            type[l] = (type[l] & (T_PMASK | T_EDGE)) | T_IF;  // active to active: edge bit stays
-            mass[l] = M(0.99 * nl);
-            aux[l] = C(nl);
-            gained += 0.01 * nl;
-            list_push(newIf, &sc->nNewIf, cap, int32_t(l), &sc->listOverflow);
-        }
-    }
-    wave_add(&sc->surplus, gained);
-}
-
-// updateMutants (LB.cpp:1751-1790)
-template <typename S>
-__device__ inline void k_fs_update_mutants(uint8_t* type, typename Types<S>::M* mass, const typename Types<S>::C* aux,
-                                    const int32_t* filled, const int32_t* emptied, DevScalars* sc) {
-    const int nF = sc->nFilled, nE = sc->nEmptied;
-    double acc = 0.0;
-    for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < nF + nE; k += gridDim.x * blockDim.x) {
-        if (k < nF) {
-            const int64_t i = filled[k];
-            if ((type[i] & T_BASE) == T_FLUID) {
-                acc += double(mass[i]) - double(aux[i]);
-                mass[i] = typename Types<S>::M(aux[i]);
-            }
-        } else {
-            const int64_t i = emptied[k - nF];
-            if ((type[i] & T_BASE) == T_GAS) acc += double(mass[i]);
-        }
-    }
-    wave_add(&sc->surplus, acc);
-}
-
-// removeIsolated part 1: interface nodes without gas neighbours become fluid (LB.cpp:1796-1816).
-// The interface list after the conversions (the old interface nodes left untouched, then the new
-// ones) is visited here and compacted into list2 for the two passes that follow. A node's filter
-// depends only on its own type and marker, which no other thread changes in this pass, and a
-// conversion to fluid changes no node's gas test, so the pass equals the sequential loop.
-template <typename S>
-__device__ inline void k_fs_isolated_a(Geom g, uint8_t* type, typename Types<S>::M* mass, const typename Types<S>::C* aux,
-                                const int32_t* ifList, const int32_t* newIf, const int32_t* marker, int32_t* list2,
-                                int cap, int* count2, DevScalars* sc) {
-    const int nIf = sc->nIf, nN = sc->nNewIf;
-    __shared__ int sPos[8];
-    __shared__ double sSum[8];
-    double acc = 0.0;
-    // the loop runs the same number of times on every thread of a block (block_reserve)
-    for (int k0 = blockIdx.x * blockDim.x; k0 < nIf + nN; k0 += gridDim.x * blockDim.x) {
-        const int k = k0 + int(threadIdx.x);
-        int64_t i = -1;
-        if (k < nIf) {
-            i = ifList[k];
-            if ((type[i] & T_BASE) != T_IF || marker[i] != -1) i = -1;
-        } else if (k < nIf + nN) {
-            i = newIf[k - nIf];
-        }
-        bool gasNb = false;
-        if (i >= 0) {
-            int x, y, z;
-            cell_xyz(g, i, x, y, z);
-            const Offs o(g, x, y, z);
-#pragma unroll
-            for (int j = 1; j < Q; ++j) gasNb |= (type[i + o.d(j)] & T_BASE) == T_GAS;  // the 18 loads overlap
-        }
-        const int pos = block_reserve(count2, i >= 0, sPos);
-        if (i >= 0) {
-            if (pos < cap) list2[pos] = int32_t(i);
-            else atomicOr(&sc->listOverflow, 1);
-            if (!gasNb) {
-                acc += double(mass[i]) - double(aux[i]);
-                mass[i] = typename Types<S>::M(aux[i]);
-                type[i] = (type[i] & (T_PMASK | T_EDGE)) | T_FLUID;  // active to active: edge bit stays
-            }
-        }
-    }
-    block_add(&sc->surplus, acc, sSum);
-}
-
-// removeIsolated part 2: interface nodes without fluid neighbours become gas (LB.cpp:1821-1841)
-template <typename S>
-__device__ inline void k_fs_isolated_b(Geom g, uint8_t* type, const typename Types<S>::M* mass, const int32_t* list2,
-                                const int* count2, DevScalars* sc, int32_t* changed, int changedCap) {
-    const int n2 = *count2;
-    __shared__ double sSum[8];
-    __shared__ int sCnt[8];
-    double acc = 0.0;
-    int keep = 0;
-    for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < n2; k += gridDim.x * blockDim.x) {
-        const int64_t i = list2[k];
-        if ((type[i] & T_BASE) != T_IF) continue;
-        int x, y, z;
-        cell_xyz(g, i, x, y, z);
-        const Offs o(g, x, y, z);
-        bool fluidNb = false;  // the 18 type loads overlap (no early exit)
-#pragma unroll
-        for (int j = 1; j < Q; ++j) fluidNb |= (type[i + o.d(j)] & T_BASE) == T_FLUID;
-        if (!fluidNb) {
-            acc += double(mass[i]);
-            type[i] = (type[i] & T_PMASK) | T_GAS;
-            push_changed(changed, changedCap, sc, int32_t(i));
-        } else {
-            keep++;
-        }
-    }
-    block_add(&sc->surplus, acc, sSum);
-    block_add(&sc->nIfFinal, keep, sCnt);
-}
-
-// redistributeMass (LB.cpp:1844-1852) and marker reset
-template <typename S>
-__device__ inline void k_fs_redistribute(const uint8_t* type, typename Types<S>::M* mass, const int32_t* list2,
-                                  const int* count2, int32_t* marker, const int32_t* filled, const int32_t* newIf,
-                                  DevScalars* sc) {
-    const int n2 = *count2;
-    const double add = sc->surplus / double(sc->nIfFinal);
-    for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < n2; k += gridDim.x * blockDim.x) {
-        const int64_t i = list2[k];
-        if ((type[i] & T_BASE) == T_IF) mass[i] = typename Types<S>::M(double(mass[i]) + add);
-    }
-    const int nF = sc->nFilled, nN = sc->nNewIf;
-    for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < nF + nN; k += gridDim.x * blockDim.x)
-        marker[k < nF ? filled[k] : newIf[k - nF]] = -1;
-    if (blockIdx.x == 0 && threadIdx.x == 0) sc->lastSurplus = sc->surplus;
-}
-
-
-template <typename S>
-static void fs_impl(Box& b, const Consts& k, DevScalars* sc, hipStream_t s) {
-    using M = typename Types<S>::M;
-    using C = typename Types<S>::C;
-    S* f = (S*)b.f;
-    M* mass = (M*)b.mass;
-    C* aux = (C*)b.aux;
-    int* count2 = (int*)(b.ifList2 + b.ifCap);  // counter stored after the list
-    const int grid = LIST_GRID, bs = 256;
-    if (b.parity == 1)
-        launch_gs<&k_fs_mass<S, 1>, 256, 1>(grid, bs, s, b.g, f, b.type, mass, aux, b.ifList, (M*)b.ifNewMass, sc, b.donor,
-                                            k.slip == 2 ? 1 : 0, k.slipCoef);
-    else
-        launch_gs<&k_fs_mass<S, 0>, 256, 1>(grid, bs, s, b.g, f, b.type, mass, aux, b.ifList, (M*)b.ifNewMass, sc, b.donor,
-                                            k.slip == 2 ? 1 : 0, k.slipCoef);
-    launch_gs<&k_fs_mutants<S>, 256, 1>(grid, bs, s, b.type, mass, aux, b.g.N, b.ifList, (M*)b.ifNewMass, b.filled, b.emptied, b.ifCap, sc, b.donor, b.changed, b.changedCap);
-    launch_gs<&k_fs_donors, 256, 1>(grid, bs, s, b.g, b.type, b.filled, b.donor, b.newIf, b.ifCap, sc);
-    if (b.parity == 1)
-        launch_gs<&k_fs_new_from_donor<S, 1>, 256, 1>(grid, bs, s, b.g, f, b.type, mass, aux, (C*)b.visc, b.newIf, b.donor, sc, k,
-                                                      b.changed, b.changedCap);
-    else
-        launch_gs<&k_fs_new_from_donor<S, 0>, 256, 1>(grid, bs, s, b.g, f, b.type, mass, aux, (C*)b.visc, b.newIf, b.donor, sc, k,
-                                                      b.changed, b.changedCap);
-    launch_gs<&k_fs_from_emptied<S>, 256, 1>(grid, bs, s, b.g, b.type, mass, aux, b.emptied, b.donor, b.newIf, b.ifCap, sc);
-    launch_gs<&k_fs_update_mutants<S>, 256, 1>(grid, bs, s, b.type, mass, aux, b.filled, b.emptied, sc);
-    launch_gs<&k_fs_isolated_a<S>, 256, 1>(grid, bs, s, b.g, b.type, mass, aux, b.ifList, b.newIf, b.donor, b.ifList2,
-                                            b.ifCap, count2, sc);
-    launch_gs<&k_fs_isolated_b<S>, 256, 1>(grid, bs, s, b.g, b.type, mass, b.ifList2, count2, sc, b.changed, b.changedCap);
-    launch_gs<&k_fs_redistribute<S>, 256, 1>(grid, bs, s, b.type, mass, b.ifList2, count2, b.donor, b.filled, b.newIf, sc);
-}
-
-void lb_free_surface(Box& b, const Consts& k, DevScalars* sc, hipStream_t s) {
-    if (b.prec == LBDEM_PREC_FP64) fs_impl<double>(b, k, sc, s);
-    else if (b.prec == LBDEM_PREC_FP32) fs_impl<float>(b, k, sc, s);
-    else fs_impl<__half>(b, k, sc, s);
+    if (b.prec == LBDEM_PREC_FP64) front<double>(b, k, sc, h, fs, n, f, s);
+    else if (b.prec == LBDEM_PREC_FP32) front<float>(b, k, sc, h, fs, n, f, s);
+    else front<__half>(b, k, sc, h, fs, n, f, s);
+    if (f.blocks > 0) std::swap(ds->xiCur, ds->xiNext);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -864,28 +449,25 @@ void lb_free_surface(Box& b, const Consts& k, DevScalars* sc, hipStream_t s) {
 // b, b + 8, ... run on one XCD, whose L2 then holds one region). A wavefront walks its box 64 nodes
 // per lane step, FLAGS_UNROLL steps at a time so that their type loads are in flight together; the
 // sphere test keeps the reference's operations (LB.cpp:705, myvector.cpp:171-175).
-constexpr int FLAGS_GRID = 2048;   // blocks of the flag pass (grid-stride; most steps return early)
+constexpr int FLAGS_GRID = 2048, FLAGS_APPLY_GRID = 1024;  // blocks of the flag passes (grid-stride; most steps return early)
 constexpr int FLAGS_WAVES = 4;     // wavefronts (particles at a time) per block
 constexpr int FLAGS_UNROLL = 6;
-__device__ inline void k_flags_compute(Geom g, const uint8_t* type, const PartLB* plb, int nPart, int32_t* flagNew,
+__device__ inline void flags_compute(int blk, int nblk, Geom g, const uint8_t* type, const PartLB* plb, int nPart, int32_t* flagNew,
                                 DevScalars* sc, const int* nbrCount, const int* nbrList, int useList,
                                 const int* order) {
-    // a coupling step that follows a coupling step without an LB step between them (the DEM
-    // start-up repeat) finishes the previous findNewActive here (no other block touches kminP)
-    if (blockIdx.x == 0 && threadIdx.x == 0) fna_finish(sc);
     if (!sc->newNeighborList) return;
-    if (blockIdx.x == 0 && threadIdx.x == 0) sc->kminP = INT_MAX;  // lowest flagged index, from k_flags_apply
+    if (blk == 0 && threadIdx.x == 0) sc->kminP = INT_MAX;  // lowest flagged index, from flags_apply
     __shared__ double sq[FLAGS_WAVES][NBR_CAP][4];  // centre and radius of overlapping higher-index partners
     const int wv = __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> 6), lane = int(threadIdx.x) & 63;
     double(*hq)[4] = sq[wv];
     const int dims[3] = {g.X, g.Y, g.Z};
     // this wavefront's particles: positions k0, k0 + step, ... below k1 of the (sorted) order
-    int k0 = int(blockIdx.x) * FLAGS_WAVES + wv, k1 = nPart, step = int(gridDim.x) * FLAGS_WAVES;
-    if (gridDim.x % 8 == 0) {
-        const int share = (nPart + 7) / 8, xcd = int(blockIdx.x) % 8;
-        k0 = xcd * share + (int(blockIdx.x) / 8) * FLAGS_WAVES + wv;
+    int k0 = blk * FLAGS_WAVES + wv, k1 = nPart, step = nblk * FLAGS_WAVES;
+    if (nblk % 8 == 0) {
+        const int share = (nPart + 7) / 8, xcd = blk % 8;
+        k0 = xcd * share + (blk / 8) * FLAGS_WAVES + wv;
         k1 = min(nPart, (xcd + 1) * share);
-        step = int(gridDim.x / 8) * FLAGS_WAVES;
+        step = (nblk / 8) * FLAGS_WAVES;
     }
     for (int k = k0; k < k1; k += step) {
         const int p = order ? order[k] : k;
@@ -961,25 +543,16 @@ __device__ inline void k_flags_compute(Geom g, const uint8_t* type, const PartLB
     }
 }
 
-void lb_flags_rebuild_compute(const Box& b, const Consts& k, const PartLB* plb, DevScalars* sc, const int* nbrCount,
-                              const int* nbrList, bool useList, const int* order, hipStream_t s) {
-    // grid-stride over the particles: most steps only test the flag and return
-    if (k.nPart > 0)
-        launch_gs<&k_flags_compute, 64 * FLAGS_WAVES, 8, 16384>(
-            std::min((k.nPart + FLAGS_WAVES - 1) / FLAGS_WAVES, FLAGS_GRID), 64 * FLAGS_WAVES, s, b.g, b.type, plb,
-            k.nPart, b.flagNew, sc, nbrCount, nbrList, useList ? 1 : 0, order);
-}
-
 // clear every flag and solid index, apply the new flags (initializeParticleBoundaries)
-__device__ inline void k_flags_apply(int64_t N, uint8_t* type, int32_t* solid, int32_t* flagNew, DevScalars* sc,
-                                     int32_t* changed, int changedCap) {
+__device__ inline void flags_apply(int blk, int nblk, int64_t N, uint8_t* type, int32_t* solid, int32_t* flagNew,
+                                   DevScalars* sc, int32_t* changed, int changedCap) {
     if (!sc->newNeighborList) return;
     __shared__ int bmin;
     if (threadIdx.x == 0) bmin = INT_MAX;
     __syncthreads();
     int mymin = INT_MAX;
     bool remark = false;  // a cleared wall index: link classes need a full pass
-    for (int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; i < N; i += int64_t(gridDim.x) * blockDim.x) {
+    for (int64_t i = int64_t(blk) * 256 + threadIdx.x; i < N; i += int64_t(nblk) * 256) {
         const int32_t s = flagNew[i];
         const uint8_t t = type[i];
         // an object node's index is part of its neighbours' link classes: re-mark around it
@@ -1009,84 +582,75 @@ __device__ inline void k_flags_apply(int64_t N, uint8_t* type, int32_t* solid, i
         atomicMin(&sc->kminP, bmin);
 }
 
-
-void lb_flags_rebuild_apply(const Box& b, DevScalars* sc, hipStream_t s) {
-    const int64_t nb = (b.g.N + 255) / 256;
-    const int grid = int(nb < FLAGS_GRID ? nb : FLAGS_GRID);
-    launch_gs<&k_flags_apply, 1024, 1, 16384>(grid, 256, s, b.g.N, b.type, b.solid, b.flagNew, sc, b.changed,
-                                              b.changedCap);
-}
-
-__device__ inline void k_fna_check(Geom g, const int32_t* solid, const PartLB* plb, int nPart, DevScalars* sc) {
-    fna_finish(sc);  // a scan still pending (boxes without particles have no k_flags_compute)
-    if (sc->newNeighborList) {  // end of the flag pass (k_flags_compute set kminP to INT_MAX)
-        if (sc->kminP == INT_MAX) sc->kminP = -1;
-        sc->newNeighborList = 0;
-    }
+// findNewActive (LB.cpp:1980-2029), one block: when the lowest flagged node has left its particle, the
+// flagged nodes below the first one still inside its own lose their flag, and that one is the lowest
+// from then on. No node below the lowest is flagged, so the nodes are taken upwards from it, 16 384 at a
+// time, until a flagged one is inside: a few thousand nodes on, in the same sphere or the next
+// (a pass over the whole box and one over the nodes below its result were two launches and, on the
+// 256x320x256 box, 20 us when one was due). A step that rebuilt the flags has nothing to do: every
+// flag was set from this step's positions.
+constexpr int FNA_WORDS = 16;  // words of four type bytes per thread and round
+__device__ inline void find_new_active(const Geom& g, uint8_t* type, int32_t* solid, const PartLB* plb, int nPart,
+                                       DevScalars* sc) {
+    __shared__ int sMin;
+    if (sc->newNeighborList) return;
     const int kp = sc->kminP;
-    sc->needScan = 0;
     if (kp < 0) return;
-    int x, y, z;
-    cell_xyz(g, kp, x, y, z);
-    const int sp = solid[kp];
-    if (sp < 0 || sp >= nPart) { sc->needScan = 1; sc->kstar = INT_MAX; return; }
-    const PartLB P = plb[sp];
-    if (!inside_sphere(x, y, z, P.c[0], P.c[1], P.c[2], P.r)) { sc->needScan = 1; sc->kstar = INT_MAX; }
-}
-
-__device__ inline void k_fna_scan(Geom g, const uint8_t* type, const int32_t* solid, const PartLB* plb, int nPart,
-                           DevScalars* sc) {
-    if (!sc->needScan) return;
-    __shared__ int bmin;
-    if (threadIdx.x == 0) bmin = INT_MAX;
-    __syncthreads();
-    int mymin = INT_MAX;
-    for (int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; i < g.N; i += int64_t(gridDim.x) * blockDim.x) {
-        if (!(type[i] & T_PMASK)) continue;
+    auto inside = [&](int64_t i) {
         const int sp = solid[i];
-        if (sp < 0 || sp >= nPart) continue;
+        if (sp < 0 || sp >= nPart) return false;
         int x, y, z;
         cell_xyz(g, i, x, y, z);
         const PartLB P = plb[sp];
-        if (inside_sphere(x, y, z, P.c[0], P.c[1], P.c[2], P.r)) mymin = min(mymin, int(i));
+        return inside_sphere(x, y, z, P.c[0], P.c[1], P.c[2], P.r);
+    };
+    if (inside(kp)) return;
+    const uint32_t* t32 = reinterpret_cast<const uint32_t*>(type);
+    const int64_t nw = g.N / 4;  // whole words; the tail is taken byte by byte
+    int found = INT_MAX;
+    for (int64_t w0 = kp / 4; w0 <= nw; w0 += 256 * FNA_WORDS) {
+        if (threadIdx.x == 0) sMin = INT_MAX;
+        __syncthreads();
+        uint32_t t[FNA_WORDS];
+#pragma unroll
+        for (int u = 0; u < FNA_WORDS; ++u) {
+            const int64_t w = w0 + int64_t(u) * 256 + threadIdx.x;
+            t[u] = w < nw ? t32[w] : 0;
+            if (w == nw)
+                for (int64_t i = 4 * nw; i < g.N; ++i) t[u] |= uint32_t(type[i]) << (8 * int(i - 4 * nw));
+        }
+        int mymin = INT_MAX;
+        for (int u = 0; u < FNA_WORDS; ++u)
+            for (uint32_t m = t[u] & 0x80808080u; m && mymin == INT_MAX; m &= m - 1u) {
+                const int64_t i = 4 * (w0 + int64_t(u) * 256 + threadIdx.x) + (__ffs(m) - 1) / 8;
+                if (i >= kp && inside(i)) mymin = int(i);
+            }
+        if (mymin != INT_MAX) atomicMin(&sMin, mymin);
+        __syncthreads();
+        found = sMin;
+        __syncthreads();
+        for (int u = 0; u < FNA_WORDS; ++u)
+            for (uint32_t m = t[u] & 0x80808080u; m; m &= m - 1u) {
+                const int64_t i = 4 * (w0 + int64_t(u) * 256 + threadIdx.x) + (__ffs(m) - 1) / 8;
+                if (i < found) { type[i] &= uint8_t(~T_PMASK); solid[i] = 0; }
+            }
+        if (found != INT_MAX) break;
     }
-    if (mymin != INT_MAX) atomicMin(&bmin, mymin);
-    __syncthreads();
-    if (threadIdx.x == 0 && bmin != INT_MAX &&
-        bmin < __hip_atomic_load(&sc->kstar, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
-        atomicMin(&sc->kstar, bmin);
-}
-
-__device__ inline void k_fna_unflag(Geom g, uint8_t* type, int32_t* solid, DevScalars* sc) {
-    if (!sc->needScan) return;
-    const int ks = sc->kstar;
-    for (int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; i < g.N && i < ks; i += int64_t(gridDim.x) * blockDim.x) {
-        if (type[i] & T_PMASK) { type[i] &= uint8_t(~T_PMASK); solid[i] = 0; }
-    }
-}
-
-void lb_find_new_active(const Box& b, const Consts& k, const PartLB* plb, DevScalars* sc, hipStream_t s) {
-    launch<&k_fna_check, 1024, 1>(1, 1, s, b.g, b.solid, plb, k.nPart, sc);
-    const int64_t nb = (b.g.N + 255) / 256;
-    const int grid = int(nb < FLAGS_GRID ? nb : FLAGS_GRID);  // grid-stride; most steps return early
-    launch_gs<&k_fna_scan, 1024, 1>(grid, 256, s, b.g, b.type, b.solid, plb, k.nPart, sc);
-    launch_gs<&k_fna_unflag, 1024, 1>(grid, 256, s, b.g, b.type, b.solid, sc);
-    // the scan's result (fna_finish) is taken by the next single-thread pass: k_begin_lb, or the
-    // next coupling step's k_flags_compute
+    if (threadIdx.x == 0) sc->kminP = found == INT_MAX ? -1 : found;
 }
 
 // ------------------------------------------------------------------------------------------
 // impactor nodes (updateObjectBoundaries + findNewActiveObject, LB.cpp:797-943)
 // ------------------------------------------------------------------------------------------
 // uncovered object nodes (LB.cpp:846-943). The previous object nodes (ascending list) that the
-// moved sphere no longer covers become fluid, interface or gas nodes. Pass 1 (k_obj_uncover_find,
+// moved sphere no longer covers become fluid, interface or gas nodes. Pass 1 (obj_uncover_find,
 // many blocks) compacts them in ascending order, each block over its slice of the list. Each
 // conversion reads the node types its predecessors in that order wrote, so pass 2
 // (k_obj_uncover, one block) takes the candidates in chunks of UNC_CHUNK: it stages their neighbour types in LDS, finds
 // neighbours that are candidates of the chunk through a hash table, decides the new types (see
 // below) and writes a chunk's results back before the next chunk stages its neighbourhood.
 constexpr int UNCOVER_THREADS = 1024, UNC_CHUNK = 1024;
-constexpr int UNC_MAX_BLOCKS = UNCOVER_BLOCKS_MAX, UNC_NODES_PER_BLOCK = 4096;
+constexpr int UNC_MAX_BLOCKS = UNCOVER_BLOCKS_MAX, UNC_NODES_PER_BLOCK = 1024, FIND_THREADS = 256;
 constexpr int UNC_HASH = 2048;  // open-addressing table of a chunk's candidates (at most half full)
 __device__ inline uint32_t unc_hash(int32_t key) { return (uint32_t(key) * 2654435761u) >> (32 - 11); }
 __device__ inline uint8_t uncover_type(bool anyFluid, bool anyGas) {
@@ -1116,17 +680,16 @@ __device__ inline int block_exclusive_scan(int v, int* sWave, int& total) {
 
 // pass 1: ordered compaction of the nodes of each block's slice of the list that left the sphere,
 // into the same slice of cand
-__device__ inline void k_obj_uncover_find(Geom g, const int32_t* objList, int32_t* cand, int* blockCount, int G,
-                                          const DevScalars* sc, const ObjLB* olb) {
-    if (int(blockIdx.x) >= G) return;  // G: the box's grid
-    __shared__ int sWave[UNCOVER_THREADS / 64 + 1];
+__device__ inline void obj_uncover_find(int blk, Geom g, const int32_t* objList, int32_t* cand, int* blockCount, int G,
+                                        const DevScalars* sc, const ObjLB* olb) {
+    __shared__ int sWave[FIND_THREADS / 64 + 1];
     const int tid = threadIdx.x;
     const int n = sc->nObjList;
     const int per = (n + G - 1) / G;
     const ObjLB O = olb[0];
-    const int beg = min(n, int(blockIdx.x) * per), end = min(n, beg + per);
+    const int beg = min(n, blk * per), end = min(n, beg + per);
     int m = 0;
-    for (int base = beg; base < end; base += UNCOVER_THREADS) {
+    for (int base = beg; base < end; base += FIND_THREADS) {
         const int kk = base + tid;
         int32_t i = 0;
         int flag = 0;
@@ -1141,7 +704,7 @@ __device__ inline void k_obj_uncover_find(Geom g, const int32_t* objList, int32_
         if (flag) cand[beg + m + pos] = i;
         m += tot;
     }
-    if (tid == 0) blockCount[blockIdx.x] = m;
+    if (tid == 0) blockCount[blk] = m;
 }
 
 // pass 2 (one block): the candidates of the G slices in order
@@ -1292,7 +855,7 @@ __device__ inline void k_obj_uncover(Geom g, S* f, uint8_t* type,
 // cover: every node inside an object sphere becomes an object node; ascending object node list.
 // Pass a covers the union box of the spheres and counts per block (blocks own consecutive
 // ranges of the box); pass b writes the list at the blocks' exclusive prefix offsets.
-constexpr int COVER_GRID = COVER_BLOCKS, COVER_BS = 256;
+constexpr int COVER_BS = 256;
 struct CoverBox {
     int lo[3], n[3], tot;
 };
@@ -1316,12 +879,13 @@ __device__ inline int inside_which(int x, int y, int z, const ObjLB* olb, int nO
         if (inside_sphere(x, y, z, olb[o].c[0], olb[o].c[1], olb[o].c[2], olb[o].r)) which = o;
     return which;
 }
-__device__ inline void k_obj_cover_a(Geom g, uint8_t* type, int32_t* solid, const ObjLB* olb,
+__device__ inline void k_obj_cover_a(int G, Geom g, uint8_t* type, int32_t* solid, const ObjLB* olb,
                                                           int nObj, int* blockCount, int32_t* seg, int segCap,
                                                           int32_t* changed, int changedCap, DevScalars* sc) {
+    if (int(blockIdx.x) >= G) return;  // G: the box's grid
     __shared__ int sWave[COVER_BS / 64 + 1];
     const CoverBox cb = cover_box(g, olb, nObj);
-    const int per = (cb.tot + gridDim.x - 1) / gridDim.x;
+    const int per = (cb.tot + G - 1) / G;
     const int beg = min(cb.tot, int(blockIdx.x) * per), end = min(cb.tot, beg + per);
     const bool segmented = cb.tot <= segCap;  // the block's nodes go to seg[beg ...] in order
     int cnt = 0;
@@ -1354,7 +918,7 @@ __device__ inline void k_obj_cover_a(Geom g, uint8_t* type, int32_t* solid, cons
     if (threadIdx.x == 0) blockCount[blockIdx.x] = cnt;
 }
 // the object node list: every block's nodes at the exclusive prefix of the block counts
-__device__ inline void k_obj_cover_b(Geom g, const uint8_t* type, const ObjLB* olb, int nObj,
+__device__ inline void obj_cover_b(int blk, int G, Geom g, const uint8_t* type, const ObjLB* olb, int nObj,
                                                           const int* blockCount, const int32_t* seg, int segCap,
                                                           int32_t* objList, int cap, DevScalars* sc) {
     __shared__ int sWave[COVER_BS / 64 + 1];
@@ -1362,10 +926,10 @@ __device__ inline void k_obj_cover_b(Geom g, const uint8_t* type, const ObjLB* o
     const CoverBox cb = cover_box(g, olb, nObj);
     {
         int before = 0, all = 0;
-        for (int b = threadIdx.x; b < int(gridDim.x); b += COVER_BS) {
+        for (int b = threadIdx.x; b < G; b += COVER_BS) {
             const int v = blockCount[b];
             all += v;
-            if (b < int(blockIdx.x)) before += v;
+            if (b < blk) before += v;
         }
         int t1, t2;
         (void)block_exclusive_scan(before, sWave, t1);
@@ -1373,15 +937,15 @@ __device__ inline void k_obj_cover_b(Geom g, const uint8_t* type, const ObjLB* o
         if (threadIdx.x == 0) { sOff = t1; sTot = t2; }
         __syncthreads();
     }
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
+    if (blk == 0 && threadIdx.x == 0) {
         sc->nObjList = sTot < cap ? sTot : cap;
         if (sTot > cap) sc->listOverflow |= 1;
     }
     int off = sOff;
-    const int per = (cb.tot + gridDim.x - 1) / gridDim.x;
-    const int beg = min(cb.tot, int(blockIdx.x) * per), end = min(cb.tot, beg + per);
+    const int per = (cb.tot + G - 1) / G;
+    const int beg = min(cb.tot, blk * per), end = min(cb.tot, beg + per);
     if (cb.tot <= segCap) {
-        const int cnt = blockCount[blockIdx.x];
+        const int cnt = blockCount[blk];
         for (int k = threadIdx.x; k < cnt; k += COVER_BS)
             if (off + k < cap) objList[off + k] = seg[beg + k];
         return;
@@ -1403,30 +967,87 @@ __device__ inline void k_obj_cover_b(Geom g, const uint8_t* type, const ObjLB* o
     }
 }
 
-template <typename S>
-static void obj_impl(Box& b, const Consts& k, const ObjLB* olb, DevScalars* sc, hipStream_t s) {
-    using M = typename Types<S>::M;
-    using C = typename Types<S>::C;
-    // the object node list holds at most objCap nodes: one block per UNC_NODES_PER_BLOCK of them
-    const int grid = std::max(1, std::min(UNC_MAX_BLOCKS, (b.objCap + UNC_NODES_PER_BLOCK - 1) / UNC_NODES_PER_BLOCK));
-    int* uncCount = b.coverCount + COVER_GRID;
-    launch<&k_obj_uncover_find, UNCOVER_THREADS, 1>(grid, UNCOVER_THREADS, s, b.g, b.objList, b.objCand, uncCount, grid, sc, olb);
-    if (b.parity == 0)
-        launch<&k_obj_uncover<S, 0>, UNCOVER_THREADS, 1>(1, UNCOVER_THREADS, s, b.g, (S*)b.f, b.type, (M*)b.mass, (C*)b.aux,
-                                                         (C*)b.visc, b.objCand, uncCount, grid, sc, k, b.changed, b.changedCap);
-    else
-        launch<&k_obj_uncover<S, 1>, UNCOVER_THREADS, 1>(1, UNCOVER_THREADS, s, b.g, (S*)b.f, b.type, (M*)b.mass, (C*)b.aux,
-                                                         (C*)b.visc, b.objCand, uncCount, grid, sc, k, b.changed, b.changedCap);
-    // the candidate buffer of the uncover pass stages the cover pass's per-block node lists
-    launch_gs<&k_obj_cover_a, COVER_BS, 1>(COVER_GRID, COVER_BS, s, b.g, b.type, b.solid, olb, k.nObj, b.coverCount, b.objCand, b.objCap, b.changed, b.changedCap, sc);
-    launch_gs<&k_obj_cover_b, COVER_BS, 1>(COVER_GRID, COVER_BS, s, b.g, b.type, olb, k.nObj, b.coverCount, b.objCand, b.objCap, b.objList, b.objCap, sc);
+// First launch of the coupling: the particle flags of a list rebuild and the nodes the impactor left
+// (neither reads what the other writes; both read the types before the impactor's nodes change).
+struct CoupleArgs {
+    Geom g;
+    uint8_t* type;
+    int32_t *solid, *flagNew, *objList, *objCand, *changed;
+    int *coverCount, *uncCount;
+    const PartLB* plb;
+    const ObjLB* olb;
+    DevScalars* sc;
+    const int *nbrCount, *nbrList, *order;
+    int nPart, nObj, useList, objCap, changedCap;
+    int flagBlocks, findBlocks, coverBlocks, applyBlocks;
+};
+__device__ inline void k_couple_first(CoupleArgs a) {
+    int blk = int(blockIdx.x);
+    if (blk < a.flagBlocks)
+        return flags_compute(blk, a.flagBlocks, a.g, a.type, a.plb, a.nPart, a.flagNew, a.sc, a.nbrCount, a.nbrList, a.useList,
+                             a.order);
+    blk -= a.flagBlocks;
+    if (blk < a.findBlocks) obj_uncover_find(blk, a.g, a.objList, a.objCand, a.uncCount, a.findBlocks, a.sc, a.olb);
+}
+// Last launch: the impactor's node list, findNewActive and the new flags. The list is made from the
+// cover pass's counts and reads base types at most, findNewActive is idle on the steps that apply
+// flags, so the three do not meet.
+__device__ inline void k_couple_last(CoupleArgs a) {
+    int blk = int(blockIdx.x);
+    if (blk == 0) return find_new_active(a.g, a.type, a.solid, a.plb, a.nPart, a.sc);
+    blk -= 1;
+    if (blk < a.coverBlocks)
+        return obj_cover_b(blk, a.coverBlocks, a.g, a.type, a.olb, a.nObj, a.coverCount, a.objCand, a.objCap, a.objList,
+                           a.objCap, a.sc);
+    blk -= a.coverBlocks;
+    if (blk < a.applyBlocks)
+        flags_apply(blk, a.applyBlocks, a.g.N, a.type, a.solid, a.flagNew, a.sc, a.changed, a.changedCap);
 }
 
-void lb_object_update(Box& b, const Consts& k, const ObjLB* olb, DevScalars* sc, hipStream_t s) {
-    if (k.nObj <= 0) return;
-    if (b.prec == LBDEM_PREC_FP64) obj_impl<double>(b, k, olb, sc, s);
-    else if (b.prec == LBDEM_PREC_FP32) obj_impl<float>(b, k, olb, sc, s);
-    else obj_impl<__half>(b, k, olb, sc, s);
+template <typename S>
+static void obj_uncover(Box& b, const Consts& k, const CoupleArgs& a, hipStream_t s) {
+    using M = typename Types<S>::M;
+    using C = typename Types<S>::C;
+    if (b.parity == 0)
+        launch<&k_obj_uncover<S, 0>, UNCOVER_THREADS, 1>(1, UNCOVER_THREADS, s, b.g, (S*)b.f, b.type, (M*)b.mass, (C*)b.aux,
+                                                         (C*)b.visc, b.objCand, a.uncCount, a.findBlocks, a.sc, k, b.changed, b.changedCap);
+    else
+        launch<&k_obj_uncover<S, 1>, UNCOVER_THREADS, 1>(1, UNCOVER_THREADS, s, b.g, (S*)b.f, b.type, (M*)b.mass, (C*)b.aux,
+                                                         (C*)b.visc, b.objCand, a.uncCount, a.findBlocks, a.sc, k, b.changed, b.changedCap);
+}
+
+// The coupling step (LB.cpp:432-467): flags, impactor nodes, findNewActive, in four launches (two
+// without an impactor). order: the particles sorted by link cell (the rebuild's cell list), or null.
+// markFollows: lb_mark_edges is enqueued next and ends the step; else a launch of its own does.
+void lb_coupling(Box& b, const Consts& k, const PartLB* plb, const ObjLB* olb, DevScalars* sc, const int* nbrCount,
+                 const int* nbrList, bool useList, const int* order, bool markFollows, hipStream_t s) {
+    CoupleArgs a;
+    a.g = b.g; a.type = b.type; a.solid = b.solid; a.flagNew = b.flagNew; a.objList = b.objList; a.objCand = b.objCand;
+    a.changed = b.changed; a.coverCount = b.coverCount; a.uncCount = b.coverCount + COVER_BLOCKS;
+    a.plb = plb; a.olb = olb; a.sc = sc; a.nbrCount = nbrCount; a.nbrList = nbrList; a.order = order;
+    a.nPart = k.nPart; a.nObj = k.nObj; a.useList = useList ? 1 : 0; a.objCap = b.objCap; a.changedCap = b.changedCap;
+    // the flag passes stride (two particles a wavefront, sixteen nodes a thread or more): most steps only
+    // test a flag and return
+    a.flagBlocks = k.nPart > 0 ? std::min((k.nPart + 2 * FLAGS_WAVES - 1) / (2 * FLAGS_WAVES), FLAGS_GRID) : 0;
+    if (a.flagBlocks > 8) a.flagBlocks = (a.flagBlocks + 7) / 8 * 8;  // one share of the cell order per XCD
+    a.applyBlocks = int(std::min<int64_t>((b.g.N + 4095) / 4096, FLAGS_APPLY_GRID));
+    a.findBlocks = a.coverBlocks = 0;
+    if (k.nObj > 0) {
+        // the impactors' node list and the union of their boxes hold about objCap nodes
+        a.findBlocks = std::max(1, std::min(UNC_MAX_BLOCKS, (b.objCap + UNC_NODES_PER_BLOCK - 1) / UNC_NODES_PER_BLOCK));
+        a.coverBlocks = std::max(16, std::min(COVER_BLOCKS, (b.objCap + 255) / 256));
+    }
+    if (a.flagBlocks + a.findBlocks > 0) launch<&k_couple_first, 256, 8>(a.flagBlocks + a.findBlocks, 256, s, a);
+    if (k.nObj > 0) {
+        if (b.prec == LBDEM_PREC_FP64) obj_uncover<double>(b, k, a, s);
+        else if (b.prec == LBDEM_PREC_FP32) obj_uncover<float>(b, k, a, s);
+        else obj_uncover<__half>(b, k, a, s);
+        // the candidate buffer of the uncover pass stages the cover pass's per-block node lists
+        launch<&k_obj_cover_a, COVER_BS, 1>(a.coverBlocks, COVER_BS, s, a.coverBlocks, b.g, b.type, b.solid, olb, k.nObj,
+                                            b.coverCount, b.objCand, b.objCap, b.changed, b.changedCap, sc);
+    }
+    launch<&k_couple_last, 256, 1>(1 + a.coverBlocks + a.applyBlocks, 256, s, a);
+    if (!markFollows) launch<&k_couple_end, 64, 1>(1, 1, s, sc);
 }
 
 // ------------------------------------------------------------------------------------------

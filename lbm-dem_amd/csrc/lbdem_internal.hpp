@@ -129,8 +129,7 @@ struct DevScalars {
                                // non-active types) since the last LB step
     int fullMark;              // edge bits and link classes must be recomputed for the whole box
     int kminP;                 // lowest index of a particle-flagged node (-1: none)
-    int needScan;              // findNewActive needs the full scan
-    int kstar;                 // first particle node still covered
+    int nPartObj, nPartWall;   // block partials of the fused kernel with impactor / wall links
     int pad[1];
 };
 
@@ -176,7 +175,6 @@ struct Box {
     int changedCap;
     int ifCap, objCap;
     double* blockPart;         // per-block partials of the fused kernel (object F/M, extra mass, walls)
-    int32_t* blockFlag;        // per block: partials written
     uint64_t* bcm;             // N, boundary-link classes of edge nodes (valid where T_EDGE is set)
     int32_t* slipList;         // nodes with a diagonal link into a wall, when the walls slip (else null)
     int nSlip;
@@ -207,6 +205,9 @@ struct Consts {
     double unitLength, unitSpeed, unitAngVel, unitForce, unitTorque, unitVolume;
 };
 
+struct DemParams;
+struct DemState;
+
 // ---------------- launchers (lb.hip) ----------------
 void lb_init_fields(const Box& b, const Consts& k, hipStream_t s);
 // rec: LBDEM_RESTART_REC values per record, written at active node node[r]
@@ -224,16 +225,18 @@ void lb_fused_step(Box& b, const Consts& k, const PartLB* plb, const ObjLB* olb,
                    bool storeVel, hipStream_t s, hipEvent_t ev0 = nullptr, hipEvent_t ev1 = nullptr);
 void lb_hydro_finalize(const Box& b, const Consts& k, double* FHydro, double* MHydro, double* fluidVol,
                        DevScalars* sc, double* objFH, double* objMH, double* wallFH, bool diag, hipStream_t s);
-void lb_free_surface(Box& b, const Consts& k, DevScalars* sc, hipStream_t s);
-// particle flags of a neighbour-list rebuild; with useList the Verlet lists of that rebuild
-// resolve overlapping spheres (highest index wins) without atomics
-// order: the particles sorted by link cell (the rebuild's cell list), or null
-void lb_flags_rebuild_compute(const Box& b, const Consts& k, const PartLB* plb, DevScalars* sc, const int* nbrCount,
-                              const int* nbrList, bool useList, const int* order, hipStream_t s);
+// The launches between two fused kernels (front.hpp): hydro: the finalisation of the fused kernel's
+// sums; fs: the free surface; dp, ds (may be null): the neighbour list (forceList: built without asking
+// the trigger, and no forces) and the forces of DEM step demTimeStep
+void lb_front(Box& b, const Consts& k, DevScalars* sc, bool hydro, bool fs, double* FHydro, double* MHydro,
+              double* fluidVol, double* objFH, double* objMH, double* wallFH, const DemParams* dp, DemState* ds,
+              int demTimeStep, bool forceList, hipStream_t s);
+// the coupling step; useList: the Verlet lists of a rebuild resolve overlapping spheres (highest index
+// wins) without atomics; order: the particles sorted by link cell, or null; markFollows:
+// lb_mark_edges is enqueued next
+void lb_coupling(Box& b, const Consts& k, const PartLB* plb, const ObjLB* olb, DevScalars* sc, const int* nbrCount,
+                 const int* nbrList, bool useList, const int* order, bool markFollows, hipStream_t s);
 constexpr int PART_STRIDE_ = 32;
-void lb_flags_rebuild_apply(const Box& b, DevScalars* sc, hipStream_t s);
-void lb_find_new_active(const Box& b, const Consts& k, const PartLB* plb, DevScalars* sc, hipStream_t s);
-void lb_object_update(Box& b, const Consts& k, const ObjLB* olb, DevScalars* sc, hipStream_t s);
 int fused_grid_blocks(const Geom& g, int fz, int prec);  // blocks of the fused kernel for z-walk length fz
 constexpr int FUSED_TILE_X = 64, FUSED_TILE_Y = 4;  // threads of a fused-kernel tile (x, y)
 constexpr int COVER_BLOCKS = 512, UNCOVER_BLOCKS_MAX = 1024;  // grids of the impactor node passes
@@ -286,11 +289,8 @@ struct DemState {
     int* cellFill;
     int* cellItems;
     int* cellKey;
-    double* objContrib;        // per particle, per object: Fc(3) Mc(3) Fl(3) Ml(3)
-    double* wallContrib;       // per particle, per wall: Fc(3) Fl(3)
-    double* objSum;            // 12*MAX_OBJECTS
-    double* redPart;           // 2*64*12*MAX_OBJECTS block partials of the object/wall reduction
-    double* wallSum;           // 6*MAX_WALLS
+    double* redPart;           // per block of the force pass: impactor and wall sums (RED_COLS in dem.hpp)
+    int* redFlag;              // per block: the sums are written
     unsigned long long* blockMax;  // [VEL_SLOTS]: largest particle |v|^2 of the last integration, per slot (bit patterns)
     // objects
     double *ox0, *ox1, *ow1, *or_, *om, *oI, *oim, *oiI;
@@ -307,11 +307,10 @@ struct DemState {
     PartLB* plb;
     ObjLB* olb;
 };
-void dem_neighbor_list(const DemParams& p, DemState& d, DevScalars* sc, bool force, hipStream_t s);
-// hydroReady (may be null): an event the integration waits for (the hydrodynamic sums it reads);
-// false if the wait could not be enqueued
-bool dem_step(const DemParams& p, DemState& d, DevScalars* sc, int demTimeStep, hipStream_t s,
-              hipEvent_t hydroReady = nullptr);
+int dem_force_blocks(int nPart);  // blocks of the force pass
+constexpr int DEM_RED_COLS = 60;
+// totals, integration, objects and walls (after the forces and the hydrodynamic sums)
+void dem_integrate(const DemParams& p, DemState& d, int demTimeStep, hipStream_t s);
 void dem_refresh_views(const DemParams& p, DemState& d, hipStream_t s);
 
 // records of a download (particles, impactors, walls): column q of a record is component comp[q]

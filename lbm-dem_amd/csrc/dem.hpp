@@ -30,6 +30,7 @@ __device__ inline V ld3(const double* p, int i) { return V{p[3 * i], p[3 * i + 1
 __device__ inline void st3(double* p, int i, V v) { p[3 * i] = v.x; p[3 * i + 1] = v.y; p[3 * i + 2] = v.z; }
 __device__ inline V add(V a, V b) { return V{a.x + b.x, a.y + b.y, a.z + b.z}; }
 __device__ inline V sub(V a, V b) { return V{a.x - b.x, a.y - b.y, a.z - b.z}; }
+__device__ inline V neg(V a) { return V{-a.x, -a.y, -a.z}; }
 
 // ------------------------------------------------------------------------------------------
 // neighbour-list trigger (DEM.cpp:366-378, 460-470)
@@ -351,8 +352,8 @@ __device__ LubOut pair_lub(const DemParams& P, V xa, V xb, double ra, double rb,
     const double alpha = M_PI * P.kinVisc * rad * P.deltat;
     const double beta1 = bnum / bden;
     const double beta2 = beta1 * beta1, beta3 = beta1 * beta2;
-    const double b12 = (1 + beta1) * (1 + beta1), beta4 = b12 * b12;
-    const double beta5 = STRESS ? beta4 * (1 + beta1) : 1.0;
+    const double beta4 = pow((1 + beta1), 4.0);
+    const double beta5 = STRESS ? pow((1 + beta1), 5.0) : 1.0;
     if (dr < dmaxd(cut, lub_N)) {
         o.normal = true;
         Xa = 4.0 * beta2 / beta4;
@@ -499,22 +500,39 @@ __device__ void wall_like_contact(const DemParams& P, double dampCoeff, double r
 // Lanes per particle in the force kernel. A lane walks its share of the partners one after the other,
 // about 5 us each (two dependent gathers, then FP64 divisions, a root, a logarithm, an exponential),
 // so while the wavefronts of 16 lanes per particle fit on the GPU they finish first (480 spheres:
-// 17.4 us a launch with 4 lanes); beyond that 4 lanes waste fewer of them (31 000 spheres: all
-// wavefronts resident at once).
-constexpr int DEM_LANES_FEW = 16, DEM_LANES_MANY = 4, DEM_FEW = 8192;
+// 17.4 us a launch with 4 lanes, 11.8 with 16); beyond that 4 lanes waste fewer of them (31 000
+// spheres: all wavefronts resident at once). Either way the sums are those of four lanes, each of which
+// adds its partners in list order: a rounding that changed with the lanes would change positions in
+// their last bit, and a run with 4- or 2-byte populations amplifies that.
+constexpr int DEM_LANES_FEW = 16, DEM_LANES_MANY = 4, DEM_FEW = 8192, DEM_CHAINS = 4;
 
-// sum over the lanes of a particle's group, in a fixed butterfly order
-template <int LANES>
+// sum over N lanes, in a fixed butterfly order
+template <int N>
 __device__ inline double group_sum(double v) {
 #pragma unroll
-    for (int m = 1; m < LANES; m <<= 1) v += __shfl_xor(v, m, 64);
+    for (int m = 1; m < N; m <<= 1) v += __shfl_xor(v, m, 64);
     return v;
 }
+template <int N>
+__device__ inline V group_sum(V v) { return V{group_sum<N>(v.x), group_sum<N>(v.y), group_sum<N>(v.z)}; }
+// acc of chain (lane % DEM_CHAINS) plus the terms of that chain's partners of this round, in list
+// order (lanes chain, chain + 4, chain + 8, ... of the particle's group; every lane of the wavefront
+// must call this)
 template <int LANES>
-__device__ inline V group_sum(V v) { return V{group_sum<LANES>(v.x), group_sum<LANES>(v.y), group_sum<LANES>(v.z)}; }
+__device__ inline double chain_add(double acc, double t) {
+    if constexpr (LANES == DEM_CHAINS) return acc + t;
+    const int base = int(__lane_id()) & ~(LANES - 1), chain = int(__lane_id()) & (DEM_CHAINS - 1);
+#pragma unroll
+    for (int m = 0; m < LANES / DEM_CHAINS; ++m) acc += __shfl(t, base + chain + DEM_CHAINS * m, 64);
+    return acc;
+}
+template <int LANES>
+__device__ inline void chain_add(V& acc, V t) {
+    acc = V{chain_add<LANES>(acc.x, t.x), chain_add<LANES>(acc.y, t.y), chain_add<LANES>(acc.z, t.z)};
+}
 
 // Forces on particle p: LANES lanes per particle share its Verlet partners (lane l takes
-// partners l, l + LANES, ...), their partial sums are combined in a fixed order, and the
+// partners l, l + LANES, ...), their terms are combined in a fixed order (chain_add), and the
 // group's first lane adds the wall and impactor terms and writes the results. STRESS also
 // accumulates the particle's stress tensors (DEM.cpp:655-771) into its SP_REC record.
 // What a particle does to impactors and walls goes to a row of LDS, and a block that has any adds its
@@ -543,103 +561,113 @@ __device__ inline void dem_forces(const ForceArgs& a, int blk) {
     const bool waited = a.demTimeStep >= P.objWaitTime;
     // One pass over the lane's partners: the pair's data are gathered once and the three pair
     // terms follow in the reference's order; each accumulator sees its terms in partner order, as
-    // three separate loops would give them.
-    for (int k = lane; k < cnt; k += LANES) {
-        const int q = a.nbrList[p * NBR_CAP + k];
-        const int n1 = p > q ? p : q, n2 = p > q ? q : p;
-        const int slot = a.nbrSlot[p * NBR_CAP + k];
-        const V A = ld3(a.x0, n1), B = ld3(a.x0, n2), vA = ld3(a.x1, n1), vB = ld3(a.x1, n2);
-        const V wA = ld3(a.w1, n1), wB = ld3(a.w1, n2);
-        const double rA = a.r[n1], rB = a.r[n2];
-        V xi{0, 0, 0};
-        if (slot >= 0) xi = ld3(a.xiOld, slot);
-        // particle lubrication (DEM.cpp:2302-2521)
-        if (waited) {
-            const LubOut o = pair_lub<STRESS>(P, A, B, rA, rB, vA, vB, wA, wB, rB, rA);
-            if (o.act) {
-                if (p == n1) { Fl = add(Fl, o.F); Ml = add(Ml, o.T1); }
-                else { Fl = sub(Fl, o.F); Ml = add(Ml, o.T2); }
+    // three separate loops would give them (a term that is not there adds zero).
+    int rounds = (cnt + LANES - 1) / LANES;  // of the wavefront's longest list: every lane joins the sums
+#pragma unroll
+    for (int m = LANES; m < 64; m <<= 1) rounds = max(rounds, __shfl_xor(rounds, m, 64));
+    for (int round = 0; round < rounds; ++round) {
+        const int k = lane + LANES * round;
+        V tFc{0, 0, 0}, tMc{0, 0, 0}, tFl{0, 0, 0}, tMl{0, 0, 0}, tFr{0, 0, 0};  // this partner's terms
+        if (k < cnt) {
+            const int q = a.nbrList[p * NBR_CAP + k];
+            const int n1 = p > q ? p : q, n2 = p > q ? q : p;
+            const int slot = a.nbrSlot[p * NBR_CAP + k];
+            const V A = ld3(a.x0, n1), B = ld3(a.x0, n2), vA = ld3(a.x1, n1), vB = ld3(a.x1, n2);
+            const V wA = ld3(a.w1, n1), wB = ld3(a.w1, n2);
+            const double rA = a.r[n1], rB = a.r[n2];
+            V xi{0, 0, 0};
+            if (slot >= 0) xi = ld3(a.xiOld, slot);
+            // particle lubrication (DEM.cpp:2302-2521)
+            if (waited) {
+                const LubOut o = pair_lub<STRESS>(P, A, B, rA, rB, vA, vB, wA, wB, rB, rA);
+                if (o.act) {
+                    if (p == n1) { tFl = o.F; tMl = o.T1; }
+                    else { tFl = neg(o.F); tMl = o.T2; }
+                    if constexpr (STRESS) {
+                        for (int e = 0; e < 6; ++e) Sl[e] += p == n1 ? o.S1[e] : o.S2[e];
+                        if (o.normal) lubc += 1.0;
+                    }
+                }
+            }
+            // particle-particle contact (DEM.cpp:1487-1791)
+            const double rad = 0.5 * (rA + rB);
+            const double x12 = A.x - B.x, y12 = A.y - B.y, z12 = A.z - B.z;
+            const double r12 = sqrt(x12 * x12 + y12 * y12 + z12 * z12);
+            const double urx = vA.x - vB.x, ury = vA.y - vB.y, urz = vA.z - vB.z;
+            const double nx = x12 / r12, ny = y12 / r12, nz = z12 / r12;
+            const double gn = urx * nx + ury * ny + urz * nz;
+            const double del = 2 * rad - r12;
+            double fnx = 0, fny = 0, fnz = 0, ftx = 0, fty = 0, ftz = 0;
+            V fel{0, 0, 0}, fvis{0, 0, 0};  // DEM.cpp:1555-1679
+            if (del > 0.0) {
+                const double k_ = P.linearStiff, mu = P.frictionCoefPart;
+                fnx = k_ * del * nx - dampCoeff * gn * nx;
+                fny = k_ * del * ny - dampCoeff * gn * ny;
+                fnz = k_ * del * nz - dampCoeff * gn * nz;
                 if constexpr (STRESS) {
-                    for (int e = 0; e < 6; ++e) Sl[e] += p == n1 ? o.S1[e] : o.S2[e];
-                    if (o.normal) lubc += 1.0;
+                    fel = V{k_ * del * nx, k_ * del * ny, k_ * del * nz};
+                    fvis = V{-dampCoeff * gn * nx, -dampCoeff * gn * ny, -dampCoeff * gn * nz};
+                    // a contact counts where the box-wrapped centres are within 2 rmax (DEM.cpp:1647-1670)
+                    const double x1 = dbox(A.x, P.demSize[0]), y1 = dbox(A.y, P.demSize[1]), z1 = dbox(A.z, P.demSize[2]);
+                    const double x2 = dbox(B.x, P.demSize[0]), y2 = dbox(B.y, P.demSize[1]), z2 = dbox(B.z, P.demSize[2]);
+                    const double zij = z1 - z2, xij = x1 - x2, yij = y1 - y2;
+                    if (sqrt(zij * zij + yij * yij + xij * xij) <= 2.0 * (P.rmax)) coord += 1.0;
                 }
-            }
-        }
-        // particle-particle contact (DEM.cpp:1487-1791)
-        const double rad = 0.5 * (rA + rB);
-        const double x12 = A.x - B.x, y12 = A.y - B.y, z12 = A.z - B.z;
-        const double r12 = sqrt(x12 * x12 + y12 * y12 + z12 * z12);
-        const double urx = vA.x - vB.x, ury = vA.y - vB.y, urz = vA.z - vB.z;
-        const double nx = x12 / r12, ny = y12 / r12, nz = z12 / r12;
-        const double gn = urx * nx + ury * ny + urz * nz;
-        const double del = 2 * rad - r12;
-        double fnx = 0, fny = 0, fnz = 0, ftx = 0, fty = 0, ftz = 0;
-        V fel{0, 0, 0}, fvis{0, 0, 0};  // DEM.cpp:1555-1679
-        if (del > 0.0) {
-            const double k_ = P.linearStiff, mu = P.frictionCoefPart;
-            fnx = k_ * del * nx - dampCoeff * gn * nx;
-            fny = k_ * del * ny - dampCoeff * gn * ny;
-            fnz = k_ * del * nz - dampCoeff * gn * nz;
-            if constexpr (STRESS) {
-                fel = V{k_ * del * nx, k_ * del * ny, k_ * del * nz};
-                fvis = V{-dampCoeff * gn * nx, -dampCoeff * gn * ny, -dampCoeff * gn * nz};
-                // a contact counts where the box-wrapped centres are within 2 rmax (DEM.cpp:1647-1670)
-                const double x1 = dbox(A.x, P.demSize[0]), y1 = dbox(A.y, P.demSize[1]), z1 = dbox(A.z, P.demSize[2]);
-                const double x2 = dbox(B.x, P.demSize[0]), y2 = dbox(B.y, P.demSize[1]), z2 = dbox(B.z, P.demSize[2]);
-                const double zij = z1 - z2, xij = x1 - x2, yij = y1 - y2;
-                if (sqrt(zij * zij + yij * yij + xij * xij) <= 2.0 * (P.rmax)) coord += 1.0;
-            }
-            if (mu != 0.0) {
-                const double ox = rA * wA.x + rB * wB.x, oy = rA * wA.y + rB * wB.y, oz = rA * wA.z + rB * wB.z;
-                const double vx = urx + ny * oz - nz * oy - gn * nx;
-                const double vy = ury + nz * ox - nx * oz - gn * ny;
-                const double vz = urz + nx * oy - ny * ox - gn * nz;
-                const double xin = xi.x * nx + xi.y * ny + xi.z * nz;
-                xi.x -= xin * nx; xi.y -= xin * ny; xi.z -= xin * nz;
-                const double kt = 0.2 * k_;
-                const double dct = P.kinVisc == 0.0 ? dampCoeff : 0.0;
-                ftx = -kt * xi.x - dct * vx; fty = -kt * xi.y - dct * vy; ftz = -kt * xi.z - dct * vz;
-                const double fnn = sqrt(fnx * fnx + fny * fny + fnz * fnz);
-                const double ftt = sqrt(ftx * ftx + fty * fty + ftz * ftz);
-                const double fri = mu * fnn;
-                const double tx = ftx / ftt, ty = fty / ftt, tz = ftz / ftt;
-                xi.x += vx * P.deltat; xi.y += vy * P.deltat; xi.z += vz * P.deltat;
-                if (fri < ftt) {
-                    ftx = fri * tx; fty = fri * ty; ftz = fri * tz;
-                    xi.x = -(1 / kt) * (ftx + dct * vx);
-                    xi.y = -(1 / kt) * (fty + dct * vy);
-                    xi.z = -(1 / kt) * (ftz + dct * vz);
+                if (mu != 0.0) {
+                    const double ox = rA * wA.x + rB * wB.x, oy = rA * wA.y + rB * wB.y, oz = rA * wA.z + rB * wB.z;
+                    const double vx = urx + ny * oz - nz * oy - gn * nx;
+                    const double vy = ury + nz * ox - nx * oz - gn * ny;
+                    const double vz = urz + nx * oy - ny * ox - gn * nz;
+                    const double xin = xi.x * nx + xi.y * ny + xi.z * nz;
+                    xi.x -= xin * nx; xi.y -= xin * ny; xi.z -= xin * nz;
+                    const double kt = 0.2 * k_;
+                    const double dct = P.kinVisc == 0.0 ? dampCoeff : 0.0;
+                    ftx = -kt * xi.x - dct * vx; fty = -kt * xi.y - dct * vy; ftz = -kt * xi.z - dct * vz;
+                    const double fnn = sqrt(fnx * fnx + fny * fny + fnz * fnz);
+                    const double ftt = sqrt(ftx * ftx + fty * fty + ftz * ftz);
+                    const double fri = mu * fnn;
+                    const double tx = ftx / ftt, ty = fty / ftt, tz = ftz / ftt;
+                    xi.x += vx * P.deltat; xi.y += vy * P.deltat; xi.z += vz * P.deltat;
+                    if (fri < ftt) {
+                        ftx = fri * tx; fty = fri * ty; ftz = fri * tz;
+                        xi.x = -(1 / kt) * (ftx + dct * vx);
+                        xi.y = -(1 / kt) * (fty + dct * vy);
+                        xi.z = -(1 / kt) * (ftz + dct * vz);
+                    }
+                    if constexpr (STRESS) fel = add(fel, V{ftx, fty, ftz});
                 }
-                if constexpr (STRESS) fel = add(fel, V{ftx, fty, ftz});
-            }
-        } else {
-            xi = V{0, 0, 0};
-        }
-        if (p == n1 && slot >= 0) st3(a.xiNew, slot, xi);
-        const double dfx = fnx + ftx, dfy = fny + fty, dfz = fnz + ftz;
-        const double dtx = fty * nz - ftz * ny, dty = ftz * nx - ftx * nz, dtz = ftx * ny - fty * nx;
-        if (p == n1) { Fc = add(Fc, V{dfx, dfy, dfz}); Mc = add(Mc, V{rA * dtx, rA * dty, rA * dtz}); }
-        else { Fc = sub(Fc, V{dfx, dfy, dfz}); Mc = add(Mc, V{rB * dtx, rB * dty, rB * dtz}); }
-        if constexpr (STRESS) {  // the same tensors for n1 and n2; FElas with the side's sign
-            add_arm(Sc, x12, y12, z12, dfx, dfy, dfz);
-            add_arm(Se, x12, y12, z12, fel.x, fel.y, fel.z);
-            add_arm(Sv, x12, y12, z12, fvis.x, fvis.y, fvis.z);
-            Fe = p == n1 ? add(Fe, fel) : sub(Fe, fel);
-        }
-        // electrostatic repulsion over every listed pair (DEM.cpp:1404-1484)
-        {
-            double fx, fy, fz;
-            if (del <= 0.0) {
-                const double e = P.electroForce * exp(del / P.debyeLength);
-                fx = e * nx; fy = e * ny; fz = e * nz;
             } else {
-                fx = P.electroForce * nx; fy = P.electroForce * ny; fz = P.electroForce * nz;
+                xi = V{0, 0, 0};
             }
-            if (p == n1) Fr = add(Fr, V{fx, fy, fz}); else Fr = sub(Fr, V{fx, fy, fz});
-            if constexpr (STRESS) add_arm(Sr, x12, y12, z12, fx, fy, fz);
+            if (p == n1 && slot >= 0) st3(a.xiNew, slot, xi);
+            const double dfx = fnx + ftx, dfy = fny + fty, dfz = fnz + ftz;
+            const double dtx = fty * nz - ftz * ny, dty = ftz * nx - ftx * nz, dtz = ftx * ny - fty * nx;
+            if (p == n1) { tFc = V{dfx, dfy, dfz}; tMc = V{rA * dtx, rA * dty, rA * dtz}; }
+            else { tFc = V{-dfx, -dfy, -dfz}; tMc = V{rB * dtx, rB * dty, rB * dtz}; }
+            if constexpr (STRESS) {  // the same tensors for n1 and n2; FElas with the side's sign
+                add_arm(Sc, x12, y12, z12, dfx, dfy, dfz);
+                add_arm(Se, x12, y12, z12, fel.x, fel.y, fel.z);
+                add_arm(Sv, x12, y12, z12, fvis.x, fvis.y, fvis.z);
+                Fe = p == n1 ? add(Fe, fel) : sub(Fe, fel);
+            }
+            // electrostatic repulsion over every listed pair (DEM.cpp:1404-1484)
+            {
+                double fx, fy, fz;
+                if (del <= 0.0) {
+                    const double e = P.electroForce * exp(del / P.debyeLength);
+                    fx = e * nx; fy = e * ny; fz = e * nz;
+                } else {
+                    fx = P.electroForce * nx; fy = P.electroForce * ny; fz = P.electroForce * nz;
+                }
+                tFr = p == n1 ? V{fx, fy, fz} : V{-fx, -fy, -fz};
+                if constexpr (STRESS) add_arm(Sr, x12, y12, z12, fx, fy, fz);
+            }
         }
+        chain_add<LANES>(Fl, tFl); chain_add<LANES>(Ml, tMl);
+        chain_add<LANES>(Fc, tFc); chain_add<LANES>(Mc, tMc); chain_add<LANES>(Fr, tFr);
     }
-    Fc = group_sum<LANES>(Fc); Mc = group_sum<LANES>(Mc); Fl = group_sum<LANES>(Fl); Ml = group_sum<LANES>(Ml); Fr = group_sum<LANES>(Fr);
+    Fc = group_sum<DEM_CHAINS>(Fc); Mc = group_sum<DEM_CHAINS>(Mc); Fl = group_sum<DEM_CHAINS>(Fl); Ml = group_sum<DEM_CHAINS>(Ml);
+    Fr = group_sum<DEM_CHAINS>(Fr);
     double Sw[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};  // contact stress of walls and impactors
     if constexpr (STRESS) {
         for (int e = 0; e < 6; ++e) Sl[e] = group_sum<LANES>(Sl[e]);

@@ -471,7 +471,7 @@ static bool plan_buffers(const Plan& p, Box& b, DemState& d, DevScalars*& sc, do
     b.ifCap = p.ifCap;
     b.objCap = p.objCap;
     b.changedCap = b.ifCap + b.objCap;
-    b.blockPartCap = std::max(fused_grid_blocks(p.g, 1, LBDEM_PREC_FP32), fused_grid_blocks(p.g, 1, LBDEM_PREC_FP16)) * PART_STRIDE_;  // the largest grid (z-walk 1)
+    b.blockPartCap = part_stride(p.g) * PART_STRIDE_;
     A(b.f, size_t(Q) * N * p.selt);
     A(b.type, N);
     A(b.solid, N);
@@ -936,6 +936,7 @@ static void finish_tuning(lbdem_ctx* c) {
     }
     if (!ok) (void)hipGetLastError();
     c->box.fz = lbdem_ctx::CAND[ok ? best : 0];
+    c->box.sumPairs = true;
     c->tuned = true;
 }
 
@@ -1165,6 +1166,7 @@ extern "C" int lbdem_set_tile(lbdem_ctx* c, int tileZ) {
         return c->fail(LBDEM_E_ARG, "tile z-walk length must be 0 (tune), 1, 2, 4 or 8");
     if (c->stream) HIPCHK(hipStreamSynchronize(c->stream));
     drop_graphs(c);  // captured steps hold the previous tile
+    c->box.sumPairs = false;
     if (tileZ == 0) {
         if (c->initialised && c->tuned)
             for (auto& pr : c->tuneEv)
@@ -1903,6 +1905,7 @@ extern "C" int lbdem_batch_create(lbdem_ctx* const* ctxs, int n, lbdem_batch** o
         (void)hipStreamSynchronize(c->stream);
         drop_graphs(c);  // captured with the context's own tile
         c->box.fz = fz;
+        c->box.sumPairs = false;
         c->batch = B;
         c->velState = 0;  // batched steps keep no velocity
     }

@@ -27,7 +27,7 @@ struct FusedArgs {
     DevScalars* sc;
     int nseg, nby, nbz;  // 64-node segments per row (tiles per row with 2-byte storage), row groups, z-slabs
     int gridBlocks;  // the box's grid (a batch launch covers the largest box; the rest return)
-    int partStride;  // of the columns of blockPart (the largest grid of the box, whatever the walk)
+    int sumMask;     // nodes of a walk that share one sum in 32 bits before the block's FP64 table, less 1
     int storeVel;    // every active node's density and velocity into aux (else interface nodes only)
     Consts k;
 };
@@ -140,12 +140,12 @@ __device__ inline T* at(T* plane, int32_t rowIdx, uint32_t laneBytes) {
 // opp(q)), wrapped through periodic faces
 template <typename S, int PAR>
 __device__ inline void load_pop(const FusedArgs<S>& a, const RowYZ& r, const LaneX& lx, bool act,
-                                typename Types<S>::C* gq) {
+                                typename StoreT<S>::Raw* gq) {
     if (!act) return;
 #pragma unroll
     for (int q = 0; q < Q; ++q) {
-        if (PAR == 0) gq[q] = StoreT<S>::ld(at(a.fq[q], r.row, lx.o));
-        else gq[q] = StoreT<S>::ld(at(a.fq[oppq(q)], r.nb(oppq(q)), lx.sel(cxq(oppq(q)))));
+        if (PAR == 0) gq[q] = StoreT<S>::raw(at(a.fq[q], r.row, lx.o));
+        else gq[q] = StoreT<S>::raw(at(a.fq[oppq(q)], r.nb(oppq(q)), lx.sel(cxq(oppq(q)))));
     }
 }
 
@@ -245,7 +245,11 @@ __device__ inline void collide_cell(const FusedArgs<S>& a, int32_t sp, uint8_t t
     }
     const C Fx = C(k.lbF[0]) + hx, Fy = C(k.lbF[1]) + hy, Fz = C(k.lbF[2]) + hz;
     const C sx = ux + C(0.5) * Fx * inv, sy = uy + C(0.5) * Fy * inv, sz = uz + C(0.5) * Fz * inv;
-    const C usq = sx * sx + sy * sy + sz * sz;
+    // 2-byte storage: the order of the fused products written out, as the rounding of usq decides free-surface
+    // and particle flags there, and which product the compiler fuses depends on the code around
+    C usq;
+    if constexpr (sizeof(S) == 2 && !NN) usq = fma(sz, sz, fma(sx, sx, sy * sy));
+    else usq = sx * sx + sy * sy + sz * sz;
     const C uF = sx * Fx + sy * Fy + sz * Fz;
     C om = C(k.omega), omf = C(k.omegaf);
     if constexpr (NN) {  // the node's own viscosity, updated first when the model asks for it
@@ -303,8 +307,8 @@ __device__ inline void flush_particles(int tid, int nthreads, const int* hkey, d
 // access stays coalesced; their boundary links run in a rolled loop over the precomputed link
 // classes, without further loads for gas and wall links.
 // Launch bounds of the fused kernel, in blocks (one wavefront per SIMD each) per CU: four for
-// 4- and 2-byte storage (128 VGPRs: the free-surface FP32 and FP16 kernels fit without spilling,
-// those without a free surface spill up to 4 words; LDS is at most 13 KB per block), two for
+// 4- and 2-byte storage (128 VGPRs: two words of the prologue's are spilled across the walk, none
+// inside it; LDS is at most 13 KB per block), two for
 // FP64 (its populations alone take 38 VGPRs per node, and two nodes are live).
 template <typename S> struct FusedOcc { static constexpr int value = sizeof(S) == 8 ? 2 : 4; };
 // Block-to-node mapping. Row order (see k_fused) for 4- and 8-byte storage; measured on the
@@ -317,11 +321,23 @@ template <typename S> struct FusedRowOrder { static constexpr bool value = sizeo
 // one 0.69 ms, two 0.78 ms (more loads in flight per CU slow the memory system down).
 template <typename S> struct FusedAhead { static constexpr int value = 1; };
 
+// Gas and wall links of edge nodes from the registers of the collision, one unrolled direction after
+// the other, instead of reading each value back from where it was stored, link by link: every link of
+// the rolled loop waits for a store and a load. For one-node walks (the boxes too small to fill the
+// GPU with longer ones, where one node's chain of waits is the launch) and FP64, which have the
+// registers; with 4- and 2-byte storage and a walk the next node's populations are live as well, the
+// kernel spills, and edge rows are few (256x320x256 FP32: 0.80 -> 0.83 ms a step with it). Whole
+// passes: 128^3 FP32 18.6 -> 18.0 ms, 91^3 FP64 closed box 8.6 -> 8.2 ms, 256x320x256 FP64 67.9 -> 67.3 ms.
+template <typename S, int FZ> struct FusedRegLinks { static constexpr bool value = FZ == 1 || sizeof(S) == 8; };
+
 // per-node bundle: type byte, populations, mass (particle or edge node), solid index (particle
-// node); the boundary-link classes of edge nodes (rare) are loaded where they are used
+// node); the boundary-link classes of edge nodes (rare) are loaded where they are used. The
+// populations stay as loaded until the node collides: converted here, 2-byte values would make the
+// wavefront wait for the next node's loads before this node's arithmetic instead of behind it
+// (256x320x256 impact box, FP16 storage, four-node walk: 0.70 -> 0.62 ms a step)
 template <typename S>
 struct Bundle {
-    typename Types<S>::C g[Q];
+    typename StoreT<S>::Raw g[Q];
     typename Types<S>::M m;
     int32_t s;
     uint8_t t;
@@ -343,6 +359,8 @@ __device__ inline void k_fused(FusedArgs<S> a) {
     using C = typename Types<S>::C;
     using M = typename Types<S>::M;
     constexpr int NT = FX * FY;
+    constexpr bool REGLINKS = FusedRegLinks<S, FZ>::value;
+    constexpr bool SUMPAIRS = sizeof(S) == 2 && FZ > 2;
     if (int(blockIdx.x) >= a.gridBlocks) return;
     __shared__ int hkey[HS];
     __shared__ double hval[HS][7];
@@ -392,9 +410,9 @@ __device__ inline void k_fused(FusedArgs<S> a) {
     const int yw = __builtin_amdgcn_readfirstlane(y);
     const int32_t N = int32_t(g.N), SZ = g.X * g.Y;
     const int lane = __lane_id();
-    const int z0 = bz * FZ;
+    const int z0 = __builtin_amdgcn_readfirstlane(bz) * FZ;
     auto type_at = [&](int zz) -> uint8_t {
-        return (col_ok && zz < FZ && z0 + zz < g.Z) ? a.type[int32_t(cidx(g, x, y, z0 + zz))] : uint8_t(T_WALL);
+        return (col_ok && zz < FZ && z0 + zz < g.Z) ? a.type[int32_t(cidx(g, x, yw, z0 + zz))] : uint8_t(T_WALL);
     };
 
     // Bundles of the current node and of the AH nodes after it are in registers; per node the
@@ -403,7 +421,7 @@ __device__ inline void k_fused(FusedArgs<S> a) {
     // so no load of a node ahead reads a slot that a store of the current node writes.
     constexpr int AH = FusedAhead<S>::value;
     Bundle<S> nb[AH + 1];  // nb[0]: current node, nb[k]: k nodes ahead
-    int32_t ic = col_ok ? int32_t(cidx(g, x, y, z0)) : 0;
+    int32_t ic = col_ok ? int32_t(cidx(g, x, yw, z0)) : 0;
     const LaneX lx(g, x, uint32_t(sizeof(S)));
 #pragma unroll
     for (int k = 0; k < AH; ++k) load_bundle<S, PAR>(a, RowYZ(g, yw, z0 + k), lx, ic + k * SZ, type_at(k), nb[k]);
@@ -422,7 +440,9 @@ __device__ inline void k_fused(FusedArgs<S> a) {
         __builtin_amdgcn_s_setprio(2);
         load_bundle<S, PAR>(a, RowYZ(g, yw, z + AH), lx, ic + AH * SZ, tAhead, nb[AH]);
         __builtin_amdgcn_s_setprio(0);
-        C* gc = nb[0].g;
+        C gc[Q];
+#pragma unroll
+        for (int q = 0; q < Q; ++q) gc[q] = StoreT<S>::value(nb[0].g[q]);
         const bool actc = nb[0].act;
         const uint8_t tc = nb[0].t;
         const double mc = double(nb[0].m);
@@ -433,11 +453,15 @@ __device__ inline void k_fused(FusedArgs<S> a) {
 #pragma unroll
         for (int c = 0; c < 7; ++c) r.d[c] = 0;
         r.n = 1; r.sx = 0; r.sy = 0; r.sz = 0; r.usq = 0;
+        uint64_t bcEarly = 0;  // the link classes of edge nodes, on their way while the node collides
+        if constexpr (REGLINKS) {
+            if (actc && (tc & T_EDGE)) bcEarly = a.bcm[ic];
+        }
         C nu = 0;
         if constexpr (NN) {
             if (actc) nu = a.visc[ic];
         }
-        if (actc) collide_cell<S, NN>(a, sc_, tc, x, y, z, mc, gc, nu, r);
+        if (actc) collide_cell<S, NN>(a, sc_, tc, x, yw, z, mc, gc, nu, r);
         if constexpr (NN) {
             if (actc && a.k.viscUpdate) a.visc[ic] = r.visc;
         }
@@ -446,21 +470,68 @@ __device__ inline void k_fused(FusedArgs<S> a) {
         __builtin_amdgcn_s_setprio(0);
 
         // boundary links of edge nodes (LB.cpp:1390-1528): the value reflected into the slot
-        // this node loads next step
-        // The post-collision value of link j is read back from where store_pop just put it
-        // (PAR 0: the node's own slot opp(j); PAR 1: slot j of the neighbour), which the same
-        // lane wrote, so it needs no staging; the reflected value then goes to the slot the node
-        // loads next step.
+        // this node loads next step (FusedRegLinks: gas and wall links from registers)
         const bool edge = actc && (tc & T_EDGE);
+        // In the rolled loop the post-collision value of link j is read back from where store_pop just
+        // put it (PAR 0: the node's own slot opp(j); PAR 1: slot j of the neighbour), which the same
+        // lane wrote, so it needs no staging; the reflected value then goes to the slot the node loads
+        // next step.
         if (__ballot(edge)) {
-            const uint64_t bc_ = edge ? a.bcm[ic] : 0;
+            const uint64_t bc_ = REGLINKS ? bcEarly : (edge ? a.bcm[ic] : 0);
             uint32_t lm = 0;
-            if (edge) {
+            if constexpr (REGLINKS) {
+                double wf[3] = {0.0, 0.0, 0.0};
+                const RowYZ rw(g, yw, z);
+#pragma unroll
+                for (int j = 1; j < Q; ++j) {
+                    const int cls = int(bc_ >> (BC_BITS * (j - 1))) & 7;
+                    if (cls == BC_NONE) continue;
+                    if (cls != BC_GAS && cls != BC_WALL) {
+                        lm |= 1u << j;
+                        continue;
+                    }
+                    const C gj = StoreT<S>::stored(gc[j]);
+                    C bcv = gj;
+                    if (cls == BC_GAS) {
+                        const C cu = C(cxq(j)) * r.sx + C(cyq(j)) * r.sy + C(czq(j)) * r.sz;
+                        bcv = -gj + C(wq(j)) * (C(9) * (cu * cu) - C(3) * r.usq);
+                    } else {
+                        const double v2 = 2.0 * double(gj);
+                        if (cxq(j)) wf[0] += cxq(j) > 0 ? v2 : -v2;
+                        if (cyq(j)) wf[1] += cyq(j) > 0 ? v2 : -v2;
+                        if (czq(j)) wf[2] += czq(j) > 0 ? v2 : -v2;
+                    }
+                    if (PAR == 0) StoreT<S>::st(at(a.fq[j], rw.nb(j), lx.sel(cxq(j))), bcv);
+                    else StoreT<S>::st(at(a.fq[oppq(j)], rw.row, lx.o), bcv);
+                }
+                // wall force of the node's links into the block's partials; the lanes of a wavefront
+                // nearly always face one wall, and add up before the one atomic per component
+                if (DIAG && a.k.nWall > 0 && !a.k.slip) {  // slip walls take no force (LB.cpp:1454-1482)
+                    const int wp = int(bc_ >> BC_WALL_SHIFT) & 7;
+                    const bool hit = wf[0] != 0.0 || wf[1] != 0.0 || wf[2] != 0.0;
+                    const unsigned long long hm = __ballot(hit);
+                    if (hm) {
+                        const int w0 = __shfl(wp, __ffsll(hm) - 1, 64);
+                        if (__ballot(hit && wp != w0) == 0) {
+#pragma unroll
+                            for (int c = 0; c < 3; ++c) {
+#pragma unroll
+                                for (int off = 32; off > 0; off >>= 1) wf[c] += __shfl_xor(wf[c], off, 64);
+                                if (lane == 0 && wf[c] != 0.0) atomicAdd(&sPart[PART_WALL + 3 * w0 + c], wf[c]);
+                            }
+                        } else if (hit) {
+#pragma unroll
+                            for (int c = 0; c < 3; ++c)
+                                if (wf[c] != 0.0) atomicAdd(&sPart[PART_WALL + 3 * wp + c], wf[c]);
+                        }
+                    }
+                }
+            } else if (edge) {
 #pragma unroll
                 for (int j = 1; j < Q; ++j)
                     if ((bc_ >> (BC_BITS * (j - 1))) & 7u) lm |= 1u << j;
             }
-            const Offs o(g, x, y, z);
+            const Offs o(g, x, yw, z);
             const int wprim = int(bc_ >> BC_WALL_SHIFT) & 7;
             while (lm) {
                 const int j = __ffs(lm) - 1;
@@ -471,10 +542,10 @@ __device__ inline void k_fused(FusedArgs<S> a) {
                 S* const nbs = a.f + int64_t(j) * N + yj;          // slot j of the neighbour
                 const C gj = StoreT<S>::ld(PAR == 0 ? own : nbs);
                 C bcv;
-                if (cls == BC_GAS) {
+                if (!REGLINKS && cls == BC_GAS) {
                     const C cu = C(cx_rt(j)) * r.sx + C(cy_rt(j)) * r.sy + C(cz_rt(j)) * r.sz;
                     bcv = -gj + C(w_rt(j)) * (C(9) * (cu * cu) - C(3) * r.usq);
-                } else if (cls == BC_WALL) {
+                } else if (!REGLINKS && cls == BC_WALL) {
                     if (DIAG && a.k.nWall > 0 && !a.k.slip) {  // slip walls take no force (LB.cpp:1454-1482)
                         const double v2 = 2.0 * double(gj);
                         double* wp = &sPart[PART_WALL + 3 * wprim];
@@ -518,7 +589,7 @@ __device__ inline void k_fused(FusedArgs<S> a) {
         // particle sums: the thread's z-walk usually stays in one sphere for several nodes, so the
         // contributions are summed in registers while the particle index is unchanged and added
         // to the block's table when it changes (and after the walk)
-        if (r.key != accKey) {
+        if (r.key != accKey || (SUMPAIRS && (zz & a.sumMask) == 0)) {
             if (accKey >= 0) add_particle<C>(accKey, acc, hkey, hval, a.hacc);
             accKey = r.key;
 #pragma unroll
@@ -535,15 +606,17 @@ __device__ inline void k_fused(FusedArgs<S> a) {
     }
     if (accKey >= 0) add_particle<C>(accKey, acc, hkey, hval, a.hacc);
     __syncthreads();
-    flush_particles(tid, NT, hkey, hval, a.hacc);
+    int tx = threadIdx.x + FX * threadIdx.y;
+    asm volatile("" : "+v"(tx));
+    flush_particles(tx, NT, hkey, hval, a.hacc);
     if (FSURF) {
         // interface list: one global reservation per block
         const int n = sIfCount;
         if (n > 0) {
-            if (tid == 0) sIfBase = atomicAdd(&a.sc->nIf, n);
+            if (tx == 0) sIfBase = atomicAdd(&a.sc->nIf, n);
             __syncthreads();
             const int base = sIfBase;
-            for (int k = tid; k < n; k += NT) {
+            for (int k = tx; k < n; k += NT) {
                 if (base + k < a.ifCap) a.ifList[base + k] = sIf[k];
                 else atomicOr(&a.sc->listOverflow, 1);
             }
@@ -555,16 +628,17 @@ __device__ inline void k_fused(FusedArgs<S> a) {
     // list of their own: the free surface needs their extra mass first.
     static_assert(PART_STRIDE <= FX, "one wavefront appends the block's partials");
     if (threadIdx.y == 0) {
-        const bool used = tid < PART_STRIDE && sPart[tid] != 0.0;
+        const bool used = tx < PART_STRIDE && sPart[tx] != 0.0;
         const uint32_t m = uint32_t(__ballot(used));
         constexpr uint32_t objBits = (1u << PART_WALL) - 1u;
         int pos = 0;
-        if (tid == 0 && (m & objBits)) pos = atomicAdd(&a.sc->nPartObj, 1);
-        if (tid == PART_WALL && (m & ~objBits)) pos = atomicAdd(&a.sc->nPartWall, 1);
+        if (tx == 0 && (m & objBits)) pos = atomicAdd(&a.sc->nPartObj, 1);
+        if (tx == PART_WALL && (m & ~objBits)) pos = atomicAdd(&a.sc->nPartWall, 1);
         const int po = __shfl(pos, 0, 64), pw = __shfl(pos, PART_WALL, 64);
-        if ((m & objBits) && tid < PART_WALL) a.blockPart[int64_t(tid) * a.partStride + po] = sPart[tid];
-        if ((m & ~objBits) && tid >= PART_WALL && tid < PART_STRIDE)
-            a.blockPart[int64_t(tid) * a.partStride + pw] = sPart[tid];
+        const int64_t col = int64_t(tx) * part_stride(g);
+        if ((m & objBits) && tx < PART_WALL) a.blockPart[col + po] = sPart[tx];
+        if ((m & ~objBits) && tx >= PART_WALL && tx < PART_STRIDE)
+            a.blockPart[col + pw] = sPart[tx];
     }
 }
 
@@ -637,7 +711,11 @@ void launch_fused(Box& b, const Consts& k, const PartLB* plb, const ObjLB* olb, 
     a.nseg = (b.g.X + FX - 1) / FX; a.nby = (b.g.Y + FY - 1) / FY; a.nbz = (b.g.Z + fz - 1) / fz;
     const int grid = fused_grid_blocks(b.g, fz, b.prec);
     a.gridBlocks = grid;
-    a.partStride = b.blockPartCap / PART_STRIDE;
+    // With 2-byte storage a rounding of these sums decides a particle flag within some hundred steps.
+    // A walk that the timing picked therefore sums pairs of nodes whatever its length, so that the
+    // pick between 2, 4 and 8 leaves the results alone (two: the pick of large boxes while the walk
+    // waited for each load). A walk set by the caller, or being timed, sums over its whole length.
+    a.sumMask = b.sumPairs ? 1 : 7;
     a.storeVel = storeVel ? 1 : 0;
     const bool fs = k.freeSurface != 0;
     if (ev0) (void)hipEventRecord(ev0, s);

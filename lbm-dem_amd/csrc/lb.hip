@@ -383,7 +383,7 @@ __device__ inline void k_hydro_finalize(HydroArgs a, Consts k, DevScalars* sc) {
 static HydroArgs hydro_args(const Box& b, const Consts& k, double* FHydro, double* MHydro, double* fluidVol, double* objFH,
                             double* objMH, double* wallFH, bool diag) {
     HydroArgs a;
-    a.part = b.blockPart; a.stride = b.blockPartCap / PART_STRIDE; a.hacc = b.hacc;
+    a.part = b.blockPart; a.stride = part_stride(b.g); a.hacc = b.hacc;
     a.FHydro = FHydro; a.MHydro = MHydro; a.fluidVol = fluidVol; a.objFH = objFH; a.objMH = objMH; a.wallFH = wallFH;
     a.diag = diag ? 1 : 0;
     a.blocks = PART_STRIDE + (k.nPart + HF_THREADS - 1) / HF_THREADS;

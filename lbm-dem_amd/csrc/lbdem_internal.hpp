@@ -136,18 +136,33 @@ struct DevScalars {
 template <typename Tst> struct StoreT;
 template <> struct StoreT<double> {
     using C = double;
+    using Raw = double;  // what a load in flight holds
+    __device__ static Raw raw(const double* p) { return *p; }
+    __device__ static double value(Raw r) { return r; }
     __device__ static double ld(const double* p) { return *p; }
     __device__ static void st(double* p, double v) { *p = v; }
+    __device__ static double stored(double v) { return v; }  // the value a store and a load give back
 };
 template <> struct StoreT<float> {
     using C = float;
+    using Raw = float;
+    __device__ static Raw raw(const float* p) { return *p; }
+    __device__ static float value(Raw r) { return r; }
     __device__ static float ld(const float* p) { return *p; }
     __device__ static void st(float* p, float v) { *p = v; }
+    __device__ static float stored(float v) { return v; }
 };
 template <> struct StoreT<__half> {
     using C = float;
+    using Raw = __half_raw;
+    __device__ static Raw raw(const __half* p) { return *reinterpret_cast<const __half_raw*>(p); }
+    __device__ static float value(Raw r) {
+#pragma clang fp contract(off)  // the product is exact; fused into a sum it would keep that sum's other product from being fused
+        return __half2float(__half(r)) * (1.0f / FP16_SCALE);
+    }
     __device__ static float ld(const __half* p) { return __half2float(*p) * (1.0f / FP16_SCALE); }
     __device__ static void st(__half* p, float v) { *p = __float2half_rn(v * FP16_SCALE); }
+    __device__ static float stored(float v) { return __half2float(__float2half_rn(v * FP16_SCALE)) * (1.0f / FP16_SCALE); }
 };
 
 // The device state of one box.
@@ -155,6 +170,7 @@ struct Box {
     Geom g;
     int prec;
     int fz = 8;                // z-walk length of the fused kernel's tiles (1, 2, 4 or 8)
+    bool sumPairs = false;     // 2-byte storage: particle sums of the walk in pairs of nodes (FusedArgs)
     void* f;                   // 19*N storage elements
     uint8_t* type;
     int32_t* solid;
@@ -239,6 +255,11 @@ void lb_coupling(Box& b, const Consts& k, const PartLB* plb, const ObjLB* olb, D
 constexpr int PART_STRIDE_ = 32;
 int fused_grid_blocks(const Geom& g, int fz, int prec);  // blocks of the fused kernel for z-walk length fz
 constexpr int FUSED_TILE_X = 64, FUSED_TILE_Y = 4;  // threads of a fused-kernel tile (x, y)
+// largest grid of the fused kernel over its walks and mappings: columns of the partials are this far apart
+__host__ __device__ inline int part_stride(const Geom& g) {
+    const int nseg = (g.X + FUSED_TILE_X - 1) / FUSED_TILE_X, nby = (g.Y + FUSED_TILE_Y - 1) / FUSED_TILE_Y;
+    return nseg * nby * g.Z + 8;
+}
 constexpr int COVER_BLOCKS = 512, UNCOVER_BLOCKS_MAX = 1024;  // grids of the impactor node passes
 void lb_download_f(const Box& b, double* out, hipStream_t s, int q0 = 0, int q1 = Q);
 void lb_download_mass(const Box& b, double* out, hipStream_t s);

@@ -87,3 +87,33 @@ def test_force_lanes_match_oracle(oracle_lib, gpu_lib, n):
     # FP64 records: 1e-10 of the largest entry, as in test_gpu_parity
     for A, B, w in ((pa, pb, "particles"), (oa, ob, "objects"), (wa, wb, "walls")):
         assert np.abs(A - B).max() <= 1e-10 * max(1.0, np.abs(A).max()), w
+
+
+@pytest.mark.parametrize("tile", [0, 4])
+def test_tuned_walk_sums_pairs_of_nodes(gpu_lib, tile):
+    """2-byte storage: the walk the timing picked gives the particle sums of the two-node walk (the
+    same 32-bit sums of pairs, added in FP64 in another order: 1e-12 of the largest force allows for
+    thousands of terms, while 32-bit sums over other groups of nodes differ by some 1e-8). A walk set by
+    the caller sums over its whole length."""
+    v, ps, obs = workloads.impact_box(**workloads.HEADLINE)
+    sims = []
+    for _ in range(2):
+        s = lbdem.Simulation(gpu_lib, lbdem.params_from_values(v, lbdem.PREC_FP16), ps, obs)
+        s.init()
+        s.cycle(40)
+        sims.append(s)
+    a, b = sims
+    pick = a.tuning()["tile"][2]
+    assert b.tuning()["tile"][2] in (1, 2, 4, 8)
+    if tile == 0 and pick == 1:
+        pytest.skip("the one-node walk was the fastest")
+    b.set_tile(2)
+    if tile:
+        a.set_tile(tile)
+    a.cycle(2)
+    b.cycle(2)
+    fa, fb = a.particles()[:, 9:15], b.particles()[:, 9:15]
+    d = np.abs(fa - fb).max() / np.abs(fb).max()
+    assert d <= 1e-12 if tile == 0 else 1e-12 < d <= 1e-5, (pick, d)
+    for s in sims:
+        s.close()

@@ -163,6 +163,19 @@ __device__ inline void store_pop(const FusedArgs<S>& a, const RowYZ& r, const La
     }
 }
 
+// c_q . (x, y, z) without the products by zero, which the compiler has to keep (a NaN times zero)
+// (419 -> 348 vector instructions a node; a step of the 256x320x256 impact box FP16 0.626 -> 0.619 ms,
+// FP32 0.792 -> 0.788, of 128^3 FP32 0.156 -> 0.152; the larger boxes mostly wait for memory)
+template <typename C>
+__device__ inline C dir_dot(int q, C x, C y, C z) {
+    C r = 0;
+    bool any = false;
+    if (cxq(q)) { r = cxq(q) > 0 ? x : -x; any = true; }
+    if (cyq(q)) { const C v = cyq(q) > 0 ? y : -y; r = any ? r + v : v; any = true; }
+    if (czq(q)) { const C v = czq(q) > 0 ? z : -z; r = any ? r + v : v; }
+    return r;
+}
+
 // one node's collision (node.cpp:75-207): reconstruct, interior forcing of particle nodes
 // (LB.cpp:1919-1962), BGK with Guo forcing. gc holds the post-streaming populations on entry
 // and the post-collision ones on return.
@@ -222,7 +235,9 @@ __device__ inline void collide_cell(const FusedArgs<S>& a, int32_t sp, uint8_t t
 #pragma unroll
     for (int q = 0; q < Q; ++q) {
         sum += gc[q];
-        jx += C(cxq(q)) * gc[q]; jy += C(cyq(q)) * gc[q]; jz += C(czq(q)) * gc[q];
+        if (cxq(q)) jx += C(cxq(q)) * gc[q];
+        if (cyq(q)) jy += C(cyq(q)) * gc[q];
+        if (czq(q)) jz += C(czq(q)) * gc[q];
     }
     const C n = C(1) + sum;
     const C inv = C(1) / n;  // one division per node: the quotients below differ by rounding only
@@ -245,12 +260,16 @@ __device__ inline void collide_cell(const FusedArgs<S>& a, int32_t sp, uint8_t t
     }
     const C Fx = C(k.lbF[0]) + hx, Fy = C(k.lbF[1]) + hy, Fz = C(k.lbF[2]) + hz;
     const C sx = ux + C(0.5) * Fx * inv, sy = uy + C(0.5) * Fy * inv, sz = uz + C(0.5) * Fz * inv;
-    // 2-byte storage: the order of the fused products written out, as the rounding of usq decides free-surface
-    // and particle flags there, and which product the compiler fuses depends on the code around
-    C usq;
-    if constexpr (sizeof(S) == 2 && !NN) usq = fma(sz, sz, fma(sx, sx, sy * sy));
-    else usq = sx * sx + sy * sy + sz * sz;
-    const C uF = sx * Fx + sy * Fy + sz * Fz;
+    // The order of the fused products is written out where the results hang on their rounding (free-surface
+    // and particle flags; 2-byte storage most): which one the compiler fuses depends on the code around.
+    C usq, uF;
+    if constexpr (NN) {
+        usq = sx * sx + sy * sy + sz * sz;
+        uF = sx * Fx + sy * Fy + sz * Fz;
+    } else {
+        usq = sizeof(S) == 2 ? fma(sz, sz, fma(sx, sx, sy * sy)) : fma(sz, sz, fma(sy, sy, sx * sx));
+        uF = fma(sz, Fz, fma(sy, Fy, sx * Fx));
+    }
     C om = C(k.omega), omf = C(k.omegaf);
     if constexpr (NN) {  // the node's own viscosity, updated first when the model asks for it
         const C nu = k.viscUpdate ? apparent_viscosity<C>(k, gc, n, sx, sy, sz, usq, nuIn) : nuIn;
@@ -260,10 +279,12 @@ __device__ inline void collide_cell(const FusedArgs<S>& a, int32_t sp, uint8_t t
     }
 #pragma unroll
     for (int q = 0; q < Q; ++q) {
-        const C cu = C(cxq(q)) * sx + C(cyq(q)) * sy + C(czq(q)) * sz;
-        const C cF = C(cxq(q)) * Fx + C(cyq(q)) * Fy + C(czq(q)) * Fz;
-        const C geq = C(wq(q)) * ((n - C(1)) + n * (C(3) * cu + C(4.5) * cu * cu - C(1.5) * usq));
-        gc[q] = gc[q] + om * (geq - gc[q]) + omf * C(wq(q)) * (C(9) * cu * cF + C(3) * (cF - uF));
+        const C cu = dir_dot(q, sx, sy, sz);
+        const C cF = dir_dot(q, Fx, Fy, Fz);
+        const C e = fma(C(-1.5), usq, fma(C(3), cu, C(4.5) * cu * cu));
+        const C fq = fma(cF, C(9) * cu, C(3) * (cF - uF));
+        // gc + om (geq - gc) + omf w fq with geq = w (n - 1 + n e)
+        gc[q] = fma(omf * C(wq(q)), fq, fma(om, fma(fma(n, e, n - C(1)), C(wq(q)), -gc[q]), gc[q]));
     }
     r.n = n; r.sx = sx; r.sy = sy; r.sz = sz; r.usq = usq; r.hx = hx; r.hy = hy; r.hz = hz;
 }

@@ -487,13 +487,12 @@ def batch_profile(prec, n_boxes=64, steps=400, tile=8):
 def step_chains(rows, first, last):
     """The dispatches between fused launches `first` and `last` of a kernel trace (rows: start ns,
     end ns, kernel name), one entry per step: the fused kernel's duration, the time to the next
-    fused launch, and for each chain of the step (free surface with the hydrodynamic finalisation;
-    DEM; coupling and edge marking) the span from its first start to its last end and its launch
+    fused launch, and for each chain of the step (free surface with the hydrodynamic finalisation, the
+    neighbour list and the forces; DEM integration; coupling and edge marking) the span from its first start to its last end and its launch
     count."""
     rows = sorted(rows)
     fused = [r for r in rows if "k_fused" in r[2]]
-    chain_of = (("free_surface", ("k_fs_", "k_hydro_finalize")),
-                ("dem", ("k_dem_", "k_maxdisp", "k_cells_", "k_nbr_")))
+    chain_of = (("free_surface", ("k_front", "k_hydro_finalize")), ("dem", ("k_dem_",)))
     steps = []
     for i in range(first, min(last, len(fused) - 1)):
         f0, f1 = fused[i], fused[i + 1]

@@ -244,7 +244,7 @@ int lbdem_estimate_bytes(const lbdem_params* params, int nParticles, const doubl
                          const double* objR, size_t* bytes);
 int lbdem_device_bytes(lbdem_ctx* ctx, size_t* bytes);
 
-/* Replay of captured step pairs in lbdem_cycle (no reference counterpart): on by default
+/* Replay of captured steps in lbdem_cycle (no reference counterpart): on by default
  * (LBDEM_GRAPHS=0 in the environment turns the default off); 0 launches every step's kernels
  * one by one. Results are the same either way. */
 int lbdem_use_graphs(lbdem_ctx* ctx, int enable);
@@ -252,7 +252,8 @@ int lbdem_use_graphs(lbdem_ctx* ctx, int enable);
 /* Tile tuner of the fused collide-stream kernel (no reference counterpart). Tiles are 64 x 4
  * threads; each thread walks tile[2] nodes along z. Unless fixed, the first LB steps time the
  * candidates 8, 4, 2, 1 (one launch per AA parity each) on the run's own state and keep the
- * fastest; results do not depend on the tile beyond FP64 summation order of block partials.
+ * fastest; results do not depend on the tile beyond the order in which a thread's particle sums
+ * and the block partials are added (with FP16 storage picks of 2, 4 and 8 add in the same order).
  * lbdem_set_tile: 0 tunes (default), 1/2/4/8 fixes the z-walk length. */
 typedef struct lbdem_tuning {
     int tile[3];
@@ -260,7 +261,7 @@ typedef struct lbdem_tuning {
     int nCandidates;
     int candidateZ[4];
     double candidateMs[4];       /* fused kernel time, both parities, per candidate */
-    int pairCaptured;            /* 1 when lbdem_cycle's next step pair replays a captured graph,
+    int pairCaptured;            /* 1 when lbdem_cycle's next steps replay a captured graph,
                                     i.e. the context's start-up (tuning, capture) is over */
 } lbdem_tuning;
 int lbdem_set_tile(lbdem_ctx* ctx, int tileZ);

@@ -511,8 +511,9 @@ static bool plan_buffers(const Plan& p, Box& b, DemState& d, DevScalars*& sc, do
     A(d.xiCur, 3 * slots); A(d.xiNext, 3 * slots);
     A(d.cellCount, size_t(p.ncell)); A(d.cellStart, size_t(p.ncell)); A(d.cellFill, size_t(p.ncell));
     A(d.cellItems, np1); A(d.cellKey, np1);
-    A(d.redPart, size_t(dem_force_blocks(int(np1))) * DEM_RED_COLS);
-    A(d.redFlag, size_t(dem_force_blocks(int(np1))));
+    const int force_blocks_cap = std::max(dem_force_blocks(int(np1), false), dem_force_blocks(int(np1), true));
+    A(d.redPart, size_t(force_blocks_cap) * DEM_RED_COLS);
+    A(d.redFlag, size_t(force_blocks_cap));
     A(d.blockMax, VEL_SLOTS);
     double** ovecs[] = {&d.ox0, &d.ox1, &d.ow1, &d.oFHydro, &d.oMHydro, &d.oFContact, &d.oMContact, &d.oFLub,
                         &d.oMLub, &d.oFTotal, &d.oMTotal, &d.oFGrav};
@@ -1671,7 +1672,7 @@ struct lbdem_batch {
         for (hipEvent_t e : mev) (void)hipEventDestroy(e);
         if (done) (void)hipEventDestroy(done);
         if (stream) (void)hipStreamDestroy(stream);
-        for (lbdem_ctx* c : m) c->batch = nullptr;
+        for (lbdem_ctx* c : m) { c->batch = nullptr; c->ds.inBatch = false; }
     }
 };
 
@@ -1907,6 +1908,7 @@ extern "C" int lbdem_batch_create(lbdem_ctx* const* ctxs, int n, lbdem_batch** o
         c->box.fz = fz;
         c->box.sumPairs = false;
         c->batch = B;
+        c->ds.inBatch = true;
         c->velState = 0;  // batched steps keep no velocity
     }
     *out = B;

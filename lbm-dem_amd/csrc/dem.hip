@@ -7,9 +7,9 @@
 
 namespace lbdem {
 
-int dem_force_blocks(int nPart) {
-    const int lanes = nPart <= DEM_FEW ? DEM_LANES_FEW : DEM_LANES_MANY;
-    return int((int64_t(nPart) * lanes + 255) / 256);
+int dem_force_lanes(int nPart, bool inBatch) { return !inBatch && nPart <= DEM_FEW ? DEM_LANES_FEW : DEM_LANES_MANY; }
+int dem_force_blocks(int nPart, bool inBatch) {
+    return int((int64_t(nPart) * dem_force_lanes(nPart, inBatch) + 255) / 256);
 }
 
 // One block (the last block of the integration launch, which runs beside the particles' blocks:
@@ -278,14 +278,15 @@ ForceArgs force_args(const DemParams& p, DemState& d, int demTimeStep) {
     f.xiw = d.xiw; f.xio = d.xio; f.nbrCount = d.nbrCount; f.nbrList = d.nbrList; f.nbrSlot = d.nbrSlot;
     f.xiOld = d.xiCur; f.xiNew = d.xiNext;
     f.ox0 = d.ox0; f.ox1 = d.ox1; f.ow1 = d.ow1; f.or_ = d.or_;
-    f.redPart = d.redPart; f.redFlag = d.redFlag; f.blocks = dem_force_blocks(p.nPart); f.demTimeStep = demTimeStep;
+    f.redPart = d.redPart; f.redFlag = d.redFlag; f.lanes = dem_force_lanes(p.nPart, d.inBatch); f.blocks = dem_force_blocks(p.nPart, d.inBatch);
+    f.demTimeStep = demTimeStep;
     f.stressPart = d.stressPart; f.shydro = d.shydro;
     return f;
 }
 
 void dem_integrate(const DemParams& p, DemState& d, int demTimeStep, hipStream_t s) {
     const int nb = (p.nPart + OBJ_THREADS - 1) / OBJ_THREADS;
-    launch<&k_dem_integrate, OBJ_THREADS, 1>(nb + 1, OBJ_THREADS, s, p, d, dem_force_blocks(p.nPart), demTimeStep, nb);
+    launch<&k_dem_integrate, OBJ_THREADS, 1>(nb + 1, OBJ_THREADS, s, p, d, dem_force_blocks(p.nPart, d.inBatch), demTimeStep, nb);
 }
 
 }  // namespace lbdem

@@ -322,7 +322,7 @@ struct ForceArgs {
     const double *ox0, *ox1, *ow1, *or_;
     double* redPart;      // per block: RED_COLS sums (see dem_forces)
     int* redFlag;         // per block: the sums are written
-    int blocks;
+    int blocks, lanes;
     int demTimeStep;
     double* stressPart;   // SP_REC per particle (with the stress diagnostics)
     const double* shydro; // 9 per particle
@@ -501,7 +501,8 @@ __device__ void wall_like_contact(const DemParams& P, double dampCoeff, double r
 // about 5 us each (two dependent gathers, then FP64 divisions, a root, a logarithm, an exponential),
 // so while the wavefronts of 16 lanes per particle fit on the GPU they finish first (480 spheres:
 // 17.4 us a launch with 4 lanes, 11.8 with 16); beyond that 4 lanes waste fewer of them (31 000
-// spheres: all wavefronts resident at once). Either way the sums are those of four lanes, each of which
+// spheres: all wavefronts resident at once). A batch's launch holds the spheres of all its boxes
+// (64 boxes of edge 48-128: 0.09 ms with 4 lanes, 0.54 with 16). Either way the sums are those of four lanes, each of which
 // adds its partners in list order: a rounding that changed with the lanes would change positions in
 // their last bit, and a run with 4- or 2-byte populations amplifies that.
 constexpr int DEM_LANES_FEW = 16, DEM_LANES_MANY = 4, DEM_FEW = 8192, DEM_CHAINS = 4;

@@ -492,7 +492,7 @@ __device__ inline void k_front5(FsArgs<S> a, NbrArgs n) {
     if (blk < n.slotBlocks) nbr_slots(n, blk, n.slotBlocks);
 }
 template <typename M, bool STRESS, int LANES>
-__device__ inline void k_front6(RedistArgs a, M* mass, ForceArgs f) {
+__device__ inline void k_front6(RedistArgs a, M* mass, const ForceArgs& f) {  // (walls indexed by a variable)
     int blk = int(blockIdx.x);
     if (blk < f.blocks) return dem_forces<STRESS, LANES>(f, blk);  // the longer pass first
     blk -= f.blocks;

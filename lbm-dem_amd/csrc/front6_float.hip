@@ -6,7 +6,7 @@ namespace lbdem {
 template <>
 void launch_front6<float>(const RedistArgs& r, float* mass, const ForceArgs& f, hipStream_t s) {
     const int g = r.blocks + f.blocks, bs = FS_THREADS;
-    const bool few = f.p.nPart <= DEM_FEW;
+    const bool few = f.lanes == DEM_LANES_FEW;
     if (f.p.stress) {
         if (few) launch<&k_front6<float, true, DEM_LANES_FEW>, FS_THREADS, 1>(g, bs, s, r, mass, f);
         else launch<&k_front6<float, true, DEM_LANES_MANY>, FS_THREADS, 1>(g, bs, s, r, mass, f);

@@ -39,10 +39,12 @@ using Pack = PackImpl<std::index_sequence_for<P...>, P...>;
 // pointers loaded from there are known to address global memory, as pointers in kernel arguments
 // are, so the bodies keep their global (not flat) memory instructions and atomic combining.
 #define LBDEM_CONST __attribute__((address_space(4)))
+// A body that takes a struct by constant reference reads it where it lies (a copy whose arrays are
+// indexed by a variable would live in scratch memory).
 template <size_t I, typename T>
-__device__ inline T leaf_value(const LBDEM_CONST PackLeaf<I, T>& l) {
+__device__ inline decltype(auto) leaf_value(const LBDEM_CONST PackLeaf<I, T>& l) {
     if constexpr (std::is_class<T>::value) return *(const T*)&l.v;  // trivially copyable struct
-    else return l.v;
+    else return T(l.v);
 }
 template <auto Body, typename... P, size_t... I>
 __device__ inline void apply_pack(const LBDEM_CONST PackImpl<std::index_sequence<I...>, P...>& t) {
@@ -79,7 +81,9 @@ template <auto Body, int MAXT, int MINW, typename Sig = decltype(Body)>
 struct Launcher;
 template <auto Body, int MAXT, int MINW, typename... P>
 struct Launcher<Body, MAXT, MINW, void (*)(P...)> {
-    using Tuple = Pack<P...>;
+    template <typename T>
+    using Held = std::remove_cv_t<std::remove_reference_t<T>>;
+    using Tuple = Pack<Held<P>...>;
     static_assert(std::is_trivially_copyable<Tuple>::value, "kernel arguments are copied as bytes");
     static inline const char tag = 0;
     static const char* signature() {  // "lbdem::Launcher<&lbdem::k_fused<float, 0, true, true, 8>, 256, 4, ...>"
@@ -93,18 +97,19 @@ struct Launcher<Body, MAXT, MINW, void (*)(P...)> {
         return s.c_str();
     }
     static void batch(dim3 g, dim3 b, size_t shm, hipStream_t s, const void* table) {
-        hipLaunchKernelGGL((kernel_batch<Body, MAXT, MINW, P...>), g, b, shm, s, static_cast<const Tuple*>(table));
+        hipLaunchKernelGGL((kernel_batch<Body, MAXT, MINW, Held<P>...>), g, b, shm, s, static_cast<const Tuple*>(table));
     }
     template <typename... A>
     static void run(unsigned elastic, dim3 g, dim3 b, size_t shm, hipStream_t s, A&&... a) {
         if (Recorder* r = current_recorder()) {
-            const Tuple t{{static_cast<P>(std::forward<A>(a))}...};
+            const Tuple t{{static_cast<Held<P>>(std::forward<A>(a))}...};
             RecordedLaunch op{&tag, signature(), &batch, g, b, shm, elastic, std::vector<unsigned char>(sizeof(Tuple))};
             std::memcpy(op.args.data(), &t, sizeof(Tuple));
             r->ops.push_back(std::move(op));
             return;
         }
-        hipLaunchKernelGGL((kernel_one<Body, MAXT, MINW, P...>), g, b, shm, s, static_cast<P>(std::forward<A>(a))...);
+        hipLaunchKernelGGL((kernel_one<Body, MAXT, MINW, Held<P>...>), g, b, shm, s,
+                           static_cast<Held<P>>(std::forward<A>(a))...);
     }
 };
 

@@ -294,6 +294,7 @@ enum { SP_HYDRO = 0, SP_LUB = 9, SP_CPAIR = 18, SP_CWALL = 27, SP_REP = 36, SP_E
        SP_FELAS = 63, SP_COORD = 66, SP_LUBC = 67, SP_REC = 68 };
 constexpr int VEL_SLOTS = 64;  // slots of the particle speed maximum (DemState::blockMax)
 struct DemState {
+    bool inBatch = false;  // stepped by a batch, whose launches hold many boxes (dem_force_lanes)
     // particles (FP64, vectors stored as 3 consecutive doubles)
     double *x0, *x1, *w1, *r, *m, *I, *im, *iI;
     double *FHydro, *MHydro, *FContact, *MContact, *FLub, *MLub, *FRep, *FTotal, *MTotal, *FGrav, *fluidVol;
@@ -328,7 +329,8 @@ struct DemState {
     PartLB* plb;
     ObjLB* olb;
 };
-int dem_force_blocks(int nPart);  // blocks of the force pass
+int dem_force_lanes(int nPart, bool inBatch);   // lanes per particle of the force pass
+int dem_force_blocks(int nPart, bool inBatch);  // its blocks
 constexpr int DEM_RED_COLS = 60;
 // totals, integration, objects and walls (after the forces and the hydrodynamic sums)
 void dem_integrate(const DemParams& p, DemState& d, int demTimeStep, hipStream_t s);

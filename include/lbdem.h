@@ -284,6 +284,8 @@ int lbdem_batch_cycle(lbdem_batch* batch, int nsteps);  /* nsteps even */
 int lbdem_batch_synchronize(lbdem_batch* batch);
 const char* lbdem_batch_last_error(const lbdem_batch* batch);
 int lbdem_batch_destroy(lbdem_batch* batch);         /* the contexts remain, usable alone again */
+/* A member may be destroyed before its batch; the batch then takes no more steps (LBDEM_E_STATE) and is
+ * only good for lbdem_batch_destroy, which leaves the other members usable. */
 /* z-walk length for every member: 1, 2, 4 or 8; 0: the batch's next step pairs run one candidate
  * each (8, 4, 2), timed with events on the batch stream, and the fastest is kept (the tile
  * autotuner of a batch) */

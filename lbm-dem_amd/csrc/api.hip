@@ -234,8 +234,11 @@ extern "C" int lbdem_create(const lbdem_params* params, lbdem_ctx** out) {
     return read_params(c);
 }
 
+static void batch_forget(lbdem_batch* B, lbdem_ctx* c);
+
 extern "C" int lbdem_destroy(lbdem_ctx* ctx) {
     if (ctx) {
+        if (ctx->batch) batch_forget(ctx->batch, ctx);
         if (ctx->stream) (void)hipStreamSynchronize(ctx->stream);
         delete ctx;
     }
@@ -1656,6 +1659,7 @@ struct lbdem_batch {
     std::vector<hipEvent_t> pev;
     std::vector<std::string> profName;  // kernels in order of first launch
     std::map<std::string, std::pair<double, int>> profTime;  // ms summed, launches
+    bool orphaned = false;  // a member was destroyed: the recorded launches name its memory
     std::string err;
     int fail(int code, const std::string& e) { err = e; return code; }
     ~lbdem_batch() {
@@ -1675,6 +1679,14 @@ struct lbdem_batch {
         for (lbdem_ctx* c : m) { c->batch = nullptr; c->ds.inBatch = false; }
     }
 };
+
+// c is about to be destroyed: the batch's work on it ends first, and the batch takes no more steps
+static void batch_forget(lbdem_batch* B, lbdem_ctx* c) {
+    (void)hipStreamSynchronize(B->stream);
+    B->m.erase(std::remove(B->m.begin(), B->m.end(), c), B->m.end());
+    B->orphaned = true;
+    c->batch = nullptr;
+}
 
 // the contexts' start-up is over: the launches of a step pair repeat (see steady_steps)
 static bool steady(const lbdem_ctx* c) {
@@ -1917,6 +1929,7 @@ extern "C" int lbdem_batch_create(lbdem_ctx* const* ctxs, int n, lbdem_batch** o
 
 extern "C" int lbdem_batch_cycle(lbdem_batch* B, int nsteps) {
     if (!B) return LBDEM_E_ARG;
+    if (B->orphaned) return B->fail(LBDEM_E_STATE, "a member of the batch was destroyed");
     if (nsteps < 0 || nsteps % 2) return B->fail(LBDEM_E_ARG, "a batch advances whole step pairs (nsteps even)");
     if (nsteps == 0) return 0;
     const size_t n = B->m.size();
@@ -1962,6 +1975,7 @@ extern "C" int lbdem_batch_cycle(lbdem_batch* B, int nsteps) {
 
 extern "C" int lbdem_batch_set_tile(lbdem_batch* B, int tileZ) {
     if (!B) return LBDEM_E_ARG;
+    if (B->orphaned) return B->fail(LBDEM_E_STATE, "a member of the batch was destroyed");
     if (tileZ != 0 && tileZ != 1 && tileZ != 2 && tileZ != 4 && tileZ != 8)
         return B->fail(LBDEM_E_ARG, "tile z-walk length must be 0 (tune), 1, 2, 4 or 8");
     if (tileZ == 0) {

@@ -389,7 +389,7 @@ static bool host_types(lbdem_ctx* c, const Geom& g, std::vector<uint8_t>& t, std
 // device buffers of a context: one list walked both by lbdem_init (allocating) and by
 // lbdem_estimate_bytes (summing), so the estimate is the bytes init takes
 // ---------------------------------------------------------------------------------------------
-constexpr size_t TMP_PLANNED = 8192;  // scratch of lbdem_total_mass / lbdem_get_info
+constexpr size_t TMP_PLANNED = 8192;  // scratch of lbdem_total_mass, lbdem_get_info, impactor and wall records
 
 struct Plan {
     Geom g;
@@ -1388,11 +1388,10 @@ static int fetch(lbdem_ctx* c, double* dst, const double* src, size_t n) {
     return 0;
 }
 
-// n records packed on the device and copied at once
-static int fetch_records(lbdem_ctx* c, const RecordMap& m, int n, double* rec) {
-    const size_t bytes = size_t(n) * size_t(m.cols) * sizeof(double);
-    double* d = c->tmp(bytes);
+// n records packed on the device into d and copied at once
+static int fetch_records(lbdem_ctx* c, const RecordMap& m, int n, double* d, double* rec) {
     if (!d) return c->fail(LBDEM_E_NOMEM, "device allocation failed");
+    const size_t bytes = size_t(n) * size_t(m.cols) * sizeof(double);
     dem_pack_records(m, n, d, c->stream);
     HIPCHK(hipGetLastError());
     HIPCHK(hipMemcpyAsync(rec, d, bytes, hipMemcpyDeviceToHost, c->stream));
@@ -1415,7 +1414,11 @@ extern "C" int lbdem_get_particles(lbdem_ctx* c, double* rec) {
     m.add(LBDEM_P_FLUIDVOL, d.fluidVol, 1);
     m.add(LBDEM_P_XIW, d.xiw, 3); m.add(LBDEM_P_XIO, d.xio, 3);
     m.add(LBDEM_P_R, d.r, 1); m.add(LBDEM_P_M, d.m, 1);
-    return fetch_records(c, m, np, rec);
+    // packed into the history buffer that is not current: between steps it holds nothing, as the next
+    // DEM step writes every entry of a list before one is read, so a read of the particles allocates
+    // nothing and needs no memory beyond the context's plan
+    static_assert(LBDEM_P_REC <= 3 * NBR_CAP, "a particle's record fits its history entries");
+    return fetch_records(c, m, np, d.xiNext, rec);
 }
 
 extern "C" int lbdem_get_objects(lbdem_ctx* c, double* rec) {
@@ -1431,7 +1434,8 @@ extern "C" int lbdem_get_objects(lbdem_ctx* c, double* rec) {
     m.add(LBDEM_O_FLUB, d.oFLub, 3); m.add(LBDEM_O_MLUB, d.oMLub, 3);
     m.add(LBDEM_O_FTOTAL, d.oFTotal, 3); m.add(LBDEM_O_MTOTAL, d.oMTotal, 3); m.add(LBDEM_O_FGRAV, d.oFGrav, 3);
     m.add(LBDEM_O_R, d.or_, 1); m.add(LBDEM_O_M, d.om, 1);
-    return fetch_records(c, m, no, rec);
+    static_assert(size_t(LBDEM_O_REC) * 2 * sizeof(double) <= TMP_PLANNED, "the planned scratch holds the records");
+    return fetch_records(c, m, no, c->tmp(size_t(no) * LBDEM_O_REC * sizeof(double)), rec);
 }
 
 extern "C" int lbdem_get_bodies(lbdem_ctx* c, double* rec) {
@@ -1530,7 +1534,8 @@ extern "C" int lbdem_get_walls(lbdem_ctx* c, double* rec) {
     m.cols = LBDEM_W_REC;
     m.add(LBDEM_W_FHYDRO, d.wFHydro, 3); m.add(LBDEM_W_FCONTACT, d.wFContact, 3);
     m.add(LBDEM_W_FLUB, d.wFLub, 3); m.add(LBDEM_W_FTOTAL, d.wFTotal, 3);
-    return fetch_records(c, m, nw, rec);
+    static_assert(size_t(LBDEM_W_REC) * MAX_WALLS * sizeof(double) <= TMP_PLANNED, "the planned scratch holds the records");
+    return fetch_records(c, m, nw, c->tmp(size_t(nw) * LBDEM_W_REC * sizeof(double)), rec);
 }
 
 extern "C" int lbdem_get_neighbors(lbdem_ctx* c, int cap, int* count, int* list) {

@@ -305,7 +305,8 @@ struct DemState {
     int* nbrCountOld;
     int* nbrListOld;
     double* xiCur;             // tangential history per slot (3 per slot), read by the force kernel
-    double* xiNext;            // written by the force kernel (buffers swap every step)
+    double* xiNext;            // written by the force kernel (buffers swap every step); between steps free
+                               // to use (lbdem_get_particles packs its records there)
     int* cellCount;
     int* cellStart;
     int* cellFill;

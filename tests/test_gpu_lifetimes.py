@@ -1,4 +1,6 @@
 """Contexts, batches and downloads against the order in which a program gives them up."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -37,3 +39,48 @@ def test_member_destroyed_before_its_batch(gpu_lib):
     assert a.info()["nActive"] == ref.info()["nActive"] and a.info()["lbTime"] == 31
     a.close()
     ref.close()
+
+
+def _free_bytes():
+    hip = ctypes.CDLL("libamdhip64.so.7")
+    free, total = ctypes.c_size_t(), ctypes.c_size_t()
+    assert hip.hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+    return free.value
+
+
+def test_record_reads_take_no_device_memory(gpu_lib, oracle_lib):
+    """Reading the particles, impactors and walls needs no memory beyond what lbdem_init took, also after a
+    field download has replaced the context's scratch, leaves the run as it is (touching spheres with
+    friction: the tangential histories are carried from step to step) and gives the oracle's values (FP64
+    tolerance of test_gpu_parity)."""
+    X, Y, Z, n = 60, 70, 62, 4000
+    rng = np.random.default_rng(2)
+    g = np.stack(np.meshgrid(np.arange(2.6, X - 2.5, 3.05), np.arange(2.6, Y - 9.0, 3.05), np.arange(2.6, Z - 2.5, 3.05),
+                             indexing="ij"), axis=-1).reshape(-1, 3)
+    x0 = g[rng.permutation(len(g))][:n] + rng.uniform(-0.12, 0.12, (n, 3))
+    v, _, _ = workloads.impact_box(size=(X, Y, Z), fluid_height=float(Y - 1), n_spheres=0, r=1.5, r_imp=3.0, y_imp=Y - 6.0,
+                                   speed=0.01, periodic=False)
+    v.update(frictionCoefPart=0.4)
+    ps = lbdem.ParticleSet(size=np.ones(len(x0), np.int32), r=np.full(len(x0), 1.5), x0=x0)
+    obs = lbdem.ObjectSet(r=np.array([3.0]), x0=np.array([[X / 2.0, Y - 6.0, Z / 2.0]]), x1=np.array([[0.0, -0.01, 0.0]]))
+    out = []
+    # the runtime takes memory of its own at the first launches and copies: a run of its own goes before
+    for lib, reads in ((gpu_lib, False), (oracle_lib, False), (gpu_lib, True)):
+        s = lbdem.Simulation(lib, lbdem.params_from_values(v, lbdem.PREC_FP64), ps, obs)
+        s.init()
+        for k in range(6):
+            s.dem_step()
+            if not reads:
+                continue
+            s.synchronize()
+            if k == 3:
+                s.fields(want_f=False)
+            before = _free_bytes()
+            s.particles(), s.objects(), s.walls()
+            assert _free_bytes() == before, k
+        out.append((s.particles(), s.objects(), s.walls()))
+        s.close()
+    out = out[1:]
+    assert np.abs(out[0][0][:, 43:46]).max() > 0 or np.abs(out[0][0][:, 40:43]).max() > 0
+    for A, B, w in zip(out[0], out[1], ("particles", "objects", "walls")):
+        assert np.abs(A - B).max() <= 1e-10 * max(1.0, np.abs(A).max()), w

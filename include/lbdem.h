@@ -249,18 +249,20 @@ int lbdem_device_bytes(lbdem_ctx* ctx, size_t* bytes);
  * one by one. Results are the same either way. */
 int lbdem_use_graphs(lbdem_ctx* ctx, int enable);
 
-/* Tile tuner of the fused collide-stream kernel (no reference counterpart). Tiles are 64 x 4
- * threads; each thread walks tile[2] nodes along z. Unless fixed, the first LB steps time the
- * candidates 8, 4, 2, 1 (one launch per AA parity each) on the run's own state and keep the
- * fastest; results do not depend on the tile beyond the order in which a thread's particle sums
- * and the block partials are added (with FP16 storage picks of 2, 4 and 8 add in the same order).
- * lbdem_set_tile: 0 tunes (default), 1/2/4/8 fixes the z-walk length. */
+/* Tile tuner of the fused collide-stream kernel (no reference counterpart). Tiles are 64 x 4 threads
+ * by tile[2] nodes along z, the nodes whose particle sums a thread adds together. Unless fixed, the
+ * first LB steps time walks of 8, 4, 2 and 1 nodes along z (one launch per AA parity each) on the run's
+ * own state and keep the fastest. A walk is one tile; with FP16 storage walks of 4 and 8 nodes run
+ * tiles of two one after the other, so picks of 2, 4 and 8 are one tile with one result. Results do not
+ * depend on the tile beyond the order in which a thread's particle sums and the block partials are
+ * added; lbdem_set_tile with the tile of a tuned run repeats that order.
+ * lbdem_set_tile: 0 tunes (default), 1/2/4/8 fixes the tile. */
 typedef struct lbdem_tuning {
     int tile[3];
     int tuned;
     int nCandidates;
     int candidateZ[4];
-    double candidateMs[4];       /* fused kernel time, both parities, per candidate */
+    double candidateMs[4];       /* fused kernel time, both parities, per candidate walk */
     int pairCaptured;            /* 1 when lbdem_cycle's next steps replay a captured graph,
                                     i.e. the context's start-up (tuning, capture) is over */
 } lbdem_tuning;
@@ -273,9 +275,9 @@ int lbdem_get_tuning(lbdem_ctx* ctx, lbdem_tuning* tuning);
  * grid dimension selects the box; each box keeps its own memory, parameters and counters). A step
  * pair of the batch is captured into a HIP graph per phase and replayed. Members must have run
  * past their start-up steps (the impactor wait, the tile tuner, the first LB step) and be at the
- * same step parity; the batch runs every member with one z-walk length of the fused kernel (at
+ * same step parity; the batch runs every member with one tile of the fused kernel (at
  * creation the largest box's; lbdem_batch_set_tile changes or tunes it). Results are those of
- * each context run alone with that walk. While a context belongs to a batch it is advanced only
+ * each context run alone with that tile. While a context belongs to a batch it is advanced only
  * through the batch; its downloads stay valid (they wait for the batch's work).
  * ------------------------------------------------------------------------------------------- */
 typedef struct lbdem_batch lbdem_batch;
@@ -286,11 +288,11 @@ const char* lbdem_batch_last_error(const lbdem_batch* batch);
 int lbdem_batch_destroy(lbdem_batch* batch);         /* the contexts remain, usable alone again */
 /* A member may be destroyed before its batch; the batch then takes no more steps (LBDEM_E_STATE) and is
  * only good for lbdem_batch_destroy, which leaves the other members usable. */
-/* z-walk length for every member: 1, 2, 4 or 8; 0: the batch's next step pairs run one candidate
+/* tile for every member: 1, 2, 4 or 8; 0: the batch's next step pairs run one candidate walk
  * each (8, 4, 2), timed with events on the batch stream, and the fastest is kept (the tile
  * autotuner of a batch) */
 int lbdem_batch_set_tile(lbdem_batch* batch, int tileZ);
-/* the batch's walk; *tuned = 0 while candidates are still being timed */
+/* the batch's tile; *tuned = 0 while candidates are still being timed */
 int lbdem_batch_get_tile(const lbdem_batch* batch, int* tileZ, int* tuned);
 /* Kernel timing of a batch (no reference counterpart; used by benchmarks): while enabled, each step
  * pair's batch launches run one by one with a HIP event after each (no graph replay; the host waits
@@ -340,7 +342,7 @@ typedef struct lbdem_run_result {
     double objects[2 * LBDEM_O_REC]; /* impactor records after the last step */
     double totalMass;            /* lbdem_total_mass after the last step */
     int nActive;                 /* active nodes after the last step */
-    int tileZ;                   /* z-walk length of the fused kernel the run finished with */
+    int tileZ;                   /* tile of the fused kernel the run finished with (lbdem_tuning) */
     int64_t nodeSteps;           /* sum over steps of the box's node count (totNodes * steps) */
     size_t deviceBytes;
     char message[128];           /* error message of a failed run */
@@ -371,7 +373,7 @@ typedef struct lbdem_pool_stats {
  * precision; see lbdem_batch_create), re-formed between chunks as runs join and leave; 0: every
  * run on its own stream. Set before the first submission. */
 int lbdem_pool_set_batching(lbdem_pool* pool, int enable);
-/* z-walk of the runs' batches: 0 (default): tuned on the batches themselves
+/* tile of the runs' batches: 0 (default): tuned on the batches themselves
  * (lbdem_batch_set_tile(batch, 0)) per storage precision, again when a batch is at least twice the
  * size of the one tuned on (up to 8 runs), the result reused by later batches, and start-up steps
  * alone use the 8-node walk (with batching off each run tunes its own); 1, 2, 4 or 8: fixed for

@@ -939,8 +939,8 @@ static void finish_tuning(lbdem_ctx* c) {
         if (ms < bestMs) { bestMs = ms; best = q; }
     }
     if (!ok) (void)hipGetLastError();
-    c->box.fz = lbdem_ctx::CAND[ok ? best : 0];
-    c->box.sumPairs = true;
+    const int walk = lbdem_ctx::CAND[ok ? best : 0];
+    c->box.use_tile(tile_of_walk(c->box.prec, walk), walk);
     c->tuned = true;
 }
 
@@ -966,7 +966,8 @@ static void enqueue_lb(lbdem_ctx* c, bool finalize = true) {  // LB::latticeBolz
     }
     if (!c->tuned && !c->profiling) {
         if (c->tuneLaunches < 2 * lbdem_ctx::NCAND) {  // next candidate launch, timed
-            c->box.fz = lbdem_ctx::CAND[c->tuneLaunches / 2];
+            const int walk = lbdem_ctx::CAND[c->tuneLaunches / 2];
+            c->box.use_tile(walk, walk);
             e0 = c->tuneEv[c->tuneLaunches][0];
             e1 = c->tuneEv[c->tuneLaunches][1];
             ++c->tuneLaunches;
@@ -1164,13 +1165,18 @@ static void drop_graphs(lbdem_ctx* c) {
     std::fill(std::begin(c->asked), std::end(c->asked), 0);
 }
 
+static int64_t walk4_blocks(const lbdem_ctx* c) {
+    Geom g{};
+    g.X = c->lbSize[0]; g.Y = c->lbSize[1]; g.Z = c->lbSize[2];
+    return fused_grid_blocks(g, 4, c->prm.precision);
+}
+
 extern "C" int lbdem_set_tile(lbdem_ctx* c, int tileZ) {
     if (!c) return LBDEM_E_ARG;
     if (tileZ != 0 && tileZ != 1 && tileZ != 2 && tileZ != 4 && tileZ != 8)
         return c->fail(LBDEM_E_ARG, "tile z-walk length must be 0 (tune), 1, 2, 4 or 8");
     if (c->stream) HIPCHK(hipStreamSynchronize(c->stream));
     drop_graphs(c);  // captured steps hold the previous tile
-    c->box.sumPairs = false;
     if (tileZ == 0) {
         if (c->initialised && c->tuned)
             for (auto& pr : c->tuneEv)
@@ -1179,7 +1185,7 @@ extern "C" int lbdem_set_tile(lbdem_ctx* c, int tileZ) {
         c->tuned = false;
         c->tuneLaunches = 0;
     } else {
-        c->box.fz = tileZ;
+        c->box.use_tile(tileZ, walk_of_tile(c->prm.precision, tileZ, walk4_blocks(c)));
         c->tuned = true;
     }
     return 0;
@@ -1190,7 +1196,7 @@ extern "C" int lbdem_get_tuning(lbdem_ctx* c, lbdem_tuning* t) {
     std::memset(t, 0, sizeof(*t));
     t->tile[0] = FUSED_TILE_X;
     t->tile[1] = FUSED_TILE_Y;
-    t->tile[2] = c->box.fz;
+    t->tile[2] = c->box.tz;
     t->tuned = c->tuned ? 1 : 0;
     t->nCandidates = lbdem_ctx::NCAND;
     for (int q = 0; q < lbdem_ctx::NCAND; ++q) {
@@ -1652,7 +1658,7 @@ struct lbdem_batch {
     BatchPhase ph[4];
     char* region = nullptr;  // caller-owned memory for the argument tables (else hipMalloc)
     size_t regionSize = 0, regionUsed = 0;
-    // z-walk of every member; while !tuned the next step pairs run one candidate each, timed (the
+    // tile of every member; while !tuned the next step pairs run one candidate walk each, timed (the
     // walks 8, 4 and 2: a batch has blocks enough that the 1-node walk never wins)
     static constexpr int NCAND = 3;
     int tile = 8;
@@ -1868,12 +1874,12 @@ static int batch_launch_pair(lbdem_batch* B, const BatchPhase& P) {
     return 0;
 }
 
-// every member on walk fz: the recorded pairs hold the previous walk and are dropped (after the
-// device is done with their tables, which the next recording may overwrite)
-static int batch_use_tile(lbdem_batch* B, int fz) {
+// every member on this tile and walk: the recorded pairs hold the previous one and are dropped (after
+// the device is done with their tables, which the next recording may overwrite)
+static int batch_use_tile(lbdem_batch* B, int tile, int walk) {
     bool same = true;
-    for (lbdem_ctx* c : B->m) same = same && c->box.fz == fz;
-    B->tile = fz;
+    for (lbdem_ctx* c : B->m) same = same && c->box.tz == tile && c->box.fz == walk;
+    B->tile = tile;
     if (same) return 0;
     BATCHCHK(hipStreamSynchronize(B->stream));
     for (BatchPhase& P : B->ph) {
@@ -1883,8 +1889,11 @@ static int batch_use_tile(lbdem_batch* B, int fz) {
         P = BatchPhase();
     }
     B->regionUsed = 0;
-    for (lbdem_ctx* c : B->m) c->box.fz = fz;
+    for (lbdem_ctx* c : B->m) c->box.use_tile(tile, walk);
     return 0;
+}
+static int batch_use_walk(lbdem_batch* B, int walk) {
+    return batch_use_tile(B, tile_of_walk(B->m[0]->box.prec, walk), walk);
 }
 
 extern "C" int lbdem_batch_create(lbdem_ctx* const* ctxs, int n, lbdem_batch** out) {
@@ -1914,16 +1923,15 @@ extern "C" int lbdem_batch_create(lbdem_ctx* const* ctxs, int n, lbdem_batch** o
     B->mev.resize(n, nullptr);
     for (hipEvent_t& e : B->mev)
         if (hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) { delete B; return LBDEM_E_DEVICE; }
-    // one z-walk tile for all members: the one tuned for the largest box
+    // one tile and walk for all members: those of the largest box
     const lbdem_ctx* big = c0;
     for (lbdem_ctx* c : B->m) if (c->box.g.N > big->box.g.N) big = c;
-    const int fz = big->box.fz;
-    B->tile = fz;
+    const int tile = big->box.tz, walk = big->box.fz;
+    B->tile = tile;
     for (lbdem_ctx* c : B->m) {
         (void)hipStreamSynchronize(c->stream);
         drop_graphs(c);  // captured with the context's own tile
-        c->box.fz = fz;
-        c->box.sumPairs = false;
+        c->box.use_tile(tile, walk);
         c->batch = B;
         c->ds.inBatch = true;
         c->velState = 0;  // batched steps keep no velocity
@@ -1946,7 +1954,7 @@ extern "C" int lbdem_batch_cycle(lbdem_batch* B, int nsteps) {
         int slot = -1;  // tuning: the candidate this pair times
         if (!B->tuned) {
             slot = B->tuneIdx++;
-            if (int e = batch_use_tile(B, lbdem_ctx::CAND[slot])) return e;
+            if (int e = batch_use_walk(B, lbdem_ctx::CAND[slot])) return e;
         }
         BatchPhase& P = B->ph[graph_phase(B->m[0])];
         if (!P.recorded) {
@@ -1969,7 +1977,7 @@ extern "C" int lbdem_batch_cycle(lbdem_batch* B, int nsteps) {
                     if (q == 0 || ms < bestMs) { bestMs = ms; best = q; }
                 }
                 B->tuned = true;
-                if (int e = batch_use_tile(B, lbdem_ctx::CAND[best])) return e;
+                if (int e = batch_use_walk(B, lbdem_ctx::CAND[best])) return e;
             }
         }
     }
@@ -1992,7 +2000,9 @@ extern "C" int lbdem_batch_set_tile(lbdem_batch* B, int tileZ) {
         return 0;
     }
     B->tuned = true;
-    return batch_use_tile(B, tileZ);
+    int64_t blocks4 = 0;
+    for (const lbdem_ctx* c : B->m) blocks4 += walk4_blocks(c);
+    return batch_use_tile(B, tileZ, walk_of_tile(B->m[0]->box.prec, tileZ, blocks4));
 }
 
 extern "C" int lbdem_batch_get_tile(const lbdem_batch* B, int* tileZ, int* tuned) {

@@ -27,7 +27,7 @@ struct FusedArgs {
     DevScalars* sc;
     int nseg, nby, nbz;  // 64-node segments per row (tiles per row with 2-byte storage), row groups, z-slabs
     int gridBlocks;  // the box's grid (a batch launch covers the largest box; the rest return)
-    int sumMask;     // nodes of a walk that share one sum in 32 bits before the block's FP64 table, less 1
+    int sumMask;     // nodes of a tile, which share one sum in 32 bits before the block's FP64 table, less 1
     int storeVel;    // every active node's density and velocity into aux (else interface nodes only)
     Consts k;
 };
@@ -381,7 +381,7 @@ __device__ inline void k_fused(FusedArgs<S> a) {
     using M = typename Types<S>::M;
     constexpr int NT = FX * FY;
     constexpr bool REGLINKS = FusedRegLinks<S, FZ>::value;
-    constexpr bool SUMPAIRS = sizeof(S) == 2 && FZ > 2;
+    constexpr bool SUBTILES = sizeof(S) == 2 && FZ > 2;
     if (int(blockIdx.x) >= a.gridBlocks) return;
     __shared__ int hkey[HS];
     __shared__ double hval[HS][7];
@@ -610,7 +610,7 @@ __device__ inline void k_fused(FusedArgs<S> a) {
         // particle sums: the thread's z-walk usually stays in one sphere for several nodes, so the
         // contributions are summed in registers while the particle index is unchanged and added
         // to the block's table when it changes (and after the walk)
-        if (r.key != accKey || (SUMPAIRS && (zz & a.sumMask) == 0)) {
+        if (r.key != accKey || (SUBTILES && (zz & a.sumMask) == 0)) {
             if (accKey >= 0) add_particle<C>(accKey, acc, hkey, hval, a.hacc);
             accKey = r.key;
 #pragma unroll
@@ -732,11 +732,7 @@ void launch_fused(Box& b, const Consts& k, const PartLB* plb, const ObjLB* olb, 
     a.nseg = (b.g.X + FX - 1) / FX; a.nby = (b.g.Y + FY - 1) / FY; a.nbz = (b.g.Z + fz - 1) / fz;
     const int grid = fused_grid_blocks(b.g, fz, b.prec);
     a.gridBlocks = grid;
-    // With 2-byte storage a rounding of these sums decides a particle flag within some hundred steps.
-    // A walk that the timing picked therefore sums pairs of nodes whatever its length, so that the
-    // pick between 2, 4 and 8 leaves the results alone (two: the pick of large boxes while the walk
-    // waited for each load). A walk set by the caller, or being timed, sums over its whole length.
-    a.sumMask = b.sumPairs ? 1 : 7;
+    a.sumMask = b.tz - 1;
     a.storeVel = storeVel ? 1 : 0;
     const bool fs = k.freeSurface != 0;
     if (ev0) (void)hipEventRecord(ev0, s);

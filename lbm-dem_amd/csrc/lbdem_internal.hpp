@@ -169,8 +169,10 @@ template <> struct StoreT<__half> {
 struct Box {
     Geom g;
     int prec;
-    int fz = 8;                // z-walk length of the fused kernel's tiles (1, 2, 4 or 8)
-    bool sumPairs = false;     // 2-byte storage: particle sums of the walk in pairs of nodes (FusedArgs)
+    int tz = 8;                // nodes along z of a tile, whose particle sums a thread adds together (1, 2, 4 or 8)
+    int fz = 8;                // nodes a thread of the fused kernel walks along z: tz, or with 2-byte storage
+                               // several tiles of two
+    void use_tile(int tile, int walk) { tz = tile; fz = walk; }
     void* f;                   // 19*N storage elements
     uint8_t* type;
     int32_t* solid;
@@ -254,6 +256,20 @@ void lb_coupling(Box& b, const Consts& k, const PartLB* plb, const ObjLB* olb, D
                  const int* nbrList, bool useList, const int* order, bool markFollows, hipStream_t s);
 constexpr int PART_STRIDE_ = 32;
 int fused_grid_blocks(const Geom& g, int fz, int prec);  // blocks of the fused kernel for z-walk length fz
+// With 2-byte storage a rounding of the particle sums in 32 bits decides a particle flag within some
+// hundred steps, so the results depend on how many nodes share one. Walks of 4 and 8 nodes are therefore
+// walks over tiles of two there whenever it is the library that chooses the walk, by timing or by the size
+// of the box: walks of 2, 4 and 8 then give the same sums, and the tile says which (two: the fastest walk
+// of large boxes while it waited for each load). The caller may still fix a tile of 4 or 8.
+inline int tile_of_walk(int prec, int walk) { return prec == LBDEM_PREC_FP16 && walk > 2 ? 2 : walk; }
+// The walk that a fixed tile takes; blocks4: blocks of the four-node walk over all boxes of a launch.
+// Event-timed launches with 2-byte storage, walks of four and two nodes: 9216 blocks 234 and 233 us, 7488
+// blocks 194 and 194, 4800 blocks 122 and 111, 256 blocks 44 and 29; 10 000 blocks 228 and 234, 12 544 blocks
+// 290 and 300, 20 480 blocks 458 and 485.
+constexpr int64_t WALK4_BLOCKS = 9600;
+inline int walk_of_tile(int prec, int tile, int64_t blocks4) {
+    return prec == LBDEM_PREC_FP16 && tile == 2 && blocks4 >= WALK4_BLOCKS ? 4 : tile;
+}
 constexpr int FUSED_TILE_X = 64, FUSED_TILE_Y = 4;  // threads of a fused-kernel tile (x, y)
 // largest grid of the fused kernel over its walks and mappings: columns of the partials are this far apart
 __host__ __device__ inline int part_stride(const Geom& g) {

@@ -47,9 +47,10 @@ def log(msg):
 def run_gpu(vals, ps, obs, prec, steps, warmup, run_steps=5000, timed_from=1500, every=100):
     """One headline run of ``run_steps`` coupled steps in precision ``prec``.
 
-    Untimed before the timed window: the ``warmup`` steps asked for, then step pairs until the
-    context's start-up is over (the fused kernel's tile tuner has picked its walk and the steady
-    step pair is captured as a HIP graph), then steps up to ``timed_from`` (the impactor meets the
+    Untimed before the timed window: the ``warmup`` steps asked for, then steps up to ``timed_from``,
+    the last four calls with the window's remainder of single steps, so that the fused kernel's tile
+    tuner has picked its walk and every chunk that the window's call replays, at its phase, is
+    captured as a HIP graph (the impactor meets the
     surface between steps 1000 and 1500, so the window lies in the impact phase: splash
     conversions, impactor uncover/cover). Timed: exactly ``steps`` steps, bracketed by device
     synchronisation. The run then continues to ``run_steps``; the whole run (first step to last,
@@ -81,15 +82,16 @@ def run_gpu(vals, ps, obs, prec, steps, warmup, run_steps=5000, timed_from=1500,
 
     t_run0 = time.perf_counter()
     advance(warmup)
-    if state["done"] < timed_from:
-        advance(timed_from - state["done"])
-    extra = 0
-    while True:
+    # a call of 20 + r steps takes a 16-step and a 4-step chunk and r single steps, as the window's call ends;
+    # single steps are captured when a phase asks a second time, and an odd r changes the phase: four calls
+    call, extra = 20 + steps % 4, 0
+    advance(max(0, timed_from - 4 * call - state["done"]))
+    for k in range(16):
         tu = sim.tuning()
-        if (tu["tuned"] and tu["pair_captured"]) or extra >= 64:
+        if k >= 4 and tu["tuned"] and tu["pair_captured"]:
             break
-        advance(4)   # a call runs its first step alone, then captures or replays step pairs
-        extra += 4
+        extra += max(0, state["done"] + call - max(timed_from, state["done"]))
+        advance(call)
     if not (tu["tuned"] and tu["pair_captured"]):
         log(f"[bench] {name}: start-up not finished after {extra} extra steps: {tu}")
     sim.synchronize()
@@ -98,7 +100,7 @@ def run_gpu(vals, ps, obs, prec, steps, warmup, run_steps=5000, timed_from=1500,
     mass0 = sim.total_mass()
     sim.synchronize()
     t0 = time.perf_counter()
-    sim.cycle(steps)   # steady-state step pairs replay a captured HIP graph
+    sim.cycle(steps)   # steady-state steps replay captured HIP graphs
     sim.synchronize()
     t1 = time.perf_counter()
     state["done"] += steps
@@ -137,7 +139,7 @@ def run_gpu(vals, ps, obs, prec, steps, warmup, run_steps=5000, timed_from=1500,
 
 def fused_kernel_run(vals, ps, obs, prec, run_steps, tile_z, every):
     """The fused collide-stream kernel over a whole run: the same run again, every fused launch
-    bracketed by HIP events on the library stream (launches outside graphs), with the z-walk the
+    bracketed by HIP events on the library stream (launches outside graphs), with the tile the
     first run's tuner chose. Returns the summed kernel time, the launch count and the mean number of
     active nodes (sampled every ``every`` steps)."""
     lib = lbdem.Library.load()
@@ -707,8 +709,8 @@ def main():
             "timed_window": {"first_step": main_res["window_start_step"], "steps": args.steps,
                              "untimed_steps_before": main_res["window_start_step"],
                              "startup_extra_steps": main_res["startup_extra_steps"],
-                             "note": "untimed: --warmup steps, steps to the impact phase, then step pairs until the "
-                                     "tile tuner is done and the step pair is captured"},
+                             "note": "untimed: --warmup steps, steps to the impact phase, in which the tile tuner "
+                                     "finishes and the window's chunks of steps are captured"},
             "tile_z": main_res["tile_z"],
             "whole_run": {"steps": main_res["run_steps"], "seconds": round(main_res["run_seconds"], 3),
                           "ms_per_step": round(main_res["run_ms_per_step"], 4),

@@ -263,8 +263,10 @@ typedef struct lbdem_tuning {
     int nCandidates;
     int candidateZ[4];
     double candidateMs[4];       /* fused kernel time, both parities, per candidate walk */
-    int pairCaptured;            /* 1 when lbdem_cycle's next steps replay a captured graph,
-                                    i.e. the context's start-up (tuning, capture) is over */
+    int pairCaptured;            /* 1 when lbdem_cycle's next steps replay captured graphs, i.e. the
+                                    context's start-up (tuning, capture) is over: the chunks of 16 and
+                                    of 4 steps at the present step parity are captured (up to three
+                                    steps that are left of a call go one by one until they come back) */
 } lbdem_tuning;
 int lbdem_set_tile(lbdem_ctx* ctx, int tileZ);
 int lbdem_get_tuning(lbdem_ctx* ctx, lbdem_tuning* tuning);

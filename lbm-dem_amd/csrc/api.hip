@@ -1203,10 +1203,11 @@ extern "C" int lbdem_get_tuning(lbdem_ctx* c, lbdem_tuning* t) {
         t->candidateZ[q] = lbdem_ctx::CAND[q];
         t->candidateMs[q] = c->tuneMs[q];
     }
-    // a chunk that the next lbdem_cycle call of its length replays
-    t->pairCaptured = 0;
+    // every chunk of the next lbdem_cycle call replays, whatever the call's length (single steps apart: a
+    // call has three at most)
+    t->pairCaptured = steady_steps(c) ? 1 : 0;
     for (int n = 0; n < lbdem_ctx::NCHUNK; ++n)
-        if (steady_steps(c) && c->graphExec[n][graph_phase(c)]) t->pairCaptured = 1;
+        if (lbdem_ctx::CHUNK[n] > 1 && !c->graphExec[n][graph_phase(c)]) t->pairCaptured = 0;
     return 0;
 }
 

@@ -1,4 +1,5 @@
-"""Contexts, batches and downloads against the order in which a program gives them up."""
+"""Contexts, batches, downloads and captured steps against the order in which a program uses and gives
+them up."""
 import ctypes
 
 import numpy as np
@@ -84,3 +85,29 @@ def test_record_reads_take_no_device_memory(gpu_lib, oracle_lib):
     assert np.abs(out[0][0][:, 43:46]).max() > 0 or np.abs(out[0][0][:, 40:43]).max() > 0
     for A, B, w in zip(out[0], out[1], ("particles", "objects", "walls")):
         assert np.abs(A - B).max() <= 1e-10 * max(1.0, np.abs(A).max()), w
+
+
+def test_start_up_is_over_when_no_chunk_is_left_to_capture(gpu_lib):
+    """lbdem_tuning.pairCaptured: not while a longer call would still capture a chunk of steps, nor at the
+    other step parity, whose chunks are graphs of their own."""
+    sim = _small(gpu_lib, 6, steps=0)
+
+    def captured():
+        return sim.tuning()["pair_captured"]
+
+    sim.cycle(4)   # start-up steps, one by one
+    assert not captured()
+    sim.cycle(4)
+    sim.cycle(4)
+    assert not captured()  # 16 steps would capture
+    sim.cycle(16)
+    assert captured()
+    sim.cycle(1)
+    assert not captured()
+    sim.cycle(20)
+    assert captured()
+    sim.cycle(1)
+    assert captured()
+    sim.use_graphs(False)
+    assert not captured()
+    sim.close()

@@ -318,12 +318,16 @@ __device__ inline void mark_full_b(Geom g, uint8_t* type, const int32_t* solid, 
     for (int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; i < g.N; i += int64_t(gridDim.x) * blockDim.x)
         mark_node(g, type, solid, bcm, int32_t(i));
 }
-// end of the coupling step's flag pass (flags_compute set kminP to INT_MAX): taken by the marking, or
-// by a launch of its own after a coupling step without an LB step
+// end of the coupling step's flag pass (flags_compute set kminP to INT_MAX) or of its search for the
+// lowest flagged node: taken by the marking, or by a launch of its own after a coupling step without an LB step
 __device__ inline void couple_end(DevScalars* sc) {
-    if (!sc->newNeighborList) return;
-    if (sc->kminP == INT_MAX) sc->kminP = -1;
-    sc->newNeighborList = 0;
+    if (sc->newNeighborList) {
+        if (sc->kminP == INT_MAX) sc->kminP = -1;
+        sc->newNeighborList = 0;
+    } else if (sc->fnaDue) {
+        sc->kminP = sc->fnaBest ? INT_MAX - sc->fnaBest : -1;
+        sc->fnaDue = sc->fnaBest = 0;
+    }
 }
 __device__ inline void k_couple_end(DevScalars* sc) { couple_end(sc); }
 
@@ -455,7 +459,6 @@ constexpr int FLAGS_UNROLL = 6;
 __device__ inline void flags_compute(int blk, int nblk, Geom g, const uint8_t* type, const PartLB* plb, int nPart, int32_t* flagNew,
                                 DevScalars* sc, const int* nbrCount, const int* nbrList, int useList,
                                 const int* order) {
-    if (!sc->newNeighborList) return;
     if (blk == 0 && threadIdx.x == 0) sc->kminP = INT_MAX;  // lowest flagged index, from flags_apply
     __shared__ double sq[FLAGS_WAVES][NBR_CAP][4];  // centre and radius of overlapping higher-index partners
     const int wv = __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> 6), lane = int(threadIdx.x) & 63;
@@ -546,7 +549,6 @@ __device__ inline void flags_compute(int blk, int nblk, Geom g, const uint8_t* t
 // clear every flag and solid index, apply the new flags (initializeParticleBoundaries)
 __device__ inline void flags_apply(int blk, int nblk, int64_t N, uint8_t* type, int32_t* solid, int32_t* flagNew,
                                    DevScalars* sc, int32_t* changed, int changedCap) {
-    if (!sc->newNeighborList) return;
     __shared__ int bmin;
     if (threadIdx.x == 0) bmin = INT_MAX;
     __syncthreads();
@@ -582,61 +584,84 @@ __device__ inline void flags_apply(int blk, int nblk, int64_t N, uint8_t* type, 
         atomicMin(&sc->kminP, bmin);
 }
 
-// findNewActive (LB.cpp:1980-2029), one block: when the lowest flagged node has left its particle, the
-// flagged nodes below the first one still inside its own lose their flag, and that one is the lowest
-// from then on. No node below the lowest is flagged, so the nodes are taken upwards from it, 16 384 at a
-// time, until a flagged one is inside: a few thousand nodes on, in the same sphere or the next
-// (a pass over the whole box and one over the nodes below its result were two launches and, on the
-// 256x320x256 box, 20 us when one was due). A step that rebuilt the flags has nothing to do: every
-// flag was set from this step's positions.
-constexpr int FNA_WORDS = 16;  // words of four type bytes per thread and round
-__device__ inline void find_new_active(const Geom& g, uint8_t* type, int32_t* solid, const PartLB* plb, int nPart,
-                                       DevScalars* sc) {
-    __shared__ int sMin;
-    if (sc->newNeighborList) return;
+// findNewActive (LB.cpp:1980-2029): when the lowest flagged node has left its particle, the flagged nodes
+// below the first one still inside its own lose their flag, and that one is the lowest from then on. No
+// node below the lowest is flagged. The search (in the coupling's first launch) takes stripes of 16 384
+// nodes upwards from it, one per block and round; a block stops once a lower stripe has a hit, so that
+// a search that ends a few thousand nodes on, in the same sphere or the next, costs one round, and one
+// that runs through the whole box, as when the only spheres low in the box leave it through a periodic
+// face, runs on every compute unit: a step with such a search of a 256x320x256 box takes 0.69 ms, as the
+// steps beside it, and 3.2 ms with one block. The flags go in the coupling's last launch (fna_unflag). In
+// between only the cover pass changes what the search reads, the index of the nodes an impactor covers,
+// which the search takes as they will be. A step that rebuilt the flags has nothing to do: every flag was
+// set from this step's positions.
+constexpr int FNA_WORDS = 16;       // words of four type bytes per thread and round
+constexpr int FNA_MAX_BLOCKS = 256; // one per compute unit
+constexpr int FNA_STRIPE = 256 * FNA_WORDS * 4;  // nodes of a block's round
+__device__ inline int inside_which(int x, int y, int z, const ObjLB* olb, int nObj) {
+    int which = -1;
+    for (int o = 0; o < nObj; ++o)
+        if (inside_sphere(x, y, z, olb[o].c[0], olb[o].c[1], olb[o].c[2], olb[o].r)) which = o;
+    return which;
+}
+// word w of the type bytes, the last N % 4 of them as one short word
+__device__ inline uint32_t type_word(const uint8_t* type, int64_t N, int64_t w) {
+    const int64_t nw = N / 4;
+    if (w < nw) return reinterpret_cast<const uint32_t*>(type)[w];
+    uint32_t t = 0;
+    if (w == nw)
+        for (int64_t i = 4 * nw; i < N; ++i) t |= uint32_t(type[i]) << (8 * int(i - 4 * nw));
+    return t;
+}
+__device__ inline void fna_scan(int blk, int nblk, const Geom& g, const uint8_t* type, const int32_t* solid, const PartLB* plb,
+                                int nPart, const ObjLB* olb, int nObj, DevScalars* sc) {
+    __shared__ int sBest, sStop;
     const int kp = sc->kminP;
     if (kp < 0) return;
     auto inside = [&](int64_t i) {
-        const int sp = solid[i];
-        if (sp < 0 || sp >= nPart) return false;
         int x, y, z;
         cell_xyz(g, i, x, y, z);
+        int sp = inside_which(x, y, z, olb, nObj);  // (the cover pass stores the impactor's index)
+        if (sp < 0) sp = solid[i];
+        if (sp < 0 || sp >= nPart) return false;
         const PartLB P = plb[sp];
         return inside_sphere(x, y, z, P.c[0], P.c[1], P.c[2], P.r);
     };
     if (inside(kp)) return;
-    const uint32_t* t32 = reinterpret_cast<const uint32_t*>(type);
-    const int64_t nw = g.N / 4;  // whole words; the tail is taken byte by byte
-    int found = INT_MAX;
-    for (int64_t w0 = kp / 4; w0 <= nw; w0 += 256 * FNA_WORDS) {
-        if (threadIdx.x == 0) sMin = INT_MAX;
+    if (blk == 0 && threadIdx.x == 0) sc->fnaDue = 1;
+    for (int64_t w0 = kp / 4 + int64_t(blk) * (FNA_STRIPE / 4); 4 * w0 < g.N; w0 += int64_t(nblk) * (FNA_STRIPE / 4)) {
+        if (threadIdx.x == 0) {
+            const int best = __hip_atomic_load(&sc->fnaBest, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            sStop = best > 0 && INT_MAX - best < 4 * w0;
+            sBest = 0;
+        }
         __syncthreads();
+        if (sStop) break;
         uint32_t t[FNA_WORDS];
 #pragma unroll
-        for (int u = 0; u < FNA_WORDS; ++u) {
-            const int64_t w = w0 + int64_t(u) * 256 + threadIdx.x;
-            t[u] = w < nw ? t32[w] : 0;
-            if (w == nw)
-                for (int64_t i = 4 * nw; i < g.N; ++i) t[u] |= uint32_t(type[i]) << (8 * int(i - 4 * nw));
-        }
+        for (int u = 0; u < FNA_WORDS; ++u) t[u] = type_word(type, g.N, w0 + int64_t(u) * 256 + threadIdx.x);
         int mymin = INT_MAX;
-        for (int u = 0; u < FNA_WORDS; ++u)
+        for (int u = 0; u < FNA_WORDS && mymin == INT_MAX; ++u)
             for (uint32_t m = t[u] & 0x80808080u; m && mymin == INT_MAX; m &= m - 1u) {
                 const int64_t i = 4 * (w0 + int64_t(u) * 256 + threadIdx.x) + (__ffs(m) - 1) / 8;
-                if (i >= kp && inside(i)) mymin = int(i);
+                if (inside(i)) mymin = int(i);
             }
-        if (mymin != INT_MAX) atomicMin(&sMin, mymin);
+        if (mymin != INT_MAX) atomicMax(&sBest, INT_MAX - mymin);
         __syncthreads();
-        found = sMin;
-        __syncthreads();
-        for (int u = 0; u < FNA_WORDS; ++u)
-            for (uint32_t m = t[u] & 0x80808080u; m; m &= m - 1u) {
-                const int64_t i = 4 * (w0 + int64_t(u) * 256 + threadIdx.x) + (__ffs(m) - 1) / 8;
-                if (i < found) { type[i] &= uint8_t(~T_PMASK); solid[i] = 0; }
-            }
-        if (found != INT_MAX) break;
+        const int best = sBest;
+        if (best == 0) continue;
+        if (threadIdx.x == 0) atomicMax(&sc->fnaBest, best);
+        break;
     }
-    if (threadIdx.x == 0) sc->kminP = found == INT_MAX ? -1 : found;
+}
+__device__ inline void fna_unflag(int blk, int nblk, int64_t N, uint8_t* type, int32_t* solid, const DevScalars* sc) {
+    if (!sc->fnaDue) return;
+    const int64_t end = sc->fnaBest ? int64_t(INT_MAX - sc->fnaBest) : N;
+    for (int64_t w = sc->kminP / 4 + int64_t(blk) * 256 + threadIdx.x; 4 * w < end; w += int64_t(nblk) * 256)
+        for (uint32_t m = type_word(type, N, w) & 0x80808080u; m; m &= m - 1u) {
+            const int64_t i = 4 * w + (__ffs(m) - 1) / 8;
+            if (i < end) { type[i] &= uint8_t(~T_PMASK); solid[i] = 0; }
+        }
 }
 
 // ------------------------------------------------------------------------------------------
@@ -873,12 +898,6 @@ __device__ inline CoverBox cover_box(const Geom& g, const ObjLB* olb, int nObj) 
     b.tot = b.n[0] * b.n[1] * b.n[2];
     return b;
 }
-__device__ inline int inside_which(int x, int y, int z, const ObjLB* olb, int nObj) {
-    int which = -1;
-    for (int o = 0; o < nObj; ++o)
-        if (inside_sphere(x, y, z, olb[o].c[0], olb[o].c[1], olb[o].c[2], olb[o].r)) which = o;
-    return which;
-}
 __device__ inline void k_obj_cover_a(int G, Geom g, uint8_t* type, int32_t* solid, const ObjLB* olb,
                                                           int nObj, int* blockCount, int32_t* seg, int segCap,
                                                           int32_t* changed, int changedCap, DevScalars* sc) {
@@ -967,8 +986,9 @@ __device__ inline void obj_cover_b(int blk, int G, Geom g, const uint8_t* type, 
     }
 }
 
-// First launch of the coupling: the particle flags of a list rebuild and the nodes the impactor left
-// (neither reads what the other writes; both read the types before the impactor's nodes change).
+// First launch of the coupling: the particle flags of a list rebuild, or findNewActive's search, and the
+// nodes the impactor left (none reads what another writes; all read the types before the impactor's nodes
+// change).
 struct CoupleArgs {
     Geom g;
     uint8_t* type;
@@ -979,29 +999,38 @@ struct CoupleArgs {
     DevScalars* sc;
     const int *nbrCount, *nbrList, *order;
     int nPart, nObj, useList, objCap, changedCap;
-    int flagBlocks, findBlocks, coverBlocks, applyBlocks;
+    int flagBlocks, scanBlocks, findBlocks, coverBlocks, applyBlocks;
 };
 __device__ inline void k_couple_first(CoupleArgs a) {
     int blk = int(blockIdx.x);
-    if (blk < a.flagBlocks)
-        return flags_compute(blk, a.flagBlocks, a.g, a.type, a.plb, a.nPart, a.flagNew, a.sc, a.nbrCount, a.nbrList, a.useList,
-                             a.order);
-    blk -= a.flagBlocks;
+    const int flags = max(a.flagBlocks, a.scanBlocks);
+    if (blk < flags) {
+        if (a.sc->newNeighborList) {
+            if (blk < a.flagBlocks)
+                flags_compute(blk, a.flagBlocks, a.g, a.type, a.plb, a.nPart, a.flagNew, a.sc, a.nbrCount, a.nbrList, a.useList,
+                              a.order);
+        } else if (blk < a.scanBlocks) {
+            fna_scan(blk, a.scanBlocks, a.g, a.type, a.solid, a.plb, a.nPart, a.olb, a.nObj, a.sc);
+        }
+        return;
+    }
+    blk -= flags;
     if (blk < a.findBlocks) obj_uncover_find(blk, a.g, a.objList, a.objCand, a.uncCount, a.findBlocks, a.sc, a.olb);
 }
-// Last launch: the impactor's node list, findNewActive and the new flags. The list is made from the
-// cover pass's counts and reads base types at most, findNewActive is idle on the steps that apply
-// flags, so the three do not meet.
+// Last launch: the impactor's node list and the new flags, or the flags that findNewActive takes away. The
+// list is made from the cover pass's counts and reads base types at most, so the two do not meet.
 __device__ inline void k_couple_last(CoupleArgs a) {
     int blk = int(blockIdx.x);
-    if (blk == 0) return find_new_active(a.g, a.type, a.solid, a.plb, a.nPart, a.sc);
-    blk -= 1;
     if (blk < a.coverBlocks)
         return obj_cover_b(blk, a.coverBlocks, a.g, a.type, a.olb, a.nObj, a.coverCount, a.objCand, a.objCap, a.objList,
                            a.objCap, a.sc);
     blk -= a.coverBlocks;
-    if (blk < a.applyBlocks)
-        flags_apply(blk, a.applyBlocks, a.g.N, a.type, a.solid, a.flagNew, a.sc, a.changed, a.changedCap);
+    if (blk < a.applyBlocks) {
+        if (a.sc->newNeighborList)
+            flags_apply(blk, a.applyBlocks, a.g.N, a.type, a.solid, a.flagNew, a.sc, a.changed, a.changedCap);
+        else
+            fna_unflag(blk, a.applyBlocks, a.g.N, a.type, a.solid, a.sc);
+    }
 }
 
 template <typename S>
@@ -1030,6 +1059,7 @@ void lb_coupling(Box& b, const Consts& k, const PartLB* plb, const ObjLB* olb, D
     // test a flag and return
     a.flagBlocks = k.nPart > 0 ? std::min((k.nPart + 2 * FLAGS_WAVES - 1) / (2 * FLAGS_WAVES), FLAGS_GRID) : 0;
     if (a.flagBlocks > 8) a.flagBlocks = (a.flagBlocks + 7) / 8 * 8;  // one share of the cell order per XCD
+    a.scanBlocks = k.nPart > 0 ? int(std::min<int64_t>((b.g.N + FNA_STRIPE - 1) / FNA_STRIPE, FNA_MAX_BLOCKS)) : 0;
     a.applyBlocks = int(std::min<int64_t>((b.g.N + 4095) / 4096, FLAGS_APPLY_GRID));
     a.findBlocks = a.coverBlocks = 0;
     if (k.nObj > 0) {
@@ -1037,7 +1067,8 @@ void lb_coupling(Box& b, const Consts& k, const PartLB* plb, const ObjLB* olb, D
         a.findBlocks = std::max(1, std::min(UNC_MAX_BLOCKS, (b.objCap + UNC_NODES_PER_BLOCK - 1) / UNC_NODES_PER_BLOCK));
         a.coverBlocks = std::max(16, std::min(COVER_BLOCKS, (b.objCap + 255) / 256));
     }
-    if (a.flagBlocks + a.findBlocks > 0) launch<&k_couple_first, 256, 8>(a.flagBlocks + a.findBlocks, 256, s, a);
+    const int first = std::max(a.flagBlocks, a.scanBlocks) + a.findBlocks;
+    if (first > 0) launch<&k_couple_first, 256, 8>(first, 256, s, a);
     if (k.nObj > 0) {
         if (b.prec == LBDEM_PREC_FP64) obj_uncover<double>(b, k, a, s);
         else if (b.prec == LBDEM_PREC_FP32) obj_uncover<float>(b, k, a, s);
@@ -1046,7 +1077,7 @@ void lb_coupling(Box& b, const Consts& k, const PartLB* plb, const ObjLB* olb, D
         launch<&k_obj_cover_a, COVER_BS, 1>(a.coverBlocks, COVER_BS, s, a.coverBlocks, b.g, b.type, b.solid, olb, k.nObj,
                                             b.coverCount, b.objCand, b.objCap, b.changed, b.changedCap, sc);
     }
-    launch<&k_couple_last, 256, 1>(1 + a.coverBlocks + a.applyBlocks, 256, s, a);
+    launch<&k_couple_last, 256, 1>(a.coverBlocks + a.applyBlocks, 256, s, a);
     if (!markFollows) launch<&k_couple_end, 64, 1>(1, 1, s, sc);
 }
 

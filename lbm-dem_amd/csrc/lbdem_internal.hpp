@@ -130,6 +130,7 @@ struct DevScalars {
     int fullMark;              // edge bits and link classes must be recomputed for the whole box
     int kminP;                 // lowest index of a particle-flagged node (-1: none)
     int nPartObj, nPartWall;   // block partials of the fused kernel with impactor / wall links
+    int fnaDue, fnaBest;       // findNewActive (fna_scan): due this step; INT_MAX less the new lowest node (0: none)
     int pad[1];
 };
 

@@ -947,7 +947,7 @@ static void finish_tuning(lbdem_ctx* c) {
 // the particle, impactor and wall sums of the fused kernel
 static void enqueue_hydro(lbdem_ctx* c) {
     lb_hydro_finalize(c->box, c->k, c->ds.FHydro, c->ds.MHydro, c->ds.fluidVol, c->sc, c->ds.oFHydro, c->ds.oMHydro,
-                      c->ds.wFHydro, true, c->stream);
+                      c->ds.wFHydro, c->stream);
 }
 // finalize = false: the sums are finalised with the free surface that follows
 static void enqueue_lb(lbdem_ctx* c, bool finalize = true) {  // LB::latticeBolzmannStep (LB.cpp:400-418)
@@ -979,7 +979,7 @@ static void enqueue_lb(lbdem_ctx* c, bool finalize = true) {  // LB::latticeBolz
     const bool storeVel = c->velState == 1;  // lbdem_store_velocity asked for this step
     c->velState = storeVel ? 2 : 0;
     // the stress diagnostics read every active node's hydrodynamic force from aux
-    lb_fused_step(c->box, c->k, c->ds.plb, c->ds.olb, c->sc, true, storeVel || c->stress, c->stream, e0, e1);
+    lb_fused_step(c->box, c->k, c->ds.plb, c->ds.olb, c->sc, storeVel || c->stress, c->stream, e0, e1);
     if (c->stress)
         lb_hydro_stress(c->box, c->ds.plb, c->dp.nPart, c->unit.Length, c->unit.Force, c->ds.shydro, c->stream);
     if (finalize) enqueue_hydro(c);
@@ -1006,11 +1006,11 @@ static void flush_fs(lbdem_ctx* c) {
     c->fsDeferred = false;
     enqueue_front(c, true, true, false);
 }
-// one goCycle (main.cpp:38-67) minus the output. With deferFs the step's free surface is left for the
-// next step (or flush_fs), whose DEM step it shares launches with: the free surface reads and writes
+// one goCycle (main.cpp:38-67) minus the output. The step's free surface is left for the next step
+// (or flush_fs), whose DEM step it shares launches with: the free surface reads and writes
 // the lattice and the DEM forces the particles, so the order between them does not matter, and the
 // integration, the first to read the fused kernel's sums, follows both.
-static void enqueue_step(lbdem_ctx* c, bool deferFs) {
+static void enqueue_step(lbdem_ctx* c) {
     c->realTime += c->unit.Time;
     ++c->currentTimeStep;
     ++c->lbTime;
@@ -1025,14 +1025,13 @@ static void enqueue_step(lbdem_ctx* c, bool deferFs) {
         if (c->prm.demSolve) enqueue_coupling(c, true);
         enqueue_lb(c, !c->freeSurface);
         c->fsDeferred = c->freeSurface;
-        if (!deferFs) flush_fs(c);
     } else if (c->demTime <= c->prm.demInitialRepeat) {
         if (c->prm.demSolve) enqueue_coupling(c);
     }
 }
 // n steps that leave whole steps behind
 static void enqueue_steps(lbdem_ctx* c, int n) {
-    for (int k = 0; k < n; ++k) enqueue_step(c, true);
+    for (int k = 0; k < n; ++k) enqueue_step(c);
     flush_fs(c);
 }
 
@@ -1146,7 +1145,7 @@ extern "C" int lbdem_cycle(lbdem_ctx* c, int nsteps) {
                 }
             }
         }
-        enqueue_step(c, true);
+        enqueue_step(c);
         ++s;
     }
     flush_fs(c);  // every call leaves whole steps behind
@@ -1610,9 +1609,9 @@ struct BatchOp {
     std::vector<size_t> who;  // the batch members it runs, in table order
     std::string name;         // the kernel body with its template arguments
 };
-// "k_fused<float, 0, true, true, 4>" from a launcher's demangled type name, whose first template
+// "k_fused<float, 0, true, 4, false>" from a launcher's demangled type name, whose first template
 // argument is the body: "&lbdem::k_mark" or, for a function template,
-// "&(void lbdem::k_fused<float, 0, true, true, 4>(lbdem::FusedArgs<float>))"
+// "&(void lbdem::k_fused<float, 0, true, 4, false>(lbdem::FusedArgs<float>))"
 static std::string body_name(const char* sig) {
     const char* p = sig ? std::strstr(sig, "Launcher<&") : nullptr;
     if (!p) return sig ? sig : "?";

@@ -17,7 +17,7 @@ int dem_force_blocks(int nPart, bool inBatch) {
 // pass's blocks (in block order within four interleaved shares), then, on thread 0, objects:
 // totals and integration (DEM.cpp:786-790, 2742-2758) and walls: totals (DEM.cpp:773-775).
 constexpr int OBJ_THREADS = 256;
-// the numbers of the blocks that wrote sums, in order, in LDS (RED_MAX_BLOCKS of them at most)
+// the numbers of the blocks that wrote sums, in order, in LDS (RED_LIST of them at most: the callers' rounds)
 __device__ inline int flagged_blocks(const int* flag, int n, int* list, int* sWave) {
     int base = 0;
     for (int b0 = 0; b0 < n; b0 += OBJ_THREADS) {
@@ -38,7 +38,7 @@ __device__ inline int flagged_blocks(const int* flag, int n, int* list, int* sWa
     }
     return base;
 }
-static_assert(RED_COLS <= 64 && OBJ_THREADS == 4 * 64, "four threads per column");
+static_assert(DEM_RED_COLS <= 64 && OBJ_THREADS == 4 * 64, "four threads per column");
 constexpr int RED_LIST = 2048;  // block numbers per round
 __device__ inline void dem_objects(DemParams P, DemState d, int redBlocks, int demTimeStep) {
 #pragma clang fp contract(off)
@@ -52,16 +52,16 @@ __device__ inline void dem_objects(DemParams P, DemState d, int redBlocks, int d
     for (int b0 = 0; b0 < redBlocks; b0 += RED_LIST) {
         const int n = flagged_blocks(d.redFlag + b0, min(RED_LIST, redBlocks - b0), list, sWave);
         if (col < nco + ncw) {
-            const double* part = d.redPart + int64_t(b0) * RED_COLS + col;
+            const double* part = d.redPart + int64_t(b0) * DEM_RED_COLS + col;
             int k = share;
             for (; k + 28 < n; k += 32) {  // eight loads in flight
                 double v[8];
 #pragma unroll
-                for (int u = 0; u < 8; ++u) v[u] = part[int64_t(list[k + 4 * u]) * RED_COLS];
+                for (int u = 0; u < 8; ++u) v[u] = part[int64_t(list[k + 4 * u]) * DEM_RED_COLS];
 #pragma unroll
                 for (int u = 0; u < 8; ++u) acc += v[u];
             }
-            for (; k < n; k += 4) acc += part[int64_t(list[k]) * RED_COLS];
+            for (; k < n; k += 4) acc += part[int64_t(list[k]) * DEM_RED_COLS];
         }
         __syncthreads();
     }

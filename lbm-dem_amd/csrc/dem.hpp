@@ -320,7 +320,7 @@ struct ForceArgs {
     const double* xiOld;
     double* xiNew;
     const double *ox0, *ox1, *ow1, *or_;
-    double* redPart;      // per block: RED_COLS sums (see dem_forces)
+    double* redPart;      // per block: DEM_RED_COLS sums (see dem_forces)
     int* redFlag;         // per block: the sums are written
     int blocks, lanes;
     int demTimeStep;
@@ -539,11 +539,10 @@ __device__ inline void chain_add(V& acc, V t) {
 // What a particle does to impactors and walls goes to a row of LDS, and a block that has any adds its
 // rows up in particle order, column by column, for the sums over the blocks (dem_objects): the same
 // result as a pass over per-particle arrays, without those arrays and without a launch of its own.
-constexpr int RED_COLS = 12 * 2 + 6 * MAX_WALLS;  // at most two impactors (lbdem_set_objects)
 template <bool STRESS, int LANES>
 __device__ inline void dem_forces(const ForceArgs& a, int blk) {
 #pragma clang fp contract(off)
-    __shared__ double sRed[256 / LANES][RED_COLS];
+    __shared__ double sRed[256 / LANES][DEM_RED_COLS];
     const int gt = blk * 256 + threadIdx.x;
     const int lane = gt % LANES;
     const DemParams& P = a.p;
@@ -876,7 +875,7 @@ __device__ inline void dem_forces(const ForceArgs& a, int blk) {
     if (int(threadIdx.x) < ncol) {
         double s = 0.0;
         for (int r = 0; r < 256 / LANES; ++r) s += sRed[r][threadIdx.x];
-        a.redPart[int64_t(blk) * RED_COLS + threadIdx.x] = s;
+        a.redPart[int64_t(blk) * DEM_RED_COLS + threadIdx.x] = s;
     }
     if (threadIdx.x == 0) a.redFlag[blk] = 1;
 }

@@ -44,7 +44,6 @@ struct HydroArgs {
     int stride;      // of the columns of part
     double* hacc;
     double *FHydro, *MHydro, *fluidVol, *objFH, *objMH, *wallFH;
-    int diag;
     int blocks;      // of the finalisation (0: none)
 };
 __device__ inline void hydro_finalize(const HydroArgs& a, const Consts& k, DevScalars* sc, int blk, double* red) {
@@ -53,7 +52,6 @@ __device__ inline void hydro_finalize(const HydroArgs& a, const Consts& k, DevSc
     if (blk < PART_STRIDE) {
         const int c = blk;
         const bool obj = c < PART_WALL;
-        if (!obj && !a.diag) return;
         if (obj && c / 7 >= k.nObj && c != PART_BB) return;            // no such object
         if (!obj && (c - PART_WALL) / 3 >= k.nWall) return;  // no such wall
         const double v = block_sum(a.part + int64_t(c) * a.stride, obj ? sc->nPartObj : sc->nPartWall, red);

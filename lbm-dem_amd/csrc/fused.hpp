@@ -68,7 +68,7 @@ __device__ inline typename Types<S>::C object_value(const FusedArgs<S>& a, int j
 
 // boundary link of the storing cell (LB.cpp:1390-1453): value reflected into the slot the cell
 // itself loads next step; momentum exchange into the block partials
-template <typename S, bool DIAG>
+template <typename S>
 __device__ inline typename Types<S>::C boundary_value(const FusedArgs<S>& a, int j, int32_t yj, uint8_t ty,
                                                      typename Types<S>::C gj, typename Types<S>::C n,
                                                      typename Types<S>::C sx, typename Types<S>::C sy,
@@ -81,7 +81,7 @@ __device__ inline typename Types<S>::C boundary_value(const FusedArgs<S>& a, int
         return -gj + C(w_rt(j)) * (C(9) * (cu * cu) - C(3) * usq);
     }
     if (ty == T_WALL) {
-        if (DIAG && k.nWall > 0 && !k.slip) {
+        if (k.nWall > 0 && !k.slip) {
             int wi = a.solid[yj];
             wi = (wi >= 0 && wi < k.nWall) ? wi : 0;
             const double v2 = 2.0 * double(gj);
@@ -375,7 +375,7 @@ __device__ inline void load_bundle(const FusedArgs<S>& a, const RowYZ& r, const 
     n.s = (n.act && (t & T_PMASK)) ? a.solid[i] : 0;
 }
 
-template <typename S, int PAR, bool FSURF, bool DIAG, int FZ, bool NN>
+template <typename S, int PAR, bool FSURF, int FZ, bool NN>
 __device__ inline void k_fused(FusedArgs<S> a) {
     using C = typename Types<S>::C;
     using M = typename Types<S>::M;
@@ -527,7 +527,7 @@ __device__ inline void k_fused(FusedArgs<S> a) {
                 }
                 // wall force of the node's links into the block's partials; the lanes of a wavefront
                 // nearly always face one wall, and add up before the one atomic per component
-                if (DIAG && a.k.nWall > 0 && !a.k.slip) {  // slip walls take no force (LB.cpp:1454-1482)
+                if (a.k.nWall > 0 && !a.k.slip) {  // slip walls take no force (LB.cpp:1454-1482)
                     const int wp = int(bc_ >> BC_WALL_SHIFT) & 7;
                     const bool hit = wf[0] != 0.0 || wf[1] != 0.0 || wf[2] != 0.0;
                     const unsigned long long hm = __ballot(hit);
@@ -567,7 +567,7 @@ __device__ inline void k_fused(FusedArgs<S> a) {
                     const C cu = C(cx_rt(j)) * r.sx + C(cy_rt(j)) * r.sy + C(cz_rt(j)) * r.sz;
                     bcv = -gj + C(w_rt(j)) * (C(9) * (cu * cu) - C(3) * r.usq);
                 } else if (!REGLINKS && cls == BC_WALL) {
-                    if (DIAG && a.k.nWall > 0 && !a.k.slip) {  // slip walls take no force (LB.cpp:1454-1482)
+                    if (a.k.nWall > 0 && !a.k.slip) {  // slip walls take no force (LB.cpp:1454-1482)
                         const double v2 = 2.0 * double(gj);
                         double* wp = &sPart[PART_WALL + 3 * wprim];
                         if (cx_rt(j)) atomicAdd(wp + 0, v2 * cx_rt(j));
@@ -580,7 +580,7 @@ __device__ inline void k_fused(FusedArgs<S> a) {
                 } else {
                     const uint8_t ty = a.type[yj] & T_BASE;
                     if (ty == T_FLUID || ty == T_IF) continue;  // an object node uncovered since marking
-                    bcv = boundary_value<S, DIAG>(a, j, yj, ty, gj, r.n, r.sx, r.sy, r.sz, r.usq, mc, sPart, sObj);
+                    bcv = boundary_value<S>(a, j, yj, ty, gj, r.n, r.sx, r.sy, r.sz, r.usq, mc, sPart, sObj);
                 }
                 StoreT<S>::st(PAR == 0 ? nbs : own, bcv);
             }
@@ -718,7 +718,7 @@ static void launch_slip(const Box& b, double s1, hipStream_t s) {
 }
 
 template <typename S>
-void launch_fused(Box& b, const Consts& k, const PartLB* plb, const ObjLB* olb, DevScalars* sc, bool diag,
+void launch_fused(Box& b, const Consts& k, const PartLB* plb, const ObjLB* olb, DevScalars* sc,
                          bool storeVel, hipStream_t s, hipEvent_t ev0, hipEvent_t ev1) {
     FusedArgs<S> a;
     a.g = b.g; a.f = (S*)b.f; a.type = b.type; a.solid = b.solid;
@@ -736,10 +736,9 @@ void launch_fused(Box& b, const Consts& k, const PartLB* plb, const ObjLB* olb, 
     a.storeVel = storeVel ? 1 : 0;
     const bool fs = k.freeSurface != 0;
     if (ev0) (void)hipEventRecord(ev0, s);
-    (void)diag;  // the wall diagnostics are always accumulated
     const bool nn = b.visc != nullptr;
 #define LBDEM_FUSED(P, F, Z, V) \
-    launch<&k_fused<S, P, F, true, Z, V>, FX * FY, FusedOcc<S>::value>(dim3(grid), dim3(FX, FY, 1), s, a)
+    launch<&k_fused<S, P, F, Z, V>, FX * FY, FusedOcc<S>::value>(dim3(grid), dim3(FX, FY, 1), s, a)
 #define LBDEM_FUSED_Z(P, F, V)                 \
     switch (fz) {                             \
         case 1: LBDEM_FUSED(P, F, 1, V); break; \

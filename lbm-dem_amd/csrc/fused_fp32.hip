@@ -2,6 +2,6 @@
 #include "fused.hpp"
 
 namespace lbdem {
-template void launch_fused<float>(Box&, const Consts&, const PartLB*, const ObjLB*, DevScalars*, bool, bool, hipStream_t,
+template void launch_fused<float>(Box&, const Consts&, const PartLB*, const ObjLB*, DevScalars*, bool, hipStream_t,
                                hipEvent_t, hipEvent_t);
 }

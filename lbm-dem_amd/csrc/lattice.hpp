@@ -85,16 +85,6 @@ __device__ inline int64_t load_slot(const Geom& g, int64_t i, const Offs& o, int
     return L == 0 ? int64_t(q) * g.N + i : int64_t(opp_rt(q)) * g.N + i + o.d(opp_rt(q));
 }
 
-template <typename C>
-__device__ inline void equilibrium_offsets(C n, C ux, C uy, C uz, C* geq) {
-    const C usq = ux * ux + uy * uy + uz * uz;
-#pragma unroll
-    for (int q = 0; q < Q; ++q) {
-        const C cu = C(cxq(q)) * ux + C(cyq(q)) * uy + C(czq(q)) * uz;
-        geq[q] = C(wq(q)) * ((n - C(1)) + n * (C(3) * cu + C(4.5) * cu * cu - C(1.5) * usq));
-    }
-}
-
 constexpr int FX = FUSED_TILE_X, FY = FUSED_TILE_Y;  // 64x4 threads: 4 row segments, each lane walks FZ cells
                                                      // along z (FZ 1, 2, 4 or 8, chosen per box)
 constexpr int HS = 64;                  // per-block particle hash slots
@@ -176,11 +166,6 @@ __device__ inline void wave_add(double* dst, double v) {
     for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
     if (__lane_id() == 0 && v != 0.0) atomicAdd(dst, v);
 }
-__device__ inline void wave_add(int* dst, int v) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-    if (__lane_id() == 0 && v != 0) atomicAdd(dst, v);
-}
 
 // check nodes and source directions of the slip reflection (LB.cpp:1454-1482; see k_slip)
 __host__ __device__ constexpr int slip1Check(int j) {
@@ -202,7 +187,7 @@ __host__ __device__ constexpr int slip2Dir(int j) {
 
 // the fused step in storage type S (fused.hpp, instantiated once per storage type)
 template <typename S>
-void launch_fused(Box& b, const Consts& k, const PartLB* plb, const ObjLB* olb, DevScalars* sc, bool diag,
+void launch_fused(Box& b, const Consts& k, const PartLB* plb, const ObjLB* olb, DevScalars* sc,
                   bool storeVel, hipStream_t s, hipEvent_t ev0, hipEvent_t ev1);
 
 }  // namespace lbdem

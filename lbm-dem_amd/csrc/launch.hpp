@@ -86,7 +86,7 @@ struct Launcher<Body, MAXT, MINW, void (*)(P...)> {
     using Tuple = Pack<Held<P>...>;
     static_assert(std::is_trivially_copyable<Tuple>::value, "kernel arguments are copied as bytes");
     static inline const char tag = 0;
-    static const char* signature() {  // "lbdem::Launcher<&lbdem::k_fused<float, 0, true, true, 8>, 256, 4, ...>"
+    static const char* signature() {  // "lbdem::Launcher<&lbdem::k_fused<float, 0, true, 8, false>, 256, 4, ...>"
         static const std::string s = [] {
             int st = 0;
             char* d = abi::__cxa_demangle(typeid(Launcher).name(), nullptr, nullptr, &st);

@@ -373,11 +373,11 @@ int fused_grid_blocks(const Geom& g, int fz, int prec) {
     return ((nseg * nby * nbz + 7) / 8) * 8;                              // XCD-spread tiles
 }
 
-void lb_fused_step(Box& b, const Consts& k, const PartLB* plb, const ObjLB* olb, DevScalars* sc, bool diag,
+void lb_fused_step(Box& b, const Consts& k, const PartLB* plb, const ObjLB* olb, DevScalars* sc,
                    bool storeVel, hipStream_t s, hipEvent_t ev0, hipEvent_t ev1) {
-    if (b.prec == LBDEM_PREC_FP64) launch_fused<double>(b, k, plb, olb, sc, diag, storeVel, s, ev0, ev1);
-    else if (b.prec == LBDEM_PREC_FP32) launch_fused<float>(b, k, plb, olb, sc, diag, storeVel, s, ev0, ev1);
-    else launch_fused<__half>(b, k, plb, olb, sc, diag, storeVel, s, ev0, ev1);
+    if (b.prec == LBDEM_PREC_FP64) launch_fused<double>(b, k, plb, olb, sc, storeVel, s, ev0, ev1);
+    else if (b.prec == LBDEM_PREC_FP32) launch_fused<float>(b, k, plb, olb, sc, storeVel, s, ev0, ev1);
+    else launch_fused<__half>(b, k, plb, olb, sc, storeVel, s, ev0, ev1);
 }
 
 __device__ inline void k_hydro_finalize(HydroArgs a, Consts k, DevScalars* sc) {
@@ -385,18 +385,17 @@ __device__ inline void k_hydro_finalize(HydroArgs a, Consts k, DevScalars* sc) {
     if (int(blockIdx.x) < a.blocks) hydro_finalize(a, k, sc, int(blockIdx.x), red);
 }
 static HydroArgs hydro_args(const Box& b, const Consts& k, double* FHydro, double* MHydro, double* fluidVol, double* objFH,
-                            double* objMH, double* wallFH, bool diag) {
+                            double* objMH, double* wallFH) {
     HydroArgs a;
     a.part = b.blockPart; a.stride = part_stride(b.g); a.hacc = b.hacc;
     a.FHydro = FHydro; a.MHydro = MHydro; a.fluidVol = fluidVol; a.objFH = objFH; a.objMH = objMH; a.wallFH = wallFH;
-    a.diag = diag ? 1 : 0;
     a.blocks = PART_STRIDE + (k.nPart + HF_THREADS - 1) / HF_THREADS;
     return a;
 }
 
 void lb_hydro_finalize(const Box& b, const Consts& k, double* FHydro, double* MHydro, double* fluidVol,
-                       DevScalars* sc, double* objFH, double* objMH, double* wallFH, bool diag, hipStream_t s) {
-    const HydroArgs a = hydro_args(b, k, FHydro, MHydro, fluidVol, objFH, objMH, wallFH, diag);
+                       DevScalars* sc, double* objFH, double* objMH, double* wallFH, hipStream_t s) {
+    const HydroArgs a = hydro_args(b, k, FHydro, MHydro, fluidVol, objFH, objMH, wallFH);
     launch<&k_hydro_finalize, HF_THREADS, 1>(a.blocks, HF_THREADS, s, a, k, sc);
 }
 
@@ -423,7 +422,7 @@ static void front(Box& b, const Consts& k, DevScalars* sc, const HydroArgs& h, b
 void lb_front(Box& b, const Consts& k, DevScalars* sc, bool hydro, bool fs, double* FHydro, double* MHydro,
               double* fluidVol, double* objFH, double* objMH, double* wallFH, const DemParams* dp, DemState* ds,
               int demTimeStep, bool forceList, hipStream_t s) {
-    HydroArgs h = hydro_args(b, k, FHydro, MHydro, fluidVol, objFH, objMH, wallFH, true);
+    HydroArgs h = hydro_args(b, k, FHydro, MHydro, fluidVol, objFH, objMH, wallFH);
     if (!hydro) h.blocks = 0;
     NbrArgs n{};
     ForceArgs f{};

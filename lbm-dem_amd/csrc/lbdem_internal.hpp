@@ -240,10 +240,10 @@ void lb_download_visc(const Box& b, double* out, hipStream_t s);
 void lb_hydro_stress(const Box& b, const PartLB* plb, int nPart, double L, double F, double* shydro, hipStream_t s);
 void lb_mark_edges(const Box& b, DevScalars* sc, hipStream_t s);
 // storeVel: every active node's density and velocity into aux (else the interface nodes' only)
-void lb_fused_step(Box& b, const Consts& k, const PartLB* plb, const ObjLB* olb, DevScalars* sc, bool diag,
+void lb_fused_step(Box& b, const Consts& k, const PartLB* plb, const ObjLB* olb, DevScalars* sc,
                    bool storeVel, hipStream_t s, hipEvent_t ev0 = nullptr, hipEvent_t ev1 = nullptr);
 void lb_hydro_finalize(const Box& b, const Consts& k, double* FHydro, double* MHydro, double* fluidVol,
-                       DevScalars* sc, double* objFH, double* objMH, double* wallFH, bool diag, hipStream_t s);
+                       DevScalars* sc, double* objFH, double* objMH, double* wallFH, hipStream_t s);
 // The launches between two fused kernels (front.hpp): hydro: the finalisation of the fused kernel's
 // sums; fs: the free surface; dp, ds (may be null): the neighbour list (forceList: built without asking
 // the trigger, and no forces) and the forces of DEM step demTimeStep
@@ -329,7 +329,7 @@ struct DemState {
     int* cellFill;
     int* cellItems;
     int* cellKey;
-    double* redPart;           // per block of the force pass: impactor and wall sums (RED_COLS in dem.hpp)
+    double* redPart;           // per block of the force pass: impactor and wall sums (DEM_RED_COLS columns)
     int* redFlag;              // per block: the sums are written
     unsigned long long* blockMax;  // [VEL_SLOTS]: largest particle |v|^2 of the last integration, per slot (bit patterns)
     // objects
@@ -349,7 +349,7 @@ struct DemState {
 };
 int dem_force_lanes(int nPart, bool inBatch);   // lanes per particle of the force pass
 int dem_force_blocks(int nPart, bool inBatch);  // its blocks
-constexpr int DEM_RED_COLS = 60;
+constexpr int DEM_RED_COLS = 12 * 2 + 6 * MAX_WALLS;  // columns of redPart: at most two impactors (lbdem_set_objects)
 // totals, integration, objects and walls (after the forces and the hydrodynamic sums)
 void dem_integrate(const DemParams& p, DemState& d, int demTimeStep, hipStream_t s);
 void dem_refresh_views(const DemParams& p, DemState& d, hipStream_t s);

@@ -500,11 +500,13 @@ __device__ void wall_like_contact(const DemParams& P, double dampCoeff, double r
 // Lanes per particle in the force kernel. A lane walks its share of the partners one after the other,
 // about 5 us each (two dependent gathers, then FP64 divisions, a root, a logarithm, an exponential),
 // so while the wavefronts of 16 lanes per particle fit on the GPU they finish first (480 spheres:
-// 17.4 us a launch with 4 lanes, 11.8 with 16); beyond that 4 lanes waste fewer of them (31 000
-// spheres: all wavefronts resident at once). A batch's launch holds the spheres of all its boxes
-// (64 boxes of edge 48-128: 0.09 ms with 4 lanes, 0.54 with 16). Either way the sums are those of four lanes, each of which
-// adds its partners in list order: a rounding that changed with the lanes would change positions in
-// their last bit, and a run with 4- or 2-byte populations amplifies that.
+// 17.4 us a launch with 4 lanes, 11.8 with 16); beyond that 4 lanes waste fewer of them. The line, by
+// whole steps of a 128x160x128 box (FP32) with 4 and 16 lanes: 1000 spheres 133 and 131 us, 2000 137 and 137,
+// 4000 148 and 150, 8000 169 and 168, 10 000 181 and 189, 16 000 237 and 251. A batch's launch holds the
+// spheres of all its boxes (64 boxes of edge 48-128: 0.09 ms with 4 lanes, 0.54 with 16). Either way the
+// force and torque sums are those of four lanes, each of which adds its partners in list order: a rounding that
+// changed with the lanes would change positions in their last bit, and a run with 4- or 2-byte
+// populations amplifies that. (The stress tensors, which nothing in a run reads, are summed lane by lane.)
 constexpr int DEM_LANES_FEW = 16, DEM_LANES_MANY = 4, DEM_FEW = 8192, DEM_CHAINS = 4;
 
 // sum over N lanes, in a fixed butterfly order

@@ -87,6 +87,10 @@ __device__ inline void hydro_finalize(const HydroArgs& a, const Consts& k, DevSc
 constexpr int FS_THREADS = 256;
 static_assert(FS_THREADS == HF_THREADS, "one launch holds the blocks of all passes");
 
+// Entries of a list whose counter went past its capacity (reported as an overflow at the next
+// synchronisation) that are there to read.
+__device__ inline int list_len(int count, int cap) { return min(count, cap); }
+
 template <typename S>
 struct FsArgs {
     Geom g;
@@ -133,7 +137,8 @@ __device__ inline void fs_mass(const FsArgs<S>& a, const HydroArgs& h, int blk, 
     if (blk * HF_THREADS >= nIf) return;
     const double extra = block_sum(h.part + int64_t(PART_BB) * h.stride, sc->nPartObj, red);
     const double addE = extra / double(nIf);
-    for (int k = blk * HF_THREADS + threadIdx.x; k < nIf; k += nblk * HF_THREADS) {
+    const int listed = list_len(nIf, a.cap);
+    for (int k = blk * HF_THREADS + threadIdx.x; k < listed; k += nblk * HF_THREADS) {
         const int64_t i = ifList[k];
         int x, y, z;
         cell_xyz(g, i, x, y, z);
@@ -179,7 +184,7 @@ template <typename S>
 __device__ inline void fs_mutants(const FsArgs<S>& a, int blk) {
     uint8_t* const type = a.type;
     DevScalars* const sc = a.sc;
-    const int nIf = sc->nIf;
+    const int nIf = list_len(sc->nIf, a.cap);
     for (int k = blk * FS_THREADS + threadIdx.x; k < nIf; k += a.blocks * FS_THREADS) {
         const int64_t i = a.ifList[k];
         const auto m = a.newMass[k];
@@ -217,7 +222,7 @@ __device__ inline void fs_neighbours(const FsArgs<S>& a, int blk) {
     const int cap = a.cap;
     using C = typename Types<S>::C;
     using M = typename Types<S>::M;
-    const int nF = sc->nFilled, nE = sc->nEmptied;
+    const int nF = list_len(sc->nFilled, cap), nE = list_len(sc->nEmptied, cap);
     if (blk * FS_THREADS >= nF + nE) return;
     double gained = 0.0;
     for (int k = blk * FS_THREADS + threadIdx.x; k < nF + nE; k += a.blocks * FS_THREADS) {
@@ -280,7 +285,8 @@ __device__ inline void fs_settle(const FsArgs<S>& a, const Consts& k, int blk) {
     const int changedCap = a.changedCap;
     using C = typename Types<S>::C;
     using M = typename Types<S>::M;
-    const int nN = sc->nNewIf, nF = sc->nFilled, nE = sc->nEmptied, tot = nN + nF + nE;
+    const int nN = list_len(sc->nNewIf, a.cap), nF = list_len(sc->nFilled, a.cap), nE = list_len(sc->nEmptied, a.cap);
+    const int tot = nN + nF + nE;
     if (blk * FS_THREADS >= tot) return;
     const int64_t N = g.N;
     double acc = 0.0;
@@ -349,7 +355,7 @@ __device__ inline void fs_isolated(const FsArgs<S>& a, int blk) {
     int* const count2 = a.count2;
     DevScalars* const sc = a.sc;
     const int cap = a.cap;
-    const int nIf = sc->nIf, nN = sc->nNewIf;
+    const int nIf = list_len(sc->nIf, cap), nN = list_len(sc->nNewIf, cap);
     if (blk * FS_THREADS >= nIf + nN) return;
     __shared__ int sPos[8];
     __shared__ double sSum[8];
@@ -416,7 +422,7 @@ struct RedistArgs {  // of FsArgs, for the pass that does not depend on the stor
     const int32_t *list2, *filled, *newIf;
     const int* count2;
     int32_t *marker, *changed;
-    int changedCap, blocks;
+    int cap, changedCap, blocks;
     DevScalars* sc;
 };
 template <typename M>
@@ -430,7 +436,7 @@ __device__ inline void fs_redistribute(const RedistArgs& a, M* mass, int blk) {
     const int* const count2 = a.count2;
     const int changedCap = a.changedCap;
     DevScalars* const sc = a.sc;
-    const int n2 = *count2;
+    const int n2 = list_len(*count2, a.cap);
     const double add = sc->surplus / double(sc->nIfFinal);
     for (int k = blk * FS_THREADS + threadIdx.x; k < n2; k += a.blocks * FS_THREADS) {
         const int32_t v = list2[k];
@@ -441,7 +447,7 @@ __device__ inline void fs_redistribute(const RedistArgs& a, M* mass, int blk) {
             push_changed(changed, changedCap, sc, ~v);
         }
     }
-    const int nF = sc->nFilled, nN = sc->nNewIf;
+    const int nF = list_len(sc->nFilled, a.cap), nN = list_len(sc->nNewIf, a.cap);
     for (int k = blk * FS_THREADS + threadIdx.x; k < nF + nN; k += a.blocks * FS_THREADS)
         marker[k < nF ? filled[k] : newIf[k - nF]] = -1;
     if (blk == 0 && threadIdx.x == 0) sc->lastSurplus = sc->surplus;

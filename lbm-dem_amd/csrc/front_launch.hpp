@@ -19,7 +19,7 @@ void launch_front(const FsArgs<S>& a, const HydroArgs& h, const Consts& k, const
         else launch<&k_front4<S, 0>, FS_THREADS, 1>(g, bs, s, a, k, n);
     }
     if (const int g = a.blocks + n.slotBlocks; g > 0) launch<&k_front5<S>, FS_THREADS, 1>(g, bs, s, a, n);
-    const RedistArgs r{a.type, a.list2, a.filled, a.newIf, a.count2, a.marker, a.changed, a.changedCap, a.blocks, a.sc};
+    const RedistArgs r{a.type, a.list2, a.filled, a.newIf, a.count2, a.marker, a.changed, a.cap, a.changedCap, a.blocks, a.sc};
     if (r.blocks + f.blocks > 0) launch_front6(r, a.mass, f, s);
 }
 

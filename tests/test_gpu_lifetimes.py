@@ -111,3 +111,27 @@ def test_start_up_is_over_when_no_chunk_is_left_to_capture(gpu_lib):
     sim.use_graphs(False)
     assert not captured()
     sim.close()
+
+
+def test_interface_list_overflow_is_reported(gpu_lib):
+    """A restart whose nodes are all interface nodes, three times what the interface list holds (a quarter of
+    the box): the free surface's passes stay within their lists, the run reports the overflow, and the
+    device goes on."""
+    E = 66
+    v, _, _ = workloads.impact_box(size=(E, E, E), fluid_height=float(E - 1), n_spheres=0, r=1.5, r_imp=3.0, y_imp=30.0,
+                                   speed=0.01, periodic=False)
+    v.update(demSolve=0, lbFY=0.0)
+    w = np.array([1.0 / 3.0] + [1.0 / 18.0] * 6 + [1.0 / 36.0] * 12)
+    rec = np.zeros(((E - 2) ** 3, lbdem.RESTART_REC))
+    rec[:, 4], rec[:, 5], rec[:, 6:] = -0.5, 0.1, w
+    sim = lbdem.Simulation(gpu_lib, lbdem.params_from_values(v, lbdem.PREC_FP32), lbdem.ParticleSet(), lbdem.ObjectSet())
+    sim.set_restart((E, E, E), np.full(E ** 3, 3, np.uint8), rec)
+    sim.init()
+    assert sim.info()["nInterface"] == (E - 2) ** 3 > E ** 3 // 4
+    sim.cycle(3)
+    with pytest.raises(lbdem.LbdemError, match="overflowed"):
+        sim.synchronize()
+    sim.close()
+    ok = _small(gpu_lib, 7)
+    assert np.isfinite(ok.total_mass())
+    ok.close()

@@ -949,8 +949,9 @@ static void enqueue_hydro(lbdem_ctx* c) {
     lb_hydro_finalize(c->box, c->k, c->ds.FHydro, c->ds.MHydro, c->ds.fluidVol, c->sc, c->ds.oFHydro, c->ds.oMHydro,
                       c->ds.wFHydro, c->stream);
 }
-// finalize = false: the sums are finalised with the free surface that follows
-static void enqueue_lb(lbdem_ctx* c, bool finalize = true) {  // LB::latticeBolzmannStep (LB.cpp:400-418)
+// finalize = false: the sums are finalised with the free surface that follows; coupled: the coupling was
+// enqueued just before with lbFollows
+static void enqueue_lb(lbdem_ctx* c, bool finalize = true, bool coupled = false) {  // LB::latticeBolzmannStep (LB.cpp:400-418)
     if (!c->forceField && !c->lbFReset) {  // LB.cpp:1303-1305
         c->k.lbF[0] = c->k.lbF[1] = c->k.lbF[2] = 0.0;
         c->lbFReset = true;
@@ -975,7 +976,7 @@ static void enqueue_lb(lbdem_ctx* c, bool finalize = true) {  // LB::latticeBolz
             finish_tuning(c);
         }
     }
-    lb_mark_edges(c->box, c->sc, c->stream);
+    lb_mark_edges(c->box, c->sc, coupled, c->stream);
     const bool storeVel = c->velState == 1;  // lbdem_store_velocity asked for this step
     c->velState = storeVel ? 2 : 0;
     // the stress diagnostics read every active node's hydrodynamic force from aux
@@ -1022,8 +1023,9 @@ static void enqueue_step(lbdem_ctx* c) {
         flush_fs(c);
     }
     if (c->demTime >= c->prm.demInitialRepeat) {
-        if (c->prm.demSolve) enqueue_coupling(c, true);
-        enqueue_lb(c, !c->freeSurface);
+        const bool coupled = c->prm.demSolve != 0;
+        if (coupled) enqueue_coupling(c, true);
+        enqueue_lb(c, !c->freeSurface, coupled);
         c->fsDeferred = c->freeSurface;
     } else if (c->demTime <= c->prm.demInitialRepeat) {
         if (c->prm.demSolve) enqueue_coupling(c);

@@ -319,7 +319,8 @@ __device__ inline void mark_full_b(Geom g, uint8_t* type, const int32_t* solid, 
         mark_node(g, type, solid, bcm, int32_t(i));
 }
 // end of the coupling step's flag pass (flags_compute set kminP to INT_MAX) or of its search for the
-// lowest flagged node: taken by the marking, or by a launch of its own after a coupling step without an LB step
+// lowest flagged node: in the marking of the LB step that was enqueued with the coupling, or in a launch of
+// its own. (An LB step without a coupling leaves a list rebuild to the next coupling.)
 __device__ inline void couple_end(DevScalars* sc) {
     if (sc->newNeighborList) {
         if (sc->kminP == INT_MAX) sc->kminP = -1;
@@ -336,11 +337,10 @@ __device__ inline void k_couple_end(DevScalars* sc) { couple_end(sc); }
 // neighbourhood (wrapped) of every node on the change list. A node reached from several changed
 // nodes is marked several times with the same result.
 __device__ inline void k_mark(Geom g, uint8_t* type, const int32_t* solid, uint64_t* bcm, const int32_t* changed, int cap,
-                              DevScalars* sc) {
-    // the coupling before this launch is complete and the fused kernel comes next: its counters start
-    // at zero, and the flag pass of a list rebuild has been taken
+                              int endCoupling, DevScalars* sc) {
+    // the fused kernel comes next: its counters start at zero
     if (blockIdx.x == 0 && threadIdx.x == 0) {
-        couple_end(sc);
+        if (endCoupling) couple_end(sc);
         sc->nIf = 0;
         sc->nPartObj = sc->nPartWall = 0;
     }
@@ -362,8 +362,8 @@ __device__ inline void k_mark(Geom g, uint8_t* type, const int32_t* solid, uint6
     }
 }
 
-void lb_mark_edges(const Box& b, DevScalars* sc, hipStream_t s) {
-    launch_gs<&k_mark, 256, 1>(MARK_GRID, 256, s, b.g, b.type, b.solid, b.bcm, b.changed, b.changedCap, sc);
+void lb_mark_edges(const Box& b, DevScalars* sc, bool endCoupling, hipStream_t s) {
+    launch_gs<&k_mark, 256, 1>(MARK_GRID, 256, s, b.g, b.type, b.solid, b.bcm, b.changed, b.changedCap, endCoupling ? 1 : 0, sc);
     // the list and the full-pass flag are reset by the finalisation of the fused kernel's sums
 }
 
@@ -1046,7 +1046,7 @@ static void obj_uncover(Box& b, const Consts& k, const CoupleArgs& a, hipStream_
 
 // The coupling step (LB.cpp:432-467): flags, impactor nodes, findNewActive, in four launches (two
 // without an impactor). order: the particles sorted by link cell (the rebuild's cell list), or null.
-// markFollows: lb_mark_edges is enqueued next and ends the step; else a launch of its own does.
+// markFollows: lb_mark_edges is enqueued next and ends the coupling (endCoupling); else a launch of its own does.
 void lb_coupling(Box& b, const Consts& k, const PartLB* plb, const ObjLB* olb, DevScalars* sc, const int* nbrCount,
                  const int* nbrList, bool useList, const int* order, bool markFollows, hipStream_t s) {
     CoupleArgs a;

@@ -238,7 +238,7 @@ void lb_download_visc(const Box& b, double* out, hipStream_t s);
 // SHydro of every particle (9 per particle, physical units: L, F = unit.Length, unit.Force) from
 // the aux planes an LB step with storeVel left
 void lb_hydro_stress(const Box& b, const PartLB* plb, int nPart, double L, double F, double* shydro, hipStream_t s);
-void lb_mark_edges(const Box& b, DevScalars* sc, hipStream_t s);
+void lb_mark_edges(const Box& b, DevScalars* sc, bool endCoupling, hipStream_t s);  // endCoupling: of lb_coupling
 // storeVel: every active node's density and velocity into aux (else the interface nodes' only)
 void lb_fused_step(Box& b, const Consts& k, const PartLB* plb, const ObjLB* olb, DevScalars* sc,
                    bool storeVel, hipStream_t s, hipEvent_t ev0 = nullptr, hipEvent_t ev1 = nullptr);

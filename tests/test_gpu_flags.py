@@ -43,3 +43,29 @@ def test_lowest_sphere_leaves_through_the_seam(oracle_lib, gpu_lib, size, sphere
     assert kept, "no step searched"
     for s in (a, b, c):
         s.close()
+
+
+def test_list_rebuild_waits_for_the_coupling(oracle_lib, gpu_lib):
+    """Sub-step calls with the coupling on the first and every third step after it: a list rebuild of a step without one has its
+    flags made by the next coupling, as the reference's flag of a new list stays set until then."""
+    v, ps, _ = workloads.impact_box(size=(30, 34, 26), fluid_height=18.0, n_spheres=14, r=2.0, r_imp=4.0, y_imp=22.5,
+                                    seed=5, relax=60, periodic=True, bed_top=14.0)
+    v.update(lbFZ=-1.5e-3)
+    a, b = (lbdem.Simulation(lib, lbdem.params_from_values(v, lbdem.PREC_FP64), ps, lbdem.ObjectSet())
+            for lib in (oracle_lib, gpu_lib))
+    a.init()
+    b.init()
+    waited = 0
+    for k in range(36):
+        for s in (a, b):
+            s.dem_step()
+            if k % 3 == 0:
+                s.coupling_step()
+            s.lb_step()
+            s.fs_step()
+        assert a.info()["newNeighborList"] == b.info()["newNeighborList"], k
+        waited += k > 2 and a.info()["newNeighborList"]
+        compare(cases.state(a), cases.state(b), lbdem.PREC_FP64, f"step {k + 1}")
+    assert waited >= 4
+    a.close()
+    b.close()

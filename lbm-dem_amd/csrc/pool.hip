@@ -134,8 +134,8 @@ struct lbdem_pool {
     int maxConcurrent = 1;
     int chunk = 32;
     bool batching = true;
-    int batchTile = 0;  // walk of the batches (0: tuned on the batches themselves)
-    // stepper-owned, per storage precision: the tuned walk and the size of the batch it was tuned
+    int batchTile = 0;  // tile of the batches (0: tuned on the batches themselves)
+    // stepper-owned, per storage precision: the tuned tile and the size of the batch it was tuned
     // on (a batch at least twice that size is tuned again, until one of 8 runs or more was: the
     // best walk changes with the batch's size while it is small)
     int tunedTile[3] = {0, 0, 0}, tunedSize[3] = {0, 0, 0};
@@ -420,7 +420,7 @@ void stepper_loop(lbdem_pool* P) {
                 if (lbdem_batch_create(ctxs.data(), int(ctxs.size()), &B.b) == 0) {
                     const size_t slice = (BATCH_REGION / 3) & ~size_t(255);  // tables are read as aligned records
                     lbdem::batch_use_region(B.b, P->batchRegion + pr * slice, slice);
-                    // the batch's walk: fixed, tuned on a batch of comparable size, or tuned now
+                    // the batch's tile: fixed, tuned on a batch of comparable size, or tuned now
                     const int nm = int(keep.size());
                     int tz = P->batchTile;
                     if (!tz && P->tunedTile[pr] && (nm < 2 * P->tunedSize[pr] || P->tunedSize[pr] >= 8))

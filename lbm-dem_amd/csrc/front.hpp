@@ -241,6 +241,10 @@ __device__ inline void fs_neighbours(const FsArgs<S>& a, int blk) {
             const int j = __ffs(m) - 1;
             const int64_t l = i + o.d(j);
             if (isF) {
+                if (!stencil_in_arrays(g, l)) {  // gas that an impactor left on a z face of the box
+                    atomicOr(&sc->typeError, 1);
+                    continue;
+                }
                 const int old = atomicMax(&marker[l], int32_t(i));
                 if (old < 0) list_push(newIf, &sc->nNewIf, cap, int32_t(l), &sc->listOverflow);
                 continue;

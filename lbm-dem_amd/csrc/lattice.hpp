@@ -80,6 +80,17 @@ struct Offs {
 
 __device__ inline int32_t offs_rt(const Offs& o, int q) { return o.d(q); }
 
+// Whether all neighbours of node i lie within the lattice arrays, wrapped or not: so it is for every node
+// inside the outer layer, and of the layer for all but its z faces and the two rows next to them (indices
+// below XY + X or not below N - XY - X). Only such nodes may become active: an impactor that passes a z face
+// leaves nodes behind on it whose populations would stream out of the arrays (in the fused kernel by 4 GiB,
+// its offsets being unsigned). A node that may not is reported as a type error, as the step that streams
+// into a periodic layer is.
+__device__ inline bool stencil_in_arrays(const Geom& g, int64_t i) {
+    const int64_t reach = int64_t(g.X) * g.Y + g.X;
+    return i >= reach && i < g.N - reach;
+}
+
 // slot holding the post-streaming population q of cell i in layout L (0 natural, 1 swapped)
 __device__ inline int64_t load_slot(const Geom& g, int64_t i, const Offs& o, int q, int L) {
     return L == 0 ? int64_t(q) * g.N + i : int64_t(opp_rt(q)) * g.N + i + o.d(opp_rt(q));

@@ -844,7 +844,11 @@ __device__ inline void k_obj_uncover(Geom g, S* f, uint8_t* type,
         __syncthreads();
         if (tid < cnt) {
             const int32_t i = sCand[tid];
-            const uint8_t nt = newT[tid];
+            uint8_t nt = newT[tid];
+            if (nt != T_GAS && !stencil_in_arrays(g, i)) {  // left behind on a z face of the box
+                nt = T_GAS;
+                atomicOr(&sc->typeError, 1);
+            }
             type[i] = uint8_t((ownT[tid] & T_PMASK) | nt);  // no other thread writes a candidate's type
             const int pos = sChBase + tid;
             if (pos < changedCap) changed[pos] = i;
